@@ -119,3 +119,19 @@ def test_eigh_psd_fp32_rounded_rank_deficient(T):
     assert np.abs(lam[r:]).max() <= 1e-4 * ev[0]
     P = u[:, :r] @ u[:, :r].T
     assert np.linalg.norm(P - V[:, :r] @ V[:, :r].T) <= 1e-5
+
+
+# the rotation rounds' two coefficient paths (squared norms within 2^(+-400) of
+# one, and beyond) and the three row chunks of jac_eig_apply (128, 256 and 512
+# rows), with ragged sizes on both sides of a block and of a chunk; the power
+# of two is exact, so the bounds are check_eig's
+@pytest.mark.parametrize("n", [17, 33, 130, 1300, 2100])
+@pytest.mark.parametrize("exp", [-500, 0, 500])
+def test_eigh_psd_scaled_by_powers_of_two(T, n, exp):
+    if exp and n > 1000:
+        pytest.skip("the range of the squared norms does not depend on the size")
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n + 5, n))
+    K = A.T @ A
+    u, lam = T._eigh_psd_device(dev(np.ldexp(K, exp)), 1)
+    check_eig(K, u.cpu().numpy(), np.ldexp(lam.cpu().numpy(), -exp), n)

@@ -181,39 +181,43 @@ struct BJob {
 };
 
 // acc += the 32 x 32 Gram of the pair's vectors (blocks I and K2 of the
-// job's k vectors of length L at W) over rows [r0, r1): 64-row tiles staged
-// through LDS, v_mfma_f64_16x16x4 by four waves (one 16 x 16 quarter each);
-// the next tile's loads are issued into registers before the current
-// tile's MFMAs, so their latency overlaps the MFMAs.
+// job's k vectors of length L at W) over rows [r0, r1): tiles of 64 NG rows
+// staged through LDS, v_mfma_f64_16x16x4 by 4 NG waves (wave w takes the
+// 16 x 16 quarter w % 4 over the tile's rows 64 (w / 4) ..; the NG partial
+// sums are the caller's to add); the next tile's loads are issued into
+// registers before the current tile's MFMAs, so their latency overlaps the
+// MFMAs.
+template <int NG>
 __device__ __forceinline__ void bgram_rows(const double* __restrict__ W, int64_t L, int k, int I,
                                            int K2, int64_t r0, int64_t r1,
                                            double (*Ps)[BJ2 + 1], f64x4b& acc) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ti = wave >> 1, tj = wave & 1;
-  constexpr int PE = 64 * BJ2 / 256;
+  const int ti = (wave >> 1) & 1, tj = wave & 1, kb = 64 * (wave >> 2);
+  constexpr int TR = 64 * NG;
+  constexpr int PE = TR * BJ2 / (256 * NG);
   double pv[PE];
   auto fetch = [&](int64_t rb) {
 #pragma unroll
     for (int i = 0; i < PE; ++i) {
-      const int e = tid + 256 * i, row = e & 63, col = e >> 6;
+      const int e = tid + 256 * NG * i, row = e % TR, col = e / TR;
       const int64_t v = col < BJB ? (int64_t)I * BJB + col : (int64_t)K2 * BJB + (col - BJB);
       const int64_t r = rb + row;
       pv[i] = (v < k && r < r1) ? W[v * L + r] : 0.0;
     }
   };
   if (r0 < r1) fetch(r0);
-  for (int64_t rb = r0; rb < r1; rb += 64) {
+  for (int64_t rb = r0; rb < r1; rb += TR) {
 #pragma unroll
     for (int i = 0; i < PE; ++i) {
-      const int e = tid + 256 * i;
-      Ps[e & 63][e >> 6] = pv[i];
+      const int e = tid + 256 * NG * i;
+      Ps[e % TR][e / TR] = pv[i];
     }
     __syncthreads();
-    if (rb + 64 < r1) fetch(rb + 64);
+    if (rb + TR < r1) fetch(rb + TR);
 #pragma unroll
     for (int k0 = 0; k0 < 64; k0 += 4) {
-      double a = Ps[k0 + (lane >> 4)][16 * ti + (lane & 15)];
-      double b = Ps[k0 + (lane >> 4)][16 * tj + (lane & 15)];
+      double a = Ps[kb + k0 + (lane >> 4)][16 * ti + (lane & 15)];
+      double b = Ps[kb + k0 + (lane >> 4)][16 * tj + (lane & 15)];
       acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
     }
     __syncthreads();
@@ -246,7 +250,7 @@ __global__ void __launch_bounds__(256) bjac_gram(double* __restrict__ Wv, const 
   if (work && tid == 0) atomicAdd(work, (unsigned long long)(r1 - r0));
   const double* base = Wv + J.wv;
   f64x4b acc = {0, 0, 0, 0};
-  bgram_rows(base, J.L, J.k, I, K2, r0, r1, Ps, acc);
+  bgram_rows<1>(base, J.L, J.k, I, K2, r0, r1, Ps, acc);
   double* out = Gpart + (int64_t)item * (BJ2 * BJ2);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -257,7 +261,7 @@ __global__ void __launch_bounds__(256) bjac_gram(double* __restrict__ Wv, const 
 
 // eig items are (job, pair) in job-major order; Gpart items for (job, pair,
 // chunk) start at gram_base + pair * nch.
-__global__ void __launch_bounds__(256) bjac_eig(const double* __restrict__ Gpart,
+__global__ void __launch_bounds__(EIG_NT) bjac_eig(const double* __restrict__ Gpart,
                                                 const BJob* __restrict__ jobs,
                                                 const int* __restrict__ e_job,
                                                 const int* __restrict__ e_pair,
@@ -273,7 +277,7 @@ __global__ void __launch_bounds__(256) bjac_eig(const double* __restrict__ Gpart
   const int pi = e_pair[item];
   {
     // every partial of a group of four chunks loaded before the first add
-    constexpr int PER = BJ2 * BJ2 / 256;
+    constexpr int PER = BJ2 * BJ2 / EIG_NT;
     const double* Gp = Gpart + ((int64_t)J.gram_base + (int64_t)pi * J.nch) * (BJ2 * BJ2);
     double acc[PER];
 #pragma unroll
@@ -284,7 +288,8 @@ __global__ void __launch_bounds__(256) bjac_eig(const double* __restrict__ Gpart
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int i = 0; i < PER; ++i) v[u][i] = Gp[(int64_t)(c + u) * (BJ2 * BJ2) + tid + 256 * i];
+        for (int i = 0; i < PER; ++i)
+          v[u][i] = Gp[(int64_t)(c + u) * (BJ2 * BJ2) + tid + EIG_NT * i];
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -293,15 +298,14 @@ __global__ void __launch_bounds__(256) bjac_eig(const double* __restrict__ Gpart
     for (; c < J.nch; ++c) {
       double v[PER];
 #pragma unroll
-      for (int i = 0; i < PER; ++i) v[i] = Gp[(int64_t)c * (BJ2 * BJ2) + tid + 256 * i];
+      for (int i = 0; i < PER; ++i) v[i] = Gp[(int64_t)c * (BJ2 * BJ2) + tid + EIG_NT * i];
 #pragma unroll
       for (int i = 0; i < PER; ++i) acc[i] += v[i];
     }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int e = tid + 256 * i;
-      sm.G[0][e / BJ2][e % BJ2] = acc[i];
-      sm.Q[0][e / BJ2][e % BJ2] = (e / BJ2 == e % BJ2) ? 1.0 : 0.0;
+      const int e = tid + EIG_NT * i;
+      sm.G[0][eig_pos(e / BJ2)][eig_pos(e % BJ2)] = acc[i];
     }
   }
   __syncthreads();
@@ -313,9 +317,9 @@ __global__ void __launch_bounds__(256) bjac_eig(const double* __restrict__ Gpart
   }
   if (tid == 0) skip[item] = 0;
   if (work && tid == 0) atomicAdd(work + 1, 1ull);
-  const int cur = eig_rotate(sm, J.tol, J.neg2);
+  eig_rotate(sm, J.tol, J.neg2);
   double* out = Qall + (int64_t)item * (BJ2 * BJ2);
-  for (int e = tid; e < BJ2 * BJ2; e += 256) out[e] = sm.Q[cur][e / BJ2][e % BJ2];
+  for (int e = tid; e < BJ2 * BJ2; e += EIG_NT) out[e] = sm.Q[e / BJ2][e % BJ2];
 }
 
 // apply items are (job, pair, chunk) over the L + k rows of [W; Z]
@@ -352,14 +356,14 @@ __global__ void __launch_bounds__(256) bjac_apply(double* __restrict__ Wv, doubl
 #pragma unroll
   for (int i = 0; i < PER; ++i) qv[i] = Qg[threadIdx.x + 256 * i];
   double x[8][BANT];
-  apply_rows_fetch<BANT>(base, ld, J.k, r, re, I, K2, x);
+  apply_rows_fetch<BANT, 4>(base, ld, J.k, r, re, I, K2, x);
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int e = threadIdx.x + 256 * i;
     Q[e / BJ2][e % BJ2] = qv[i];
   }
   lds_barrier();
-  apply_rows_finish<BANT>(base, ld, J.k, r, re, I, K2, x, Q);
+  apply_rows_finish<BANT, 4>(base, ld, J.k, r, re, I, K2, x, Q);
 }
 
 // One Jacobi step for batches whose jobs fit one row chunk (L <= BCH and
@@ -370,7 +374,7 @@ __global__ void __launch_bounds__(256) bjac_apply(double* __restrict__ Wv, doubl
 // still reads them for its Gram would race).  The same arithmetic as
 // bjac_gram + bjac_eig + bjac_apply, in one launch and without the partial
 // Grams and rotations passing through global memory.
-__global__ void __launch_bounds__(256) bjac_fused(double* __restrict__ Wv, double* __restrict__ Zb,
+__global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, double* __restrict__ Zb,
                                                   const BJob* __restrict__ jobs,
                                                   const int* __restrict__ e_job,
                                                   const int* __restrict__ e_pair,
@@ -378,7 +382,7 @@ __global__ void __launch_bounds__(256) bjac_fused(double* __restrict__ Wv, doubl
                                                   const int* __restrict__ gbase, int goff,
                                                   unsigned long long* __restrict__ offmax,
                                                   unsigned long long* __restrict__ work) {
-  __shared__ double Ps[64][BJ2 + 1];
+  __shared__ double Ps[128][BJ2 + 1];
   __shared__ EigLds sm;
   const int item = blockIdx.x, tid = threadIdx.x;
   const int j = e_job[item];
@@ -388,18 +392,28 @@ __global__ void __launch_bounds__(256) bjac_fused(double* __restrict__ Wv, doubl
   const int pi = e_pair[item];
   const int I = brr(pi, s, J.nblk), K2 = brr(J.nblk - 1 - pi, s, J.nblk);
   const int wave = tid >> 6, lane = tid & 63;
-  const int ti = wave >> 1, tj = wave & 1;
+  const int ti = (wave >> 1) & 1, tj = wave & 1;
   double* W = Wv + J.wv;
   double* Z = Zb + J.z;
-  double x[8][4], z[8][4];
-  apply_rows_fetch<4>(W, J.L, J.k, 0, J.L, I, K2, x);  // in flight during the Gram and rounds
-  apply_rows_fetch<4>(Z, J.k, J.k, 0, J.k, I, K2, z);
+  double x[8][2], z[8][2];
+  apply_rows_fetch<2, EIG_NW>(W, J.L, J.k, 0, J.L, I, K2, x);  // in flight during the Gram, rounds
+  apply_rows_fetch<2, EIG_NW>(Z, J.k, J.k, 0, J.k, I, K2, z);
   f64x4b acc = {0, 0, 0, 0};
-  bgram_rows(W, J.L, J.k, I, K2, 0, J.L, Ps, acc);
+  bgram_rows<2>(W, J.L, J.k, I, K2, 0, J.L, Ps, acc);
+  // the two halves' partial sums: the second group's through G[1]
+  int gr[4], gc = eig_pos(16 * tj + (lane & 15));
 #pragma unroll
-  for (int e = 0; e < 4; ++e) sm.G[0][16 * ti + (lane >> 4) + 4 * e][16 * tj + (lane & 15)] = acc[e];
-  for (int e = tid; e < BJ2 * BJ2; e += 256) sm.Q[0][e / BJ2][e % BJ2] = (e / BJ2 == e % BJ2) ? 1.0 : 0.0;
-  __syncthreads();
+  for (int e = 0; e < 4; ++e) gr[e] = eig_pos(16 * ti + (lane >> 4) + 4 * e);
+  if (wave >= 4) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sm.G[1][gr[e]][gc] = acc[e];
+  }
+  lds_barrier();
+  if (wave < 4) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sm.G[0][gr[e]][gc] = acc[e] + sm.G[1][gr[e]][gc];
+  }
+  lds_barrier();
   const double off = eig_off(sm, J.tol, J.neg2);
   if (tid == 0) atomicMax(offmax + j, dbits(off));
   if (off <= J.tol) return;
@@ -408,9 +422,9 @@ __global__ void __launch_bounds__(256) bjac_fused(double* __restrict__ Wv, doubl
     atomicAdd(work + 1, 1ull);
     atomicAdd(work + 2, (unsigned long long)(J.L + J.k));
   }
-  const int cur = eig_rotate(sm, J.tol, J.neg2);
-  apply_rows_finish<4>(W, J.L, J.k, 0, J.L, I, K2, x, sm.Q[cur]);
-  apply_rows_finish<4>(Z, J.k, J.k, 0, J.k, I, K2, z, sm.Q[cur]);
+  eig_rotate(sm, J.tol, J.neg2);
+  apply_rows_finish<2, EIG_NW>(W, J.L, J.k, 0, J.L, I, K2, x, sm.Q);
+  apply_rows_finish<2, EIG_NW>(Z, J.k, J.k, 0, J.k, I, K2, z, sm.Q);
 }
 
 // After global step g: retire jobs whose sweep just ended with off <= tol.
@@ -1042,7 +1056,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
       // work is counted on the device (cnt) and added once at the end
       if (fused) {
         ProfScope p(PROF_JAC_EIG, st, 0.0, 0.0);
-        hipLaunchKernelGGL(bjac_fused, dim3(nei), dim3(256), 0, st, dWv, dZ, dbj, det, det + nei,
+        hipLaunchKernelGGL(bjac_fused, dim3(nei), dim3(EIG_NT), 0, st, dWv, dZ, dbj, det, det + nei,
                            ddone, dgbase, o, doff, cnt);
       } else {
         {
@@ -1052,7 +1066,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
         }
         {
           ProfScope p(PROF_JAC_EIG, st, 0.0, 0.0);
-          hipLaunchKernelGGL(bjac_eig, dim3(nei), dim3(256), 0, st, dG, dbj, det, det + nei, ddone,
+          hipLaunchKernelGGL(bjac_eig, dim3(nei), dim3(EIG_NT), 0, st, dG, dbj, det, det + nei, ddone,
                              dQ, dskip, doff, cnt);
         }
         {

@@ -38,11 +38,25 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+constexpr int EIG_NT = 512;  // threads of a pair eigensolve (8 waves)
+constexpr int EIG_NW = EIG_NT / 64;
+constexpr int GPAD = 2;      // G row padding: rows stay 16-byte aligned
+// Exponents of the pair's squared norms up to which products of two Gram
+// entries (and of tol^2) stay inside FP64's range unscaled.
+constexpr int EIG_RANGE = 400;
+
 struct EigLds {
-  double G[2][J2][J2 + 4];   // row padding: fewer LDS bank conflicts in the rounds (measured)
-  double Q[2][J2][J2 + 1];
-  double red[4];
+  // the pair Gram in circle positions (eig_pos), ping-pong over the rounds
+  __attribute__((aligned(16))) double G[2][J2][J2 + GPAD];
+  __attribute__((aligned(16))) double cs[2][JB][2];  // (c, s) of the 16 rotations of a round
+  double Q[J2][J2 + 1];
+  float red[EIG_NW];
+  int wide;  // a squared norm beyond 2^(+-EIG_RANGE): the rounds scale every pair
 };
+
+// Circle position of index v: slot s holds the pair (s, 31 - s), its first
+// member at position 2 s and its second at 2 s + 1.
+__device__ __forceinline__ int eig_pos(int v) { return v < JB ? 2 * v : 2 * (J2 - 1 - v) + 1; }
 
 // Largest normalised off-diagonal over the pair, encoded for atomicMax.
 __device__ __forceinline__ unsigned long long dbits(double x) {
@@ -78,27 +92,38 @@ __device__ __forceinline__ bool pair_rotates(double gpq, double gpp, double gqq,
 // negligible vectors (squared norms <= neg2) are left out: the caller has
 // shown that the space they span lies below its truncation threshold
 // whether or not they are orthogonalised (neg2 = 0: every pair).
-// Block-uniform.
+// Block-uniform.  Also leaves in sm whether eig_rotate has to scale the pairs.
 __device__ inline double eig_off(EigLds& sm, double tol, double neg2 = 0.0) {
   const int tid = threadIdx.x;
   const float above = (float)tol * (1.0f + 0x1p-20f) + 0x1p-126f;
   float off = 0.0f;
-  for (int e = tid; e < J2 * J2; e += 256) {
-    const int p = e / J2, q = e % J2;
-    if (p < q) {
-      double spq, spp, sqq;
-      const bool rot = pair_rotates(sm.G[0][p][q], sm.G[0][p][p], sm.G[0][q][q], tol, neg2, spq,
-                                    spp, sqq);
-      // (float)(spp sqq) may flush to 0: rsq then gives inf (or NaN for a
-      // zero spq), which fminf clamps
-      const float v = fminf(fabsf((float)spq) * __builtin_amdgcn_rsqf((float)(spp * sqq)), 1e30f);
-      if (rot) off = fmaxf(off, fmaxf(v, above));
-    }
+  // one pair a thread: the 31 rounds of 16 circle pairs
+  if (tid < (J2 - 1) * JB) {
+    const int r = tid >> 4, sl = tid & 15;
+    const int va = sl == 0 ? 0 : 1 + (sl - 1 + r) % (J2 - 1), vb = 1 + (J2 - 2 - sl + r) % (J2 - 1);
+    const int p = eig_pos(va), q = eig_pos(vb);
+    double spq, spp, sqq;
+    const bool rot = pair_rotates(sm.G[0][p][q], sm.G[0][p][p], sm.G[0][q][q], tol, neg2, spq,
+                                  spp, sqq);
+    // (float)(spp sqq) may flush to 0: rsq then gives inf (or NaN for a
+    // zero spq), which fminf clamps
+    const float v = fminf(fabsf((float)spq) * __builtin_amdgcn_rsqf((float)(spp * sqq)), 1e30f);
+    if (rot) off = fmaxf(v, above);
   }
   off = wave_max_dpp(off);
   if ((tid & 63) == 0) sm.red[tid >> 6] = off;
+  if (tid >= EIG_NT - 64) {
+    // the last wave (its lanes carry the fewest pairs): the largest exponent,
+    // in magnitude, of the nonzero squared norms
+    const double d = sm.G[0][tid & 31][tid & 31];
+    const int ex = d > 0.0 ? abs(__builtin_amdgcn_frexp_exp(d)) : 0;
+    const float far = wave_max_dpp((float)ex);
+    if ((tid & 63) == 0) sm.wide = far > (float)EIG_RANGE ? 1 : 0;
+  }
   lds_barrier();
-  off = fmaxf(fmaxf(sm.red[0], sm.red[1]), fmaxf(sm.red[2], sm.red[3]));
+  off = 0.0f;
+#pragma unroll
+  for (int w = 0; w < EIG_NW; ++w) off = fmaxf(off, sm.red[w]);
   lds_barrier();
   return (double)off;
 }
@@ -152,11 +177,11 @@ __device__ __forceinline__ void rot_coef_v(double gpq, double gpp, double gqq, b
   b = rot ? (x_is_l ? -sn : sn) : 0.0;
 }
 
-// v from the lane whose byte address (4 * lane) is addr, within the wave.
-__device__ __forceinline__ double lane_fetch(int addr, double v) {
+// v of the first lane of this lane's row of 16 (DPP row_newbcast:0)
+__device__ __forceinline__ double dpp_row_first(double v) {
   const long long u = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_ds_bpermute(addr, (int)(unsigned)u);
-  const int hi = __builtin_amdgcn_ds_bpermute(addr, (int)(u >> 32));
+  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, 0x150, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(u >> 32), 0x150, 0xf, 0xf, true);
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
@@ -175,45 +200,124 @@ __device__ __forceinline__ double dpp_from_prev(double v) {
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+// rot_coef_v(..., x_is_l = true) for Gram entries whose products stay in
+// range (EIG_RANGE), on a shorter chain: no scaling, the hypotenuse and the
+// tangent from v_rsq_f64 and v_rcp_f64 (about 2^-23 relative, as good as the
+// FP32 angle), and c from v_rsq_f64 by one third-order step,
+// y (1 + e / 2 + 3 e^2 / 8) with e = 1 - x y^2 (relative error about e^3 / 3,
+// below 2^-65).
+__device__ __forceinline__ void rot_coef_n(double gpq, double gpp, double gqq, double tol2,
+                                           double neg2, double& a, double& b) {
+  const bool rot = gpq * gpq > tol2 * gpp * gqq && fmax(gpp, gqq) > neg2;
+  const double D = gqq - gpp, P = gpq + gpq;
+  const double h2 = fma(D, D, P * P);
+  const double hyp = h2 * __builtin_amdgcn_rsq(h2);
+  const double tp = P * __builtin_amdgcn_rcp(fabs(D) + hyp);
+  // -t: the sign of P, flipped where D is not negative
+  const long long flip = ~__double_as_longlong(D) & (long long)0x8000000000000000ull;
+  const double u = __longlong_as_double(__double_as_longlong(tp) ^ flip);
+  const double x = fma(u, u, 1.0);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  const double c = fma(y * e, fma(e, 0.375, 0.5), y);
+  a = rot ? c : 1.0;
+  b = rot ? u * c : 0.0;
+}
+
 // One cyclic sweep (31 rounds of 16 disjoint rotations, circle order) of the
-// two-sided Jacobi on G, accumulating Q = J_1 ... J_31, one barrier per
-// round.  Thread t (row pair rp = t/16, column pair cp = t%16) owns the 2x2
-// block of G' = J^T G J at rows (x0, x1) and columns (y0, y1), the circle
-// slots of rp and cp (G ping-pongs between two LDS buffers), and rows 2 rp,
-// 2 rp + 1 of Q at the columns of its slots, in registers: Q' = Q J only
-// mixes columns, and the circle moves a column between neighbouring column
-// slots (first slots from lane cp + 1 to cp, second slots from cp - 1 to cp,
-// slot 1-first to 0-second, 15-second to 15-first, vector 0 fixed), which
-// stay within the lane's DPP row of 16 lanes.  Each lane computes the
-// rotation of its column pair from the LDS values; the rotation of its row
-// pair is the one computed by the lane of the same 16-lane row whose column
-// pair it is (fetched across the wave, so row and column rotations of a pair
-// are the same bits).  One inner sweep per outer step: the outer block
+// two-sided Jacobi on G, accumulating Q = J_1 ... J_31, by 8 waves and one
+// barrier per round.  One inner sweep per outer step: the outer block
 // iteration needs the same number of sweeps with one inner sweep as with
-// full inner convergence (measured), at a fraction of the cost.  Q is left
-// in sm.Q[0]; returns that buffer's index (0).
-__device__ inline int eig_rotate(EigLds& sm, double tol, double neg2 = 0.0) {
-  auto& G = sm.G;
-  const int tid = threadIdx.x;
-  const int rp = tid >> 4, cp = tid & 15;
-  const int src = ((tid & 0x30) | rp) << 2;   // lane of this row with column pair rp
-  int cur = 0;
-  // circle positions, advanced by one (mod 31, in 1..31) each round; after
-  // 31 rounds every slot holds its first vector again
-  int x0 = rp == 0 ? 0 : rp, x1 = J2 - 1 - rp, y0 = cp == 0 ? 0 : cp, y1 = J2 - 1 - cp;
+// full inner convergence (measured), at a fraction of the cost.
+//
+// A round is one dependent chain (the pair's entries, the rotation, the
+// update, the exchange), so what bounds it is the chain's instructions and
+// LDS trips, and the layout keeps everything else off it:
+//  * waves 0-3 carry G.  G lies in LDS in circle positions, where a round's
+//    moves are the same for every round: a lane reads its 2 x 2 block (row
+//    pair rp, column pair cp) and its column pair's diagonal block from fixed
+//    addresses and writes the updated block to the fixed addresses it moves
+//    to.  Lane l of the 16-lane row of row pair rp owns column pair
+//    (l + rp) mod 16, so the rotation of the row pair is always in the row's
+//    first lane and reaches the row by a DPP broadcast (row and column
+//    rotations of a pair are the same bits) instead of an LDS permute.
+//  * waves 4-7 carry Q, one round behind, from the (c, s) that wave 0 leaves
+//    in LDS: Q' = Q J only mixes columns, and the circle moves a column
+//    between neighbouring column slots (first slots from lane cp + 1 to cp,
+//    second slots from cp - 1 to cp, slot 1-first to 0-second, 15-second to
+//    15-first, vector 0 fixed), which stay within the lane's DPP row of 16.
+//    Their work fills the issue slots that the G waves' latencies leave.
+// Measured (in-kernel clock, n = 1024): 1220 cycles a round with one group of
+// four waves for G and Q on index-ordered LDS and an LDS permute for the row
+// rotations, 797 in this layout, 719 with rot_coef_n's shorter chain; of
+// those the coefficients are 250, the reads 75, the 16 products and the DPP
+// moves 120, the writes 130, the barrier and the loop the rest, and the Q
+// waves nothing.  jac_eig_apply at n = 256 with Z 17.8 -> 12.4 us, at
+// 512 x 2560 SVDs 31.8 -> 20.5 us.  A conflict-free split of the positions
+// (first members 0-15, second 16-31, rows 32 banks apart, 8-byte accesses)
+// measured the same 725 cycles: the accesses' number, not conflicts, counts.
+// Pairs are rotated down to a quarter of tol, the convergence measure counts
+// those above tol: a sweep then leaves none just under tol, which the next
+// measure, rounded differently, may find above it (eigensolves at n = 1024
+// otherwise run a sweep that rotates next to nothing one time in two).
+// Q is left in sm.Q.
+struct EigSlots {  // a G lane's fixed places: rows and columns of its block, and where they move
+  int rp, cp, r0, r1, c0, c1;
+  __device__ explicit EigSlots(int tid) {
+    rp = tid >> 4;
+    cp = ((tid & 15) + rp) & 15;
+    r0 = rp == 0 ? 0 : (rp == 1 ? 1 : 2 * (rp - 1));
+    r1 = rp == 15 ? 30 : 2 * (rp + 1) + 1;
+    c0 = cp == 0 ? 0 : (cp == 1 ? 1 : 2 * (cp - 1));
+    c1 = cp == 15 ? 30 : 2 * (cp + 1) + 1;
+  }
+};
+
+// The G waves' side of the rounds; coef(gpq, gpp, gqq, c, s): the rotation of
+// a pair.
+template <typename Coef>
+__device__ __forceinline__ void eig_rounds_g(EigLds& sm, Coef coef) {
+  const EigSlots z(threadIdx.x);
+  constexpr int LD = J2 + GPAD;
+  const int ix0 = 2 * z.rp * LD + 2 * z.cp, ix1 = ix0 + LD, iy = 2 * z.cp * LD + 2 * z.cp;
+  const int o00 = z.r0 * LD + z.c0, o01 = z.r0 * LD + z.c1;
+  const int o10 = z.r1 * LD + z.c0, o11 = z.r1 * LD + z.c1;
+  auto round = [&](const double* g, double* h, double* cs) {
+    const double2 y0 = *(const double2*)(g + iy);
+    const double yqq = g[iy + LD + 1];
+    const double2 g0 = *(const double2*)(g + ix0), g1 = *(const double2*)(g + ix1);
+    // (c, s) for the first member of each pair; the second's s is -s
+    double cy, sy;
+    coef(y0.y, y0.x, yqq, cy, sy);
+    if (threadIdx.x < 16) *(double2*)(cs + 2 * z.cp) = double2{cy, sy};
+    const double cx = dpp_row_first(cy), sx = dpp_row_first(sy);
+    const double r00 = cx * g0.x + sx * g1.x, r01 = cx * g0.y + sx * g1.y;
+    const double r10 = cx * g1.x - sx * g0.x, r11 = cx * g1.y - sx * g0.y;
+    h[o00] = cy * r00 + sy * r01;
+    h[o01] = cy * r01 - sy * r00;
+    h[o10] = cy * r10 + sy * r11;
+    h[o11] = cy * r11 - sy * r10;
+    lds_barrier();
+  };
+  double* const ga = &sm.G[0][0][0];
+  double* const gb = &sm.G[1][0][0];
+  for (int r = 0; r < J2 - 2; r += 2) {
+    round(ga, gb, &sm.cs[0][0][0]);
+    round(gb, ga, &sm.cs[1][0][0]);
+  }
+  round(ga, gb, &sm.cs[0][0][0]);
+}
+
+// The Q waves' side of the rounds.
+__device__ __forceinline__ void eig_rounds_q(EigLds& sm) {
+  const int t = threadIdx.x - 256, rp = t >> 4, cp = t & 15;
+  const int y0 = cp, y1 = J2 - 1 - cp;
   const int R0 = 2 * rp, R1 = 2 * rp + 1;
   double qa0 = R0 == y0 ? 1.0 : 0.0, qa1 = R0 == y1 ? 1.0 : 0.0;   // Q[R0][y0], Q[R0][y1]
   double qb0 = R1 == y0 ? 1.0 : 0.0, qb1 = R1 == y1 ? 1.0 : 0.0;   // Q[R1][y0], Q[R1][y1]
-  for (int r = 0; r < J2 - 1; ++r) {
-    const int nxt = cur ^ 1;
-    const int yl = min(y0, y1), yh = max(y0, y1);
-    const double ypq = G[cur][yl][yh], ypp = G[cur][yl][yl], yqq = G[cur][yh][yh];
-    const double g00 = G[cur][x0][y0], g01 = G[cur][x0][y1];
-    const double g10 = G[cur][x1][y0], g11 = G[cur][x1][y1];
-    // (c, b) for the first index of each pair; the partner's b is -b
-    double cy, sy;
-    rot_coef_v(ypq, ypp, yqq, y0 == yl, tol, neg2, cy, sy);
-    const double cx = lane_fetch(src, cy), sx = lane_fetch(src, sy);
+  auto step = [&](int b) {
+    const double2 v = *(const double2*)&sm.cs[b][cp][0];
+    const double cy = v.x, sy = v.y;
     // Q' = Q J on the column pair, then the circle shift of the columns
     const double na0 = cy * qa0 + sy * qa1, na1 = cy * qa1 - sy * qa0;
     const double nb0 = cy * qb0 + sy * qb1, nb1 = cy * qb1 - sy * qb0;
@@ -223,29 +327,39 @@ __device__ inline int eig_rotate(EigLds& sm, double tol, double neg2 = 0.0) {
     qb0 = cp == 0 ? nb0 : (cp == 15 ? nb1 : fb);
     qa1 = cp == 0 ? fa : pa;
     qb1 = cp == 0 ? fb : pb;
-    const double bX0 = sx, bX1 = -sx, bY0 = sy, bY1 = -sy;
-    const double r00 = cx * g00 + bX0 * g10, r01 = cx * g01 + bX0 * g11;
-    const double r10 = cx * g10 + bX1 * g00, r11 = cx * g11 + bX1 * g01;
-    G[nxt][x0][y0] = cy * r00 + bY0 * r01;
-    G[nxt][x0][y1] = cy * r01 + bY1 * r00;
-    G[nxt][x1][y0] = cy * r10 + bY0 * r11;
-    G[nxt][x1][y1] = cy * r11 + bY1 * r10;
-    cur = nxt;
-    if (x0 != 0) x0 = x0 == J2 - 1 ? 1 : x0 + 1;
-    x1 = x1 == J2 - 1 ? 1 : x1 + 1;
-    if (y0 != 0) y0 = y0 == J2 - 1 ? 1 : y0 + 1;
-    y1 = y1 == J2 - 1 ? 1 : y1 + 1;
+  };
+  lds_barrier();
+  for (int r = 0; r < J2 - 2; r += 2) {
+    step(0);
+    lds_barrier();
+    step(1);
     lds_barrier();
   }
-  sm.Q[0][R0][y0] = qa0;
-  sm.Q[0][R0][y1] = qa1;
-  sm.Q[0][R1][y0] = qb0;
-  sm.Q[0][R1][y1] = qb1;
-  lds_barrier();
-  return 0;
+  step(0);
+  // after 31 rounds every slot holds its first members again
+  sm.Q[R0][y0] = qa0;
+  sm.Q[R0][y1] = qa1;
+  sm.Q[R1][y0] = qb0;
+  sm.Q[R1][y1] = qb1;
 }
 
-// Rows [rs, re) (re - rs <= 64 NT) of the pair's 32 vectors (vector v at
+__device__ inline void eig_rotate(EigLds& sm, double tol, double neg2 = 0.0) {
+  if (threadIdx.x >= 256) {
+    eig_rounds_q(sm);
+  } else if (__builtin_amdgcn_readfirstlane(sm.wide)) {
+    eig_rounds_g(sm, [&](double gpq, double gpp, double gqq, double& c, double& s) {
+      rot_coef_v(gpq, gpp, gqq, true, 0.25 * tol, neg2, c, s);
+    });
+  } else {
+    const double tol2 = (0.25 * tol) * (0.25 * tol);
+    eig_rounds_g(sm, [&](double gpq, double gpp, double gqq, double& c, double& s) {
+      rot_coef_n(gpq, gpp, gqq, tol2, neg2, c, s);
+    });
+  }
+  lds_barrier();
+}
+
+// Rows [rs, re) (re - rs <= 16 NT NW, NW waves) of the pair's 32 vectors (vector v at
 // base + v * ld, nv vectors) <- rows . Q, as the transposed product
 // (Q^T X^T) on v_mfma_f64_16x16x4: the B operand of each 16 x 16 output tile
 // is 16 consecutive rows of 4 vectors, read straight from memory (four
@@ -258,21 +372,21 @@ __device__ inline int eig_rotate(EigLds& sm, double tol, double neg2 = 0.0) {
 //                      the caller computes Q);
 //   apply_rows_finish: 16 NT MFMAs per wave (2 vector tiles x NT row tiles x
 //                      8 k-steps) and the stores.
-// Whether the chunk is a whole 64 NT rows and all 32 vectors of the pair
+// Whether the chunk is a whole 16 NT NW rows and all 32 vectors of the pair
 // exist (block-uniform): then the loads and stores need no bounds test.
-template <int NT>
+template <int NT, int NW>
 __device__ __forceinline__ bool apply_rows_full(int64_t nv, int64_t rs, int64_t re, int I, int J) {
-  return re - rs == 64 * NT && (int64_t)max(I, J) * JB + JB <= nv;
+  return re - rs == 16 * NT * NW && (int64_t)max(I, J) * JB + JB <= nv;
 }
 
-template <int NT>
+template <int NT, int NW>
 __device__ __forceinline__ void apply_rows_fetch(const double* __restrict__ base, int64_t ld,
                                                  int64_t nv, int64_t rs, int64_t re, int I,
                                                  int J, double (&x)[8][NT]) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int lr = lane & 15, lk = lane >> 4;
   const int64_t r0 = rs + 16 * NT * wave + lr;
-  if (apply_rows_full<NT>(nv, rs, re, I, J)) {
+  if (apply_rows_full<NT, NW>(nv, rs, re, I, J)) {
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
       const double* p = base + pair_vec(4 * ks + lk, I, J) * ld + r0;
@@ -292,7 +406,7 @@ __device__ __forceinline__ void apply_rows_fetch(const double* __restrict__ base
   }
 }
 
-template <int NT>
+template <int NT, int NW>
 __device__ __forceinline__ void apply_rows_finish(double* __restrict__ base, int64_t ld,
                                                   int64_t nv, int64_t rs, int64_t re, int I,
                                                   int J, const double (&x)[8][NT],
@@ -317,7 +431,7 @@ __device__ __forceinline__ void apply_rows_finish(double* __restrict__ base, int
     }
   }
   // output tile (mt, nt): lane holds vector 16 mt + lk + 4 e, row 16 nt + lr
-  if (apply_rows_full<NT>(nv, rs, re, I, J)) {
+  if (apply_rows_full<NT, NW>(nv, rs, re, I, J)) {
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll

@@ -32,14 +32,15 @@
 
 namespace tn {
 
-// Rows per chunk of jac_eig_apply: 64 NT with NT = 2 (128 rows), or NT = 4
-// (256 rows) when 128-row chunks would put more than two blocks on a CU:
-// the blocks' rotation rounds then share the SIMDs' issue slots and stop
-// being latency-bound (n = 2048: 64 pairs x 8 chunks of 256 instead of 16
-// chunks of 128).
-constexpr int kEigResident = 512;
+// Rows per chunk of jac_eig_apply: 128 NT, the smallest NT that keeps the
+// launch at one 8-wave block per CU: two blocks on a CU share the SIMDs'
+// issue slots, so their rotation rounds stop being latency-bound.
+constexpr int kEigResident = 256;
 static int eig_nt(int npairs, int64_t L, int64_t kz) {
-  return (int64_t)npairs * (ceil_div(L, 128) + ceil_div(kz, 128)) <= kEigResident ? 2 : 4;
+  int nt = 1;
+  while (nt < 4 && (int64_t)npairs * (ceil_div(L, 128 * nt) + ceil_div(kz, 128 * nt)) > kEigResident)
+    nt *= 2;
+  return nt;
 }
 constexpr int GCH = 128;     // rows per Gram partial of jac_gram (twice the blocks)
 
@@ -96,39 +97,39 @@ __device__ void gram_partial(double (*Ps)[64][J2 + 1], const double* __restrict_
 }
 
 // G (sm.G[0]) = sum of the pair's nchunk partials (fixed order, so every
-// block that sums them gets the same bits); Q (sm.Q[0]) = I.  The partials
-// are read four chunks at a time with every load issued before the first
-// add: a load-add chain would pay one memory latency per partial element.
+// block that sums them gets the same bits).  The partials are read eight
+// chunks at a time with every load issued before the first add: a load-add
+// chain would pay one memory latency per partial element.
 __device__ void eig_load(EigLds& sm, const double* __restrict__ Gp, int nchunk) {
-  constexpr int PER = J2 * J2 / 256;  // elements per thread
+  constexpr int PER = J2 * J2 / EIG_NT;  // elements per thread
+  constexpr int U = 8;
   double acc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) acc[i] = 0.0;
   int c = 0;
-  for (; c + 4 <= nchunk; c += 4) {
-    double v[4][PER];
+  for (; c + U <= nchunk; c += U) {
+    double v[U][PER];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < PER; ++i)
-        v[u][i] = Gp[(int64_t)(c + u) * (J2 * J2) + threadIdx.x + 256 * i];
+        v[u][i] = Gp[(int64_t)(c + u) * (J2 * J2) + threadIdx.x + EIG_NT * i];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < PER; ++i) acc[i] += v[u][i];
   }
   for (; c < nchunk; ++c) {
     double v[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) v[i] = Gp[(int64_t)c * (J2 * J2) + threadIdx.x + 256 * i];
+    for (int i = 0; i < PER; ++i) v[i] = Gp[(int64_t)c * (J2 * J2) + threadIdx.x + EIG_NT * i];
 #pragma unroll
     for (int i = 0; i < PER; ++i) acc[i] += v[i];
   }
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int e = threadIdx.x + 256 * i;
-    sm.G[0][e / J2][e % J2] = acc[i];
-    sm.Q[0][e / J2][e % J2] = (e / J2 == e % J2) ? 1.0 : 0.0;
+    const int e = threadIdx.x + EIG_NT * i;
+    sm.G[0][eig_pos(e / J2)][eig_pos(e % J2)] = acc[i];
   }
   lds_barrier();
 }
@@ -153,12 +154,12 @@ __global__ void __launch_bounds__(256) jac_gram(const double* __restrict__ Wv, i
 // chunk costs nothing in latency and saves a launch and the Q round trip
 // through memory.
 template <int NT>
-__global__ void __launch_bounds__(256) jac_eig_apply(double* __restrict__ Wv, int64_t L,
+__global__ void __launch_bounds__(EIG_NT) jac_eig_apply(double* __restrict__ Wv, int64_t L,
                                                      double* __restrict__ Z, int64_t nv, int s,
                                                      int nblk, int nchW, int nchG,
                                                      const double* __restrict__ Gpart, double tol,
                                                      unsigned long long* __restrict__ offmax) {
-  constexpr int CH = 64 * NT;
+  constexpr int CH = 16 * EIG_NW * NT;
   __shared__ EigLds sm;
   const int pi = blockIdx.x, ch = blockIdx.y;
   int I, J;
@@ -172,12 +173,12 @@ __global__ void __launch_bounds__(256) jac_eig_apply(double* __restrict__ Wv, in
   }
   eig_load(sm, Gpart + (int64_t)pi * nchG * (J2 * J2), nchG);
   double x[8][NT];
-  apply_rows_fetch<NT>(base, ld, nv, rs, re, I, J, x);   // in flight during the rounds
+  apply_rows_fetch<NT, EIG_NW>(base, ld, nv, rs, re, I, J, x);   // in flight during the rounds
   const double off = eig_off(sm, tol);
   if (ch == 0 && threadIdx.x == 0) atomicMax(offmax, dbits(off));
   if (off <= tol) return;
-  const int cur = eig_rotate(sm, tol);
-  apply_rows_finish<NT>(base, ld, nv, rs, re, I, J, x, sm.Q[cur]);
+  eig_rotate(sm, tol);
+  apply_rows_finish<NT, EIG_NW>(base, ld, nv, rs, re, I, J, x, sm.Q);
 }
 
 // Convergence of the whole vector set from its Gram matrix G = Wv^T Wv
@@ -413,7 +414,7 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   // Z == nullptr: the rotations are not accumulated (eigensolver use)
   const int64_t kz0 = Z ? k : 0;
   const int ent = eig_nt(npairs, L, kz0);
-  const int nchW = (int)ceil_div(L, 64 * ent), nchZ = Z ? (int)ceil_div(k, 64 * ent) : 0;
+  const int nchW = (int)ceil_div(L, 128 * ent), nchZ = Z ? (int)ceil_div(k, 128 * ent) : 0;
   const int nchG = (int)ceil_div(L, GCH);
   const int64_t kz = Z ? k : 0;
   if (Z)
@@ -457,12 +458,16 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
         // chunks read and written
         ProfScope p(PROF_JAC_EIG, st, 31.0 * 9216.0 * npairs + apply_fl,
                     8.0 * (double)nchG * J2 * J2 * npairs + 16.0 * (double)(L + kz) * J2 * npairs);
-        if (ent == 2)
-          hipLaunchKernelGGL(jac_eig_apply<2>, dim3(npairs, nchW + nchZ), dim3(256), 0, st, Wv,
-                             L, Z, k, s, nblk, nchW, nchG, w.Gpart, tol, w.off);
+        const dim3 eg(npairs, nchW + nchZ);
+        if (ent == 1)
+          hipLaunchKernelGGL(jac_eig_apply<1>, eg, dim3(EIG_NT), 0, st, Wv, L, Z, k, s, nblk, nchW,
+                             nchG, w.Gpart, tol, w.off);
+        else if (ent == 2)
+          hipLaunchKernelGGL(jac_eig_apply<2>, eg, dim3(EIG_NT), 0, st, Wv, L, Z, k, s, nblk, nchW,
+                             nchG, w.Gpart, tol, w.off);
         else
-          hipLaunchKernelGGL(jac_eig_apply<4>, dim3(npairs, nchW + nchZ), dim3(256), 0, st, Wv,
-                             L, Z, k, s, nblk, nchW, nchG, w.Gpart, tol, w.off);
+          hipLaunchKernelGGL(jac_eig_apply<4>, eg, dim3(EIG_NT), 0, st, Wv, L, Z, k, s, nblk, nchW,
+                             nchG, w.Gpart, tol, w.off);
       }
     }
     TN_CHECK_LAUNCH();
