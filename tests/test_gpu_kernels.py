@@ -189,3 +189,31 @@ def test_contract_with_non_fusing_operands(L, prec, tol):
     Ct = dev(C.transpose(1, 0, 3, 2).copy()).permute(1, 0, 3, 2)
     F2 = T._contract_data(dev(E), [0, 1], Ct, [0, 2], prec)
     assert np.abs(F2.double().cpu().numpy() - F_ref).max() <= tol * scale * 10
+
+
+# The split-bf16 product on its 16-byte-load path and beside it: edges of the
+# 128 x 128 x 32 tile, the four operand layouts, odd row pitches and bases
+# that are only 4-byte aligned.  Per product of x and y the split keeps
+# |x y| (1 + d) with |d| <= 3 * 2^-18 (each half rounds to 8 bits, lo * lo is
+# dropped), FP32 accumulation adds at most (3 K + 8) 2^-24 of sum |x y|.
+@pytest.mark.parametrize("M,K,N", [(128, 128, 128), (129, 97, 131), (127, 33, 257), (300, 31, 70),
+                                   (70, 1000, 41), (1030, 64, 1021)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+def test_contract_bf16x3_tiles(L, M, K, N, layout):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(M + 3 * K + 7 * N)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = rng.standard_normal((K, N)).astype(np.float32)
+
+    def strided(x, t):  # x as a view into a larger buffer, row pitch + 3, base + 1
+        y = x.T if t else x
+        buf = torch.zeros(y.shape[0] * (y.shape[1] + 3) + 1, dtype=torch.float32, device="cuda")
+        v = buf[1:].view(y.shape[0], y.shape[1] + 3)[:, :y.shape[1]]
+        v.copy_(torch.from_numpy(np.ascontiguousarray(y)))
+        return v.T if t else v
+
+    c = T._contract_data(strided(a, layout[0] == "t"), [1], strided(b, layout[1] == "t"), [0],
+                         precision="bf16x3").cpu().numpy().astype(np.float64)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    bound = (3 * 2.0 ** -18 + (3 * K + 8) * 2.0 ** -24) * (np.abs(a) @ np.abs(b))
+    assert np.all(np.abs(c - a @ b) <= bound)

@@ -241,27 +241,77 @@ __global__ void __launch_bounds__(NT, 2) gemm_mfma_kernel(GemmArgs g) {
 
 // ------------------------------------------------------------ BF16x3
 // LDS layout [row][BK + 8] bf16 (k contiguous): lane l of a 16x16x32 MFMA
-// reads 8 consecutive k of row l%16 starting at k = 8*(l/16).
+// reads 8 consecutive k of row l%16 starting at k = 8*(l/16).  The 80-byte
+// row pitch spreads 16 rows' 16-byte reads, and the 8-byte stores of either
+// tile mapping, over all 64 banks.
+//
+// What bounds it: three MFMAs per product and, next to them, the LDS traffic
+// of four bf16 tiles.  Each FP32 operand is split once per block, in
+// registers, on its way to LDS; two LDS buffers, so a k-tile needs one
+// barrier and the next tile's loads are in flight during the MFMAs.  VEC
+// (single-mode operands, each with a unit-stride dimension, offsets below
+// 2^31): a thread loads 4 x 4 elements of each operand by four 16-byte loads
+// (4-byte alignment is enough for them) -- rows of 4 k where k is the unit
+// stride, else 4 k rows of 4 columns, transposed in registers -- and stores
+// runs of 4 k.  2560 x 2560 x 5110: 1194 -> 342 us (56 -> 196 TFLOP/s
+// FP32-equivalent; its 800 tiles fill 3.1 of 4 rounds of the CUs); 4096^3: 74
+// -> 275-308 TFLOP/s, i.e. 825-925 TFLOP/s of bf16 MFMA.  Operands that need
+// the mode tables stay on scalar loads and one LDS buffer (two would leave
+// one block per CU).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ void split_bf16(float x, __bf16& hi, __bf16& lo) {
   hi = (__bf16)x;
   lo = (__bf16)(x - (float)hi);
 }
 
-__global__ void __launch_bounds__(NT) gemm_bf16x3_kernel(GemmArgs g) {
+__device__ __forceinline__ void split_bf16x4(f32x4 x, bf16x4& hi, bf16x4& lo) {
+  hi = __builtin_convertvector(x, bf16x4);
+  lo = __builtin_convertvector(x - __builtin_convertvector(hi, f32x4), bf16x4);
+}
+
+// Tile (x, y) of a launch: consecutive workgroups go to the eight XCDs in
+// turn, so XCD c takes the c-th eighth of the tiles, in column strips of
+// eight row tiles: what one XCD works on at a time shares its operands in
+// that XCD's L2.
+__device__ __forceinline__ void xcd_tile(int& tx, int& ty) {
+  const int nx = gridDim.x, ny = gridDim.y, total = nx * ny;
+  int id = blockIdx.y * nx + blockIdx.x;
+  tx = blockIdx.x;
+  ty = blockIdx.y;
+  if (total < 64) return;
+  const int per = total / 8, rem = total % 8, c = id % 8;
+  id = c * per + min(c, rem) + id / 8;
+  constexpr int GY = 8;
+  const int strip = id / (GY * nx), r0 = strip * GY, h = min(GY, ny - r0);
+  const int in = id - r0 * nx;
+  ty = r0 + in % h;
+  tx = in / h;
+}
+
+template <bool VEC, int AKF, int BNF>
+__global__ void __launch_bounds__(NT, VEC ? 2 : 1) gemm_bf16x3_kernel(GemmArgs g) {
   constexpr int BK = 32;
   constexpr int LD = BK + 8;
   constexpr int EPT = BM * BK / NT;  // 16
-  __shared__ __attribute__((aligned(16))) __bf16 Ah[BM * LD], Al[BM * LD];
-  __shared__ __attribute__((aligned(16))) __bf16 Bh[BN * LD], Bl[BN * LD];
-  __shared__ int64_t rowA[BM], colB[BN], rowC[BM], colC[BN];
+  // the table path keeps one buffer (and a second barrier), so that two
+  // blocks fit a CU's LDS next to the tables
+  constexpr int NB = VEC ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) __bf16 Ah[NB][BM * LD], Al[NB][BM * LD];
+  __shared__ __attribute__((aligned(16))) __bf16 Bh[NB][BN * LD], Bl[NB][BN * LD];
+  __shared__ int64_t rowA[VEC ? 1 : BM], colB[VEC ? 1 : BN], rowC[VEC ? 1 : BM],
+      colC[VEC ? 1 : BN];
   // the BK offsets of a k-tile, decoded once per tile, two tiles ahead
-  __shared__ int64_t kA[2][BK], kB[2][BK];
+  __shared__ int64_t kA[VEC ? 1 : 2][VEC ? 1 : BK], kB[VEC ? 1 : 2][VEC ? 1 : BK];
 
   const float* __restrict__ A = (const float*)g.A;
   const float* __restrict__ B = (const float*)g.B;
   float* __restrict__ C = (float*)g.C;
   const int tid = threadIdx.x;
-  const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
+  int tx, ty;
+  xcd_tile(tx, ty);
+  const int64_t m0 = (int64_t)ty * BM, n0 = (int64_t)tx * BN;
   const int64_t kbeg = (int64_t)blockIdx.z * g.kchunk;
   const int64_t kend = min(g.K, kbeg + g.kchunk);
   auto koffs = [&](int slot, int64_t k0) {
@@ -273,53 +323,115 @@ __global__ void __launch_bounds__(NT) gemm_bf16x3_kernel(GemmArgs g) {
       kB[slot][tid - BK] = k < kend ? goff(g.bk, k) : 0;
     }
   };
-  koffs(0, kbeg);
-  koffs(1, kbeg + BK);
-  for (int i = tid; i < BM; i += NT) {
-    int64_t m = m0 + i;
-    rowA[i] = m < g.M ? goff(g.am, m) : 0;
-    rowC[i] = m < g.M ? goff(g.cm, m) : 0;
-  }
-  for (int i = tid; i < BN; i += NT) {
-    int64_t n = n0 + i;
-    colB[i] = n < g.N ? goff(g.bn, n) : 0;
-    colC[i] = n < g.N ? goff(g.cn, n) : 0;
-  }
-  __syncthreads();
-
-  float ra[EPT], rb[EPT];
-  auto load = [&](int64_t k0, int slot) {
-#pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      int e = tid + NT * j;
-      int r, kk;
-      if (g.a_kfast) { kk = e % BK; r = e / BK; } else { r = e % BM; kk = e / BM; }
-      int64_t m = m0 + r, k = k0 + kk;
-      ra[j] = (m < g.M && k < kend) ? A[rowA[r] + kA[slot][kk]] : 0.f;
+  if constexpr (!VEC) {
+    koffs(0, kbeg);
+    koffs(1, kbeg + BK);
+    for (int i = tid; i < BM; i += NT) {
+      int64_t m = m0 + i;
+      rowA[i] = m < g.M ? goff(g.am, m) : 0;
+      rowC[i] = m < g.M ? goff(g.cm, m) : 0;
     }
+    for (int i = tid; i < BN; i += NT) {
+      int64_t n = n0 + i;
+      colB[i] = n < g.N ? goff(g.bn, n) : 0;
+      colC[i] = n < g.N ? goff(g.cn, n) : 0;
+    }
+    __syncthreads();
+  }
+
+  // VEC: the operand's strides along its free index (f) and along k
+  const uint32_t saf = VEC && g.am.n ? (uint32_t)g.am.strides[0] : 0;
+  const uint32_t sak = VEC && g.ak.n ? (uint32_t)g.ak.strides[0] : 0;
+  const uint32_t sbf = VEC && g.bn.n ? (uint32_t)g.bn.strides[0] : 0;
+  const uint32_t sbk = VEC && g.bk.n ? (uint32_t)g.bk.strides[0] : 0;
+  const uint32_t scm = VEC && g.cm.n ? (uint32_t)g.cm.strides[0] : 0;
+  const uint32_t scn = VEC && g.cn.n ? (uint32_t)g.cn.strides[0] : 0;
+
+  f32x4 va[4], vb[4];
+  float ra[VEC ? 1 : EPT], rb[VEC ? 1 : EPT];
+  // Four 16-byte loads of a thread's part of a 128 x 32 tile.  KF (k unit
+  // stride): v[i] = 4 k at 4 (tid % 8) of row tid / 8 + 32 i.  Else: v[i] =
+  // rows 4 cg .. + 3 at k = 4 kg + i, cg = 8 (tid / 64) + tid % 8, kg = tid /
+  // 8 % 8 (a wave's eight lanes of one k read 128 bytes in a row).
+  auto vload = [&](const float* __restrict__ X, uint32_t sf, uint32_t sk, bool kf, int64_t f0,
+                   int64_t F, int64_t k0, f32x4 (&v)[4]) {
+    const bool full = f0 + 128 <= F && k0 + BK <= kend;
 #pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      int e = tid + NT * j;
-      int c, kk;
-      if (g.b_nfast) { c = e % BN; kk = e / BN; } else { kk = e % BK; c = e / BK; }
-      int64_t n = n0 + c, k = k0 + kk;
-      rb[j] = (n < g.N && k < kend) ? B[kB[slot][kk] + colB[c]] : 0.f;
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t f = kf ? tid / 8 + 32 * i : 4 * (8 * (tid / 64) + tid % 8);
+      const uint32_t k = kf ? 4 * (tid % 8) : 4 * (tid / 8 % 8) + i;
+      const float* p = X + (((uint32_t)f0 + f) * sf + ((uint32_t)k0 + k) * sk);
+      if (full) {
+        v[i] = *(const f32x4u*)p;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool in = kf ? (f0 + f < F && k0 + k + e < kend) : (f0 + f + e < F && k0 + k < kend);
+          v[i][e] = in ? p[e] : 0.f;
+        }
+      }
     }
   };
-  auto store = [&]() {
+  auto load = [&](int64_t k0, int slot) {
+    if constexpr (VEC) {
+      vload(A, saf, sak, AKF == 1, m0, g.M, k0, va);
+      vload(B, sbf, sbk, BNF == 0, n0, g.N, k0, vb);
+    } else {
 #pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      int e = tid + NT * j;
-      int r, kk;
-      if (g.a_kfast) { kk = e % BK; r = e / BK; } else { r = e % BM; kk = e / BM; }
-      split_bf16(ra[j], Ah[r * LD + kk], Al[r * LD + kk]);
+      for (int j = 0; j < EPT; ++j) {
+        int e = tid + NT * j;
+        int r, kk;
+        if (g.a_kfast) { kk = e % BK; r = e / BK; } else { r = e % BM; kk = e / BM; }
+        int64_t m = m0 + r, k = k0 + kk;
+        ra[j] = (m < g.M && k < kend) ? A[rowA[r] + kA[slot][kk]] : 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) {
+        int e = tid + NT * j;
+        int c, kk;
+        if (g.b_nfast) { c = e % BN; kk = e / BN; } else { kk = e % BK; c = e / BK; }
+        int64_t n = n0 + c, k = k0 + kk;
+        rb[j] = (n < g.N && k < kend) ? B[kB[slot][kk] + colB[c]] : 0.f;
+      }
     }
+  };
+  auto vstore = [&](bool kf, const f32x4 (&v)[4], __bf16* Xh, __bf16* Xl) {
 #pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      int e = tid + NT * j;
-      int c, kk;
-      if (g.b_nfast) { c = e % BN; kk = e / BN; } else { kk = e % BK; c = e / BK; }
-      split_bf16(rb[j], Bh[c * LD + kk], Bl[c * LD + kk]);
+    for (int i = 0; i < 4; ++i) {
+      f32x4 x;
+      int at;
+      if (kf) {
+        x = v[i];
+        at = (tid / 8 + 32 * i) * LD + 4 * (tid % 8);
+      } else {
+        x = f32x4{v[0][i], v[1][i], v[2][i], v[3][i]};
+        at = (4 * (8 * (tid / 64) + tid % 8) + i) * LD + 4 * (tid / 8 % 8);
+      }
+      bf16x4 hi, lo;
+      split_bf16x4(x, hi, lo);
+      *(bf16x4*)(Xh + at) = hi;
+      *(bf16x4*)(Xl + at) = lo;
+    }
+  };
+  auto store = [&](int buf) {
+    if constexpr (VEC) {
+      vstore(AKF == 1, va, Ah[buf], Al[buf]);
+      vstore(BNF == 0, vb, Bh[buf], Bl[buf]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) {
+        int e = tid + NT * j;
+        int r, kk;
+        if (g.a_kfast) { kk = e % BK; r = e / BK; } else { r = e % BM; kk = e / BM; }
+        split_bf16(ra[j], Ah[buf][r * LD + kk], Al[buf][r * LD + kk]);
+      }
+#pragma unroll
+      for (int j = 0; j < EPT; ++j) {
+        int e = tid + NT * j;
+        int c, kk;
+        if (g.b_nfast) { c = e % BN; kk = e / BN; } else { kk = e % BK; c = e / BK; }
+        split_bf16(rb[j], Bh[buf][c * LD + kk], Bl[buf][c * LD + kk]);
+      }
     }
   };
 
@@ -335,37 +447,39 @@ __global__ void __launch_bounds__(NT) gemm_bf16x3_kernel(GemmArgs g) {
   const int64_t nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
   if (nk > 0) {
     load(kbeg, 0);
-    store();
+    store(0);
     __syncthreads();
   }
+  int cur = 0;
   for (int64_t kt = 0; kt < nk; ++kt) {
     if (kt + 1 < nk) load(kbeg + (kt + 1) * BK, (int)((kt + 1) & 1));
     // tile kt + 2 reuses the slot tile kt's loads read (before the last barrier)
-    if (kt + 2 < nk) koffs((int)(kt & 1), kbeg + (kt + 2) * BK);
-    bf16x8 ah[4], al[4], bh[4], bl[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ah[i] = *(const bf16x8*)&Ah[(wr + 16 * i + lr) * LD + lk];
-      al[i] = *(const bf16x8*)&Al[(wr + 16 * i + lr) * LD + lk];
-    }
+    if (!VEC && kt + 2 < nk) koffs((int)(kt & 1), kbeg + (kt + 2) * BK);
+    bf16x8 bh[4], bl[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      bh[j] = *(const bf16x8*)&Bh[(wc + 16 * j + lr) * LD + lk];
-      bl[j] = *(const bf16x8*)&Bl[(wc + 16 * j + lr) * LD + lk];
+      bh[j] = *(const bf16x8*)&Bh[cur][(wc + 16 * j + lr) * LD + lk];
+      bl[j] = *(const bf16x8*)&Bl[cur][(wc + 16 * j + lr) * LD + lk];
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) {
+      const bf16x8 ah = *(const bf16x8*)&Ah[cur][(wr + 16 * i + lr) * LD + lk];
+      const bf16x8 al = *(const bf16x8*)&Al[cur][(wr + 16 * i + lr) * LD + lk];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-      }
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[j], acc[i][j], 0, 0, 0);
+    }
+    // the other buffer was last read before the previous barrier
+    if (!VEC) __syncthreads();
+    if (kt + 1 < nk) store(VEC ? cur ^ 1 : 0);
     __syncthreads();
-    if (kt + 1 < nk) {
-      store();
-      __syncthreads();
-    }
+    if (VEC) cur ^= 1;
   }
   const float alpha = (float)g.alpha, beta = (float)g.beta;
 #pragma unroll
@@ -381,7 +495,7 @@ __global__ void __launch_bounds__(NT) gemm_bf16x3_kernel(GemmArgs g) {
           if (g.part) {
             ((float*)g.part)[((int64_t)blockIdx.z * g.M + m) * g.N + n] = acc[i][j][e];
           } else {
-            float* p = C + rowC[r] + colC[c];
+            float* p = VEC ? C + ((uint32_t)m * scm + (uint32_t)n * scn) : C + rowC[r] + colC[c];
             float v = alpha * acc[i][j][e];
             if (g.beta != 0.0) v += beta * *p;
             *p = v;
@@ -742,6 +856,13 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
       (double)(M + BM) * st1(g.am) + (double)(K + 64) * st1(g.ak) < lim &&
       (double)(K + 64) * st1(g.bk) + (double)(N + BN) * st1(g.bn) < lim &&
       (double)(M + BM) * st1(g.cm) + (double)(N + BN) * st1(g.cn) < lim;
+  // operands with a unit stride along k or along their free index: 16-byte
+  // loads (negative strides, a size-1 operand axis or a stride-0 one take the
+  // table path)
+  const bool vak = st1(g.ak) == 1, vbk = st1(g.bk) == 1;
+  const bool vec = simple && st1(g.am) >= 0 && st1(g.ak) >= 0 && st1(g.bk) >= 0 &&
+                   st1(g.bn) >= 0 && st1(g.cm) >= 0 && st1(g.cn) >= 0 &&
+                   (vak || st1(g.am) == 1) && (vbk || st1(g.bn) == 1);
   // single-mode FP64 operands (the hot case): the tile-load mapping of each
   // operand is a template flag, so only one index mapping is live
   if (prec == P_F64 && simple && t64) {
@@ -770,8 +891,17 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
     hipLaunchKernelGGL((gemm_mfma_kernel<P_F32, true, -1, -1, 128>), grid, dim3(NT), 0, st, g);
   else if (prec == P_F32)
     hipLaunchKernelGGL((gemm_mfma_kernel<P_F32, false, -1, -1, 128>), grid, dim3(NT), 0, st, g);
-  else if (prec == P_BF16X3)
-    hipLaunchKernelGGL(gemm_bf16x3_kernel, grid, dim3(NT), 0, st, g);
+  else if (prec == P_BF16X3 && vec) {
+    if (vak && !vbk)
+      hipLaunchKernelGGL((gemm_bf16x3_kernel<true, 1, 1>), grid, dim3(NT), 0, st, g);
+    else if (vak)
+      hipLaunchKernelGGL((gemm_bf16x3_kernel<true, 1, 0>), grid, dim3(NT), 0, st, g);
+    else if (!vbk)
+      hipLaunchKernelGGL((gemm_bf16x3_kernel<true, 0, 1>), grid, dim3(NT), 0, st, g);
+    else
+      hipLaunchKernelGGL((gemm_bf16x3_kernel<true, 0, 0>), grid, dim3(NT), 0, st, g);
+  } else if (prec == P_BF16X3)
+    hipLaunchKernelGGL((gemm_bf16x3_kernel<false, -1, -1>), grid, dim3(NT), 0, st, g);
   else {
     set_error(TN_ERR_UNSUPPORTED, "contract: unknown precision %d", prec);
     return TN_ERR_UNSUPPORTED;
