@@ -217,3 +217,30 @@ def test_contract_bf16x3_tiles(L, M, K, N, layout):
     a, b = a.astype(np.float64), b.astype(np.float64)
     bound = (3 * 2.0 ** -18 + (3 * K + 8) * 2.0 ** -24) * (np.abs(a) @ np.abs(b))
     assert np.all(np.abs(c - a @ b) <= bound)
+
+
+# Small and few-output contractions with more than eight terms: every lane
+# count (4 to 256 per output), ranges split over blocks, several contracted
+# modes, permuted views.  A sum of K products in any order is within
+# (K + 4) u sum |a b| of the exact one.
+@pytest.mark.parametrize("shape_a,ax_a,shape_b,ax_b", [
+    ((3, 9), [1], (9, 5), [0]), ((16, 16), [1], (2, 16, 16), [1]), ((7, 63), [1], (63, 2), [0]),
+    ((5, 64), [1], (64, 3), [0]), ((4, 3, 5, 17), [3, 1], (3, 17, 6), [1, 0]),
+    ((13, 300), [1], (300, 11), [0]), ((2, 40, 3, 50), [1, 3], (40, 50, 4), [0, 1]),
+    ((4097,), [0], (4097,), [0]), ((3, 8191), [1], (8191, 1), [0]),
+    ((1, 70001), [1], (70001, 2), [0]), ((30, 40, 50), [0, 1, 2], (50, 30, 40), [1, 2, 0]),
+    ((600000,), [0], (600000,), [0])])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_contract_many_lanes_per_output(L, shape_a, ax_a, shape_b, ax_b, dtype):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(sum(shape_a) + sum(shape_b))
+    a, b = rng.standard_normal(shape_a).astype(dtype), rng.standard_normal(shape_b).astype(dtype)
+    # b as a view with its axes stored in reverse order
+    db = dev(b.transpose()).permute(*range(b.ndim - 1, -1, -1))
+    c = T._contract_data(dev(a), ax_a, db, ax_b).cpu().numpy()
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    K = int(np.prod([shape_a[i] for i in ax_a]))
+    ref, mag = np.tensordot(a, b, (ax_a, ax_b)), np.tensordot(np.abs(a), np.abs(b), (ax_a, ax_b))
+    # (plus the oracle's own FP64 rounding)
+    bound = (K + 4) * (np.finfo(dtype).eps / 2 + 2.0 ** -53) * mag
+    assert c.shape == ref.shape and np.all(np.abs(c - ref) <= bound)

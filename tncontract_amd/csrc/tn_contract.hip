@@ -12,9 +12,10 @@
 //  * contract_direct: one thread per output element, iterated in the
 //    output's memory order; used when K is small (e.g. the K = d = 2 MPO
 //    application), where the work is HBM-bound on the stores.  With 32-bit
-//    offsets and K <= 8 (the usual case) contract_direct32 decodes the
-//    output index by magic-number division and reads the contracted offsets
-//    from a host-built table.
+//    offsets (the usual case) contract_direct32 (K <= 8) decodes the output
+//    index by magic-number division and reads the contracted offsets from a
+//    host-built table, and contract_dot (K > 8: small products, and long ones
+//    with few outputs) puts several lanes on an output.
 #include "tn_internal.h"
 #include "tn_prof.h"
 
@@ -612,6 +613,111 @@ __global__ void __launch_bounds__(256) contract_direct32(Direct32Args g) {
   }
 }
 
+// The direct contraction with more than eight contracted terms: G lanes per
+// output (a power of two up to 64, or the block's 256), lane g taking every
+// G-th term, the lanes' sums added by shuffles (and through LDS for G = 256);
+// blockIdx.y splits the terms further into `kchunk`-long ranges whose sums go
+// to `part` (dense M x N per range, summed by splitk_reduce).  One thread per
+// output walked all K terms with 64-bit divisions: what bounded these small
+// products was that serial chain (chi = 16 site absorption, K = 16: 9.8 us;
+// K = 32 ... 64 steps of a 20-site compression: 15 us; full contractions with
+// M = N = 1 ran on one lane).
+struct DotArgs {
+  const void* A;
+  const void* B;
+  void* C;
+  void* part;
+  int no, nk;
+  FastDiv od[2 * TN_MAX_MODES], kd[TN_MAX_MODES];
+  int32_t oa[2 * TN_MAX_MODES], ob[2 * TN_MAX_MODES], oc[2 * TN_MAX_MODES];
+  int32_t ka[TN_MAX_MODES], kb[TN_MAX_MODES];
+  // index of an output in the dense M x N partial sums: per output mode
+  int32_t op[2 * TN_MAX_MODES];
+  uint32_t nout, K, kchunk;
+  double alpha, beta;
+};
+
+template <typename T, int G>
+__global__ void __launch_bounds__(256) contract_dot(DotArgs g) {
+  const T* __restrict__ A = (const T*)g.A;
+  const T* __restrict__ B = (const T*)g.B;
+  T* __restrict__ C = (T*)g.C;
+  constexpr int PB = 256 / G;  // outputs per block
+  const uint32_t l = threadIdx.x % G;
+  const uint32_t o = blockIdx.x * PB + threadIdx.x / G;
+  const bool live = o < g.nout;
+  uint32_t idx = live ? o : 0;
+  int32_t pa = 0, pb = 0, pc = 0, pp = 0;
+  for (int i = g.no - 1; i >= 0; --i) {
+    const uint32_t q = fast_div(idx, g.od[i]);
+    const int32_t r = (int32_t)(idx - q * g.od[i].d);
+    pa += r * g.oa[i];
+    pb += r * g.ob[i];
+    pc += r * g.oc[i];
+    pp += r * g.op[i];
+    idx = q;
+  }
+  const uint32_t k1 = min(g.K, (blockIdx.y + 1) * g.kchunk);
+  uint32_t k = blockIdx.y * g.kchunk + l;
+  T acc = 0;
+  if (g.nk == 1) {
+    const int32_t ka = g.ka[0], kb = g.kb[0];
+    // four terms' loads in flight at a time
+    for (; k + 3 * G < k1; k += 4 * G) {
+      T a[4], b[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[u] = A[pa + (int32_t)(k + u * G) * ka];
+        b[u] = B[pb + (int32_t)(k + u * G) * kb];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = fma(a[u], b[u], acc);
+    }
+    for (; k < k1; k += G) acc = fma(A[pa + (int32_t)k * ka], B[pb + (int32_t)k * kb], acc);
+  } else {
+    for (; k < k1; k += G) {
+      uint32_t kx = k;
+      int32_t qa = pa, qb = pb;
+      for (int i = g.nk - 1; i >= 0; --i) {
+        const uint32_t q = fast_div(kx, g.kd[i]);
+        const int32_t r = (int32_t)(kx - q * g.kd[i].d);
+        qa += r * g.ka[i];
+        qb += r * g.kb[i];
+        kx = q;
+      }
+      acc = fma(A[qa], B[qb], acc);
+    }
+  }
+#pragma unroll
+  for (int sh = 1; sh < (G < 64 ? G : 64); sh <<= 1) acc += __shfl_xor(acc, sh, 64);
+  if constexpr (G == 256) {
+    __shared__ T red[4];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    acc = (red[0] + red[1]) + (red[2] + red[3]);
+  }
+  if (l != 0 || !live) return;
+  if (g.part) {
+    ((T*)g.part)[(int64_t)blockIdx.y * g.nout + pp] = acc;
+  } else {
+    T v = (T)(g.alpha * (double)acc);
+    if (g.beta != 0.0) v += (T)g.beta * C[pc];
+    C[pc] = v;
+  }
+}
+
+template <typename T>
+static void launch_dot(int G, dim3 grid, hipStream_t st, const DotArgs& d) {
+  if (G == 4)
+    hipLaunchKernelGGL((contract_dot<T, 4>), grid, dim3(256), 0, st, d);
+  else if (G == 16)
+    hipLaunchKernelGGL((contract_dot<T, 16>), grid, dim3(256), 0, st, d);
+  else if (G == 64)
+    hipLaunchKernelGGL((contract_dot<T, 64>), grid, dim3(256), 0, st, d);
+  else
+    hipLaunchKernelGGL((contract_dot<T, 256>), grid, dim3(256), 0, st, d);
+}
+
 // Merge adjacent modes of a group when the merge is valid for every operand
 // that shares the group (strides of the slower mode = stride*dim of the faster).
 static void merge_group(std::vector<int64_t>& dims, std::vector<std::vector<int64_t>*> strides) {
@@ -728,10 +834,12 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
   if (K == 0 || small_k || tiny || (M < 16 && N < 16)) {
     // direct kernel: output modes sorted by C stride (descending) so that
     // consecutive threads store consecutive addresses.
-    struct OM { int64_t d, a, b, c; };
+    // p: the mode's stride in a dense row-major M x N array
+    struct OM { int64_t d, a, b, c, p; };
     std::vector<OM> om;
-    for (size_t i = 0; i < md.size(); ++i) om.push_back({md[i], mas[i], 0, mcs[i]});
-    for (size_t i = 0; i < nd.size(); ++i) om.push_back({nd[i], 0, nbs[i], ncs[i]});
+    int64_t pm = M * N, pn = N;
+    for (size_t i = 0; i < md.size(); ++i) { pm /= md[i]; om.push_back({md[i], mas[i], 0, mcs[i], pm}); }
+    for (size_t i = 0; i < nd.size(); ++i) { pn /= nd[i]; om.push_back({nd[i], 0, nbs[i], ncs[i], pn}); }
     std::stable_sort(om.begin(), om.end(), [](const OM& x, const OM& y) { return x.c > y.c; });
     std::vector<OM> om2;
     for (auto& x : om)
@@ -761,13 +869,60 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
       return m;
     };
     const int64_t lim = (int64_t)1 << 31;
-    bool fits = g.nout < lim && K >= 1 && K <= 8;
+    bool fits = g.nout < lim && K >= 1 && K < lim;
     for (int i = 0; i < g.no && fits; ++i)
       fits = g.oa[i] >= 0 && g.ob[i] >= 0 && g.oc[i] >= 0;
     for (int i = 0; i < g.nk && fits; ++i) fits = g.ka[i] >= 0 && g.kb[i] >= 0;
     fits = fits && span(g.odim, g.oa, g.no) + span(g.kdim, g.ka, g.nk) < lim &&
            span(g.odim, g.ob, g.no) + span(g.kdim, g.kb, g.nk) < lim &&
            span(g.odim, g.oc, g.no) < lim;
+    if (fits && K > 8) {
+      DotArgs h{};
+      h.A = A; h.B = B; h.C = C;
+      h.no = g.no;
+      h.nk = g.nk;
+      for (int i = 0; i < g.no; ++i) {
+        h.od[i] = make_fastdiv((uint32_t)g.odim[i]);
+        h.oa[i] = (int32_t)g.oa[i]; h.ob[i] = (int32_t)g.ob[i]; h.oc[i] = (int32_t)g.oc[i];
+        h.op[i] = (int32_t)om2[i].p;
+      }
+      for (int i = 0; i < g.nk; ++i) {
+        h.kd[i] = make_fastdiv((uint32_t)g.kdim[i]);
+        h.ka[i] = (int32_t)g.ka[i]; h.kb[i] = (int32_t)g.kb[i];
+      }
+      h.nout = (uint32_t)g.nout;
+      h.K = (uint32_t)K;
+      h.alpha = alpha;
+      h.beta = beta;
+      // four lanes from 9 terms on, 16 from 64, a wave from 256, the block
+      // from 4096: four to sixteen terms a lane where the outputs alone do
+      // not fill the chip
+      const int G = K < 64 ? 4 : (K < 256 ? 16 : (K < 4096 ? 64 : 256));
+      const int64_t ob = ceil_div(g.nout, 256 / G);
+      // ... and ranges of at least 4096 terms over more blocks
+      int64_t S = splitk_ws && K >= 8192
+                      ? std::min<int64_t>({K / 4096, ceil_div(512, ob), 64}) : 1;
+      while (S > 1 && (size_t)(S * g.nout) * (dtype == TN_F64 ? 8 : 4) > splitk_bytes) --S;
+      h.kchunk = (uint32_t)ceil_div(K, S);
+      S = ceil_div(K, (int64_t)h.kchunk);
+      h.part = S > 1 ? splitk_ws : nullptr;
+      const dim3 grid((unsigned)ob, (unsigned)S);
+      if (dtype == TN_F64) launch_dot<double>(G, grid, st, h);
+      else launch_dot<float>(G, grid, st, h);
+      TN_CHECK_LAUNCH();
+      if (S > 1) {
+        const Modes cm = make_modes(md, mcs), cn = make_modes(nd, ncs);
+        const unsigned rb = (unsigned)ceil_div(M * N, 256);
+        if (dtype == TN_F64)
+          hipLaunchKernelGGL(splitk_reduce<double>, dim3(rb), dim3(256), 0, st,
+                             (const double*)splitk_ws, (int)S, M, N, cm, cn, (double*)C, alpha, beta);
+        else
+          hipLaunchKernelGGL(splitk_reduce<float>, dim3(rb), dim3(256), 0, st,
+                             (const float*)splitk_ws, (int)S, M, N, cm, cn, (float*)C, alpha, beta);
+        TN_CHECK_LAUNCH();
+      }
+      return TN_OK;
+    }
     if (fits) {
       Direct32Args h{};
       h.A = A; h.B = B; h.C = C;
