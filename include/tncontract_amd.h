@@ -136,6 +136,15 @@ int tn_contract_ws(const void* A, const tn_modes* a_m, const tn_modes* a_k,
                    int dtype, int precision, double alpha, double beta,
                    void* ws, size_t ws_bytes, void* stream);
 
+/* tn_contract_ws with the axes in one flat list, as a host with strided
+ * tensors has them: axes = {nm, nk, nn} followed by (extent, A stride, C
+ * stride) of the nm free axes of A, (extent, A stride, B stride) of the nk
+ * contracted axes and (extent, B stride, C stride) of the nn free axes of B,
+ * each group slowest first, at most TN_MAX_MODES axes each. */
+int tn_contract_axes(const void* A, const void* B, void* C, const int64_t* axes, int dtype,
+                     int precision, double alpha, double beta, void* ws, size_t ws_bytes,
+                     void* stream);
+
 /* ---- QR (np.linalg.qr(mode="reduced") in tensor_qr, tensor.py:1044) ------
  * A is the m x n matrix whose row index is decoded through a_rows and column
  * index through a_cols.  Q: m x k row-major, R: k x n row-major, k=min(m,n).

@@ -72,3 +72,16 @@ def test_merged_modes_reproduce_view_offsets():
         offs = [off0 + sum(i * s for i, s in zip(idx, st))
                 for idx in itertools.product(*[range(d) for d in dims])]
         assert offs == list(view.reshape(-1))
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="library not built")
+def test_contract_axes_rejects_bad_groups_on_the_host():
+    import torch  # noqa: F401
+    from tncontract_amd import _lib as L
+    lib = L.lib()
+    ok = [1, 1, 1] + [2, 1, 1] * 3
+    for bad in ([9, 1, 1] + [2, 1, 1] * 11, [1, -1, 1] + [2, 1, 1] * 3,
+                [1, 1, 1, -2, 1, 1] + [2, 1, 1] * 2, ok):  # ok: null operands
+        axes = (ctypes.c_int64 * len(bad))(*bad)
+        rc = lib.tn_contract_axes(None, None, None, axes, L.TN_F64, 0, 1.0, 0.0, None, 0, None)
+        assert rc == L.TN_ERR_INVALID and lib.tn_last_error()

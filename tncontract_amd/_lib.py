@@ -85,6 +85,7 @@ def lib():
         "tn_normalize": (i32, [vp, i32, i64, vp, vp, sz, vp]),
         "tn_contract": (i32, [vp, mp, mp, vp, mp, mp, vp, mp, mp, i32, i32, dbl, dbl, vp]),
         "tn_contract_workspace": (sz, [i64, i64, i64, i32]),
+        "tn_contract_axes": (i32, [vp, vp, vp, ctypes.POINTER(i64), i32, i32, dbl, dbl, vp, sz, vp]),
         "tn_contract_ws": (i32, [vp, mp, mp, vp, mp, mp, vp, mp, mp, i32, i32, dbl, dbl, vp, sz, vp]),
         "tn_qr_workspace": (sz, [i64, i64, i32]),
         "tn_qr": (i32, [vp, mp, mp, i64, i64, vp, vp, i32, vp, sz, vp]),
@@ -159,7 +160,8 @@ def device():
 
 
 def stream_ptr():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device, as the address the C ABI takes."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def ptr(t):
@@ -178,26 +180,43 @@ def workspace(nbytes):
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device())
 
 
-_SPLITK_WS = {}
+# ctypes array types of the axis lists contract_axes passes (3 counts and at
+# most 8 + 8 + 8 axes of three numbers)
+_AXES = [ctypes.c_int64 * n for n in range(3 + 9 * TN_MAX_MODES + 1)]
 
 
-def contract(A, am, ak, B, bk, bn, C, cm, cn, dtype_code, prec, M, N, K, alpha=1.0, beta=0.0):
-    """tn_contract through the split-K variant: the partial-sum workspace is
-    one buffer per device, grown on demand and reused by every call (all
-    calls are ordered on the current stream)."""
-    need = lib().tn_contract_workspace(int(M), int(N), int(K), dtype_code)
+def contract_axes(d1, free1, ax1, d2, ax2, free2, out, ostrides, prec, M, N, K):
+    """out[free1, free2] = sum over ax1 / ax2 of d1 * d2, out's element strides
+    `ostrides` per axis of free1 then free2, as one tn_contract_axes call (the
+    axes' extents and strides in one flat list: building the six mode groups
+    as ctypes structures cost more than the launch).  The partial sums of a
+    split contraction go to a buffer of this call's own, so calls on other
+    streams and threads do not meet in it."""
+    if len(free1) > TN_MAX_MODES or len(free2) > TN_MAX_MODES or len(ax1) > TN_MAX_MODES:
+        raise NotImplementedError("more than %d modes in one group" % TN_MAX_MODES)
+    sh1, st1, sh2, st2 = d1.shape, d1.stride(), d2.shape, d2.stride()
+    v = [len(free1), len(ax1), len(free2)]
+    i = 0
+    for a in free1:
+        v += (sh1[a], st1[a], ostrides[i])
+        i += 1
+    for a, b in zip(ax1, ax2):
+        v += (sh1[a], st1[a], st2[b])
+    for b in free2:
+        v += (sh2[b], st2[b], ostrides[i])
+        i += 1
+    L = lib()
+    code = dtype_code(d1)
     ws, nb = None, 0
-    if need:
-        dev = torch.cuda.current_device()
-        ws = _SPLITK_WS.get(dev)
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(max(int(need), 1 << 24), dtype=torch.uint8, device=device())
-            _SPLITK_WS[dev] = ws
-        nb = ws.numel()
-    check(lib().tn_contract_ws(ptr(A), ctypes.byref(am), ctypes.byref(ak), ptr(B), ctypes.byref(bk),
-                               ctypes.byref(bn), ptr(C), ctypes.byref(cm), ctypes.byref(cn),
-                               dtype_code, prec, alpha, beta, ptr(ws) if ws is not None else None,
-                               nb, stream_ptr()))
+    if K >= 128:
+        nb = L.tn_contract_workspace(M, N, K, code)
+        if nb:
+            buf = torch.empty(nb, dtype=torch.uint8, device=d1.device)
+            ws = buf.data_ptr()
+    rc = L.tn_contract_axes(d1.data_ptr(), d2.data_ptr(), out.data_ptr(), _AXES[len(v)](*v), code,
+                            prec, 1.0, 0.0, ws, nb, stream_ptr())
+    if rc:
+        check(rc)
 
 
 def empty(shape, dtype=torch.float64):

@@ -1131,3 +1131,32 @@ extern "C" int tn_contract_ws(const void* A, const tn_modes* a_m, const tn_modes
   return contract_launch(A, am, ak, B, bk, bn, C, cm, cn, dtype, precision, alpha, beta,
                          ws_bytes ? ws : nullptr, ws ? ws_bytes : 0, as_stream(stream));
 }
+
+extern "C" int tn_contract_axes(const void* A, const void* B, void* C, const int64_t* axes,
+                                int dtype, int precision, double alpha, double beta, void* ws,
+                                size_t ws_bytes, void* stream) {
+  TN_REQUIRE(axes != nullptr, "tn_contract_axes: null pointer");
+  for (int i = 0; i < 3; ++i)
+    TN_REQUIRE(axes[i] >= 0 && axes[i] <= TN_MAX_MODES,
+               "tn_contract_axes: mode group has too many modes");
+  const int64_t* p = axes + 3;
+  // extents and the two strides of a group
+  auto group = [&](int64_t n, Modes& x, Modes& y) -> bool {
+    x = Modes{};
+    x.n = (int32_t)n;
+    for (int i = 0; i < TN_MAX_MODES; ++i) x.dims[i] = 1;
+    y = x;
+    for (int i = 0; i < x.n; ++i, p += 3) {
+      if (p[0] < 0) return false;
+      x.dims[i] = y.dims[i] = p[0];
+      x.strides[i] = p[1];
+      y.strides[i] = p[2];
+    }
+    return true;
+  };
+  Modes am, cm, ak, bk, bn, cn;
+  TN_REQUIRE(group(axes[0], am, cm) && group(axes[1], ak, bk) && group(axes[2], bn, cn),
+             "tn_contract_axes: negative dimension");
+  return contract_launch(A, am, ak, B, bk, bn, C, cm, cn, dtype, precision, alpha, beta,
+                         ws_bytes ? ws : nullptr, ws ? ws_bytes : 0, as_stream(stream));
+}

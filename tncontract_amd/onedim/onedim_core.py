@@ -11,6 +11,7 @@ reference itself reads.
 from __future__ import annotations
 
 import warnings
+from math import prod
 
 import numpy as np
 import torch
@@ -955,14 +956,17 @@ def contract_mps_mpo(mps, mpo):
 def _contract_consolidated(t1, t2, l1, l2):
     """contract(t1, t2, l1, l2) followed by consolidate_indices(), computed as
     one kernel whose store offsets encode the consolidated layout."""
-    import ctypes
-    import torch
-    ax1 = [i for i, x in enumerate(t1.labels) if x == l1]
-    ax2 = [i for i, x in enumerate(t2.labels) if x == l2]
-    free1 = [i for i in range(t1.rank) if i not in ax1]
-    free2 = [i for i in range(t2.rank) if i not in ax2]
-    labels = [t1.labels[i] for i in free1] + [t2.labels[i] for i in free2]
-    dims = [t1.shape[i] for i in free1] + [t2.shape[i] for i in free2]
+    names1, names2 = t1.labels, t2.labels
+    ax1 = [i for i, x in enumerate(names1) if x == l1]
+    ax2 = [i for i, x in enumerate(names2) if x == l2]
+    d1, d2 = tsr._common_dtype(t1.data, t2.data)
+    sh1, sh2 = d1.shape, d2.shape
+    if len(ax1) != len(ax2) or any(sh1[a] != sh2[b] for a, b in zip(ax1, ax2)):
+        raise ValueError("contract_mps_mpo: physical dimensions do not match")
+    free1 = [i for i in range(len(names1)) if i not in ax1]
+    free2 = [i for i in range(len(names2)) if i not in ax2]
+    labels = [names1[i] for i in free1] + [names2[i] for i in free2]
+    dims = [sh1[i] for i in free1] + [sh2[i] for i in free2]
     # consolidated layout: simulate consolidate_indices on (labels, axis ids)
     groups = [[i] for i in range(len(labels))]
     labs = list(labels)
@@ -972,29 +976,19 @@ def _contract_consolidated(t1, t2, l1, l2):
         fused = [a for i in idx for a in groups[i]]
         groups = [groups[i] for i in rest[:p]] + [fused] + [groups[i] for i in rest[p:]]
         labs = [labs[i] for i in rest[:p]] + [lab] + [labs[i] for i in rest[p:]]
-    order = [a for g in groups for a in g]
     # stride of each uncontracted axis in the final dense layout
     stride = [0] * len(dims)
     acc = 1
-    for a in reversed(order):
-        stride[a] = acc
-        acc *= dims[a]
-    d1, d2 = tsr._common_dtype(t1.data, t2.data)
-    out = torch.empty(acc, dtype=d1.dtype, device=d1.device)
-    nf1 = len(free1)
-    am = L.tensor_modes(d1, free1)
-    ak = L.tensor_modes(d1, ax1)
-    bk = L.tensor_modes(d2, ax2)
-    bn = L.tensor_modes(d2, free2)
-    cm = L.modes(dims[:nf1], stride[:nf1])
-    cn = L.modes(dims[nf1:], stride[nf1:])
-    if len(ax1) != len(ax2) or any(t1.shape[a] != t2.shape[b] for a, b in zip(ax1, ax2)):
-        raise ValueError("contract_mps_mpo: physical dimensions do not match")
-    L.contract(d1, am, ak, d2, bk, bn, out, cm, cn, L.dtype_code(d1), 0,
-               int(np.prod([d1.shape[a] for a in free1])), int(np.prod([d2.shape[a] for a in free2])),
-               int(np.prod([d1.shape[a] for a in ax1])))
-    shape = [int(np.prod([dims[a] for a in g])) for g in groups]
-    return tsr.Tensor._wrap(out.view(shape), labs)
+    for g in reversed(groups):
+        for a in reversed(g):
+            stride[a] = acc
+            acc *= dims[a]
+    out = torch.empty([prod([dims[a] for a in g]) for g in groups], dtype=d1.dtype, device=d1.device)
+    if acc:
+        nf1 = len(free1)
+        L.contract_axes(d1, free1, ax1, d2, ax2, free2, out, stride, 0, prod(dims[:nf1]),
+                        prod(dims[nf1:]), prod([sh1[a] for a in ax1]))
+    return tsr.Tensor._wrap(out, labs)
 
 
 def _from_owned(cls, tensors, left_label, right_label, phys_label):

@@ -17,6 +17,7 @@ from __future__ import annotations
 import copy as _copy
 import ctypes
 import warnings
+from math import prod
 
 import numpy as np
 import torch
@@ -248,7 +249,7 @@ class Tensor:
             groups = [groups[i] for i in rest[:p]] + [fused] + [groups[i] for i in rest[p:]]
             labs = [labs[i] for i in rest[:p]] + [lab] + [labs[i] for i in rest[p:]]
         perm = [a for g in groups for a in g]
-        shape = [int(np.prod([self._data.shape[a] for a in g])) for g in groups]
+        shape = [prod([self._data.shape[a] for a in g]) for g in groups]
         self._data = _reshape(self._data.permute(perm), shape)
         self.labels = labs
 
@@ -420,23 +421,24 @@ def _contract_data(d1, ax1, d2, ax2, precision="native"):
     the free axes of d1 then those of d2 (each in order)."""
     if len(ax1) != len(ax2):
         raise ValueError("Number of indices in contraction does not match.")
+    sh1, sh2 = d1.shape, d2.shape
     for a, b in zip(ax1, ax2):
-        if d1.shape[a] != d2.shape[b]:
+        if sh1[a] != sh2[b]:
             raise ValueError("shape-mismatch for sum")
     d1, d2 = _common_dtype(d1, d2)
-    free1 = [i for i in range(d1.dim()) if i not in ax1]
-    free2 = [i for i in range(d2.dim()) if i not in ax2]
-    out_shape = [d1.shape[i] for i in free1] + [d2.shape[i] for i in free2]
+    free1 = [i for i in range(len(sh1)) if i not in ax1]
+    free2 = [i for i in range(len(sh2)) if i not in ax2]
+    out_shape = [sh1[i] for i in free1] + [sh2[i] for i in free2]
     dtype = d1.dtype
     prec = L.PREC[precision]
     if prec != 0 and dtype == torch.float64:
         d1, d2, dtype = L.convert(d1, torch.float32), L.convert(d2, torch.float32), torch.float32
-    out = torch.empty(tuple(out_shape), dtype=dtype, device=d1.device)
-    if out.numel() == 0:
+    out = torch.empty(out_shape, dtype=dtype, device=d1.device)
+    nf1 = len(free1)
+    M, N = prod(out_shape[:nf1]), prod(out_shape[nf1:])
+    if M * N == 0:
         return out
-    M = int(np.prod(out_shape[:len(free1)])) if free1 else 1
-    N = int(np.prod(out_shape[len(free1):])) if free2 else 1
-    K = int(np.prod([d1.shape[a] for a in ax1])) if ax1 else 1
+    K = prod([sh1[a] for a in ax1])
     # An operand whose free or contracted axes do not fuse into one stride
     # makes the MFMA contraction decode its tile offsets through per-mode
     # tables (15-30 % slower on the sweep's products).  For a GEMM-sized
@@ -453,19 +455,7 @@ def _contract_data(d1, ax1, d2, ax2, precision="native"):
                 and flops >= 512.0 * d2.numel()):
             d2 = L.contiguous(d2.permute(*(ax2 + free2)))
             ax2, free2 = list(range(len(ax2))), list(range(len(ax2), d2.dim()))
-    # dense output strides
-    strides, acc = [0] * len(out_shape), 1
-    for i in range(len(out_shape) - 1, -1, -1):
-        strides[i] = acc
-        acc *= out_shape[i]
-    nf1 = len(free1)
-    am = L.tensor_modes(d1, free1)
-    ak = L.tensor_modes(d1, ax1)
-    bk = L.tensor_modes(d2, ax2)
-    bn = L.tensor_modes(d2, free2)
-    cm = L.modes(out_shape[:nf1], strides[:nf1])
-    cn = L.modes(out_shape[nf1:], strides[nf1:])
-    L.contract(d1, am, ak, d2, bk, bn, out, cm, cn, L.dtype_code(d1), prec, M, N, K)
+    L.contract_axes(d1, free1, ax1, d2, ax2, free2, out, out.stride(), prec, M, N, K)
     return out
 
 
@@ -494,12 +484,9 @@ def contract(tensor1, tensor2, labels1, labels2, index_slice1=None, index_slice2
         labels1 = [labels1]
     if not isinstance(labels2, list):
         labels2 = [labels2]
-    ax1 = []
-    for label in labels1:
-        ax1.extend(i for i, x in enumerate(tensor1.labels) if x == label)
-    ax2 = []
-    for label in labels2:
-        ax2.extend(i for i, x in enumerate(tensor2.labels) if x == label)
+    names1, names2 = tensor1.labels, tensor2.labels
+    ax1 = [i for label in labels1 for i, x in enumerate(names1) if x == label]
+    ax2 = [i for label in labels2 for i, x in enumerate(names2) if x == label]
     if index_slice1 is not None:
         sl = [x if x != -1 else len(ax1) - 1 for x in index_slice1]
         ax1 = [j for i, j in enumerate(ax1) if i in sl]
@@ -508,16 +495,16 @@ def contract(tensor1, tensor2, labels1, labels2, index_slice1=None, index_slice2
         ax2 = [j for i, j in enumerate(ax2) if i in sl]
     if len(ax1) != len(ax2):
         raise ValueError("Number of indices in contraction does not match.")
-    for i in range(len(ax1)):
-        d1 = tensor1.shape[ax1[i]]
-        d2 = tensor2.shape[ax2[i]]
-        if d1 != d2:
-            raise ValueError(str(labels1[min(i, len(labels1) - 1)]) + " with dim=" + str(d1)
+    data1, data2 = tensor1.data, tensor2.data
+    sh1, sh2 = data1.shape, data2.shape
+    for i, (a, b) in enumerate(zip(ax1, ax2)):
+        if sh1[a] != sh2[b]:
+            raise ValueError(str(labels1[min(i, len(labels1) - 1)]) + " with dim=" + str(sh1[a])
                              + " does not match " + str(labels2[min(i, len(labels2) - 1)])
-                             + " with dim=" + str(d2))
-    out = _contract_data(tensor1.data, ax1, tensor2.data, ax2, precision)
-    labels = ([x for j, x in enumerate(tensor1.labels) if j not in ax1]
-              + [x for j, x in enumerate(tensor2.labels) if j not in ax2])
+                             + " with dim=" + str(sh2[b]))
+    out = _contract_data(data1, ax1, data2, ax2, precision)
+    labels = ([x for j, x in enumerate(names1) if j not in ax1]
+              + [x for j, x in enumerate(names2) if j not in ax2])
     return Tensor._wrap(out, labels)
 
 
@@ -581,8 +568,8 @@ def _row_view(tensor, row_labels, move_all):
 def _matrix_modes(d, nrow):
     rows = L.tensor_modes(d, range(nrow))
     cols = L.tensor_modes(d, range(nrow, d.dim()))
-    m = int(np.prod(d.shape[:nrow])) if nrow else 1
-    n = int(np.prod(d.shape[nrow:])) if d.dim() > nrow else 1
+    m = prod(d.shape[:nrow])
+    n = prod(d.shape[nrow:])
     return rows, cols, m, n
 
 
