@@ -244,3 +244,62 @@ def test_contract_many_lanes_per_output(L, shape_a, ax_a, shape_b, ax_b, dtype):
     # (plus the oracle's own FP64 rounding)
     bound = (K + 4) * (np.finfo(dtype).eps / 2 + 2.0 ** -53) * mag
     assert c.shape == ref.shape and np.all(np.abs(c - ref) <= bound)
+
+
+# QR blocks through their orthonormal factor (64 columns, at least 256 rows
+# below the diagonal), beside the panels: ragged edges of both, columns of very
+# different lengths, and the inputs that have to stay with the panels -- zero
+# and unit columns, triangular and rank-deficient matrices, zero pivots, NaN.
+# LAPACK's R is reached to rounding, its diagonal's signs with it.
+@pytest.mark.parametrize("m,n", [(256, 64), (257, 65), (319, 64), (320, 128), (700, 129),
+                                 (1285, 643), (500, 1500)])
+@pytest.mark.parametrize("scale", ["flat", "graded"])
+def test_qr_blocks_match_lapack(L, m, n, scale):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(m + n)
+    a = rng.standard_normal((m, n))
+    if scale == "graded":
+        a *= 2.0 ** rng.integers(-300, 300, size=n)
+    q, r = (x.cpu().numpy() for x in T._qr_device(dev(a), 1))
+    k = min(m, n)
+    ref = np.linalg.qr(a)[1]
+    norms = np.linalg.norm(a, axis=0)
+    assert np.abs(q.T @ q - np.eye(k)).max() <= 1e-13
+    assert (np.linalg.norm(q @ r - a, axis=0) <= 1e-13 * norms).all()
+    assert (np.abs(r - ref).max(axis=0) <= 1e-11 * norms).all()
+    assert not np.tril(r, -1).any()
+
+
+@pytest.mark.parametrize("case", ["eye", "triu", "zero", "zero_column", "rank", "zero_pivot", "nan"])
+def test_qr_blocks_leave_special_inputs_to_the_panels(L, case):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(3)
+    m, n = 700, 200
+    a = rng.standard_normal((m, n))
+    if case == "eye":
+        a = np.eye(m, n)
+    elif case == "triu":
+        a = np.triu(a)
+    elif case == "zero":
+        a[:] = 0.0
+    elif case == "zero_column":
+        a[:, 70] = 0.0
+    elif case == "rank":
+        a = a[:, :40] @ rng.standard_normal((40, n))
+    elif case == "zero_pivot":
+        a[:64, :64] = 0.0
+    elif case == "nan":
+        a[300, 100] = np.nan
+    q, r = (x.cpu().numpy() for x in T._qr_device(dev(a), 1))
+    if case == "nan":
+        assert np.isnan(q).any() and np.isnan(r).any()
+        return
+    assert np.abs(q.T @ q - np.eye(n)).max() <= 1e-13
+    assert np.abs(q @ r - a).max() <= 1e-12 * max(1.0, np.abs(a).max()) * np.sqrt(n)
+    if case in ("eye", "triu", "zero"):
+        # no reflection at all: R is the matrix, with its own signs
+        np.testing.assert_array_equal(r, a[:n])
+    elif case in ("zero_pivot", "zero_column"):
+        ref = np.linalg.qr(a)[1]
+        keep = 70 if case == "zero_column" else n  # (past it the signs are rounding's)
+        assert np.abs(r[:keep] - ref[:keep]).max() <= 1e-11 * np.abs(ref).max()

@@ -93,7 +93,9 @@ __global__ void __launch_bounds__(512) cq_diag(const double* __restrict__ S, int
                                                int64_t j0, int w,
                                                const double* __restrict__ pivmin,
                                                double* __restrict__ F, double* __restrict__ X,
-                                               int* __restrict__ fail) {
+                                               int* __restrict__ fail,
+                                               const int* __restrict__ skip) {
+  if (skip && *skip) return;
   // panel columns of L (Ls[b][kc][t] = L[t][QC b + kc], zero above the
   // diagonal) and 1 / L[c][c] (0 for a dropped column); XP: per wave, the
   // panel's rows of X at its columns
@@ -285,7 +287,7 @@ int cq_pass(double* S, double* F, int64_t m, int64_t n, double thr, const CqWs& 
   for (int64_t j0 = 0; j0 < n; j0 += QB) {
     const int w = (int)std::min<int64_t>(QB, n - j0);
     hipLaunchKernelGGL(cq_diag<false>, dim3(1), dim3(512), 0, st, S, ld, j0, w, ws.pivmin, F, ws.X,
-                       ws.fail);
+                       ws.fail, (const int*)nullptr);
     TN_CHECK_LAUNCH();
     // [L21; Q_j] = [G21; W_j] L11^{-T}:  B[k][c] = X[c][k] = X[k * QB + c]
     const int64_t rows = ld - j0 - w;
@@ -306,9 +308,9 @@ int cq_pass(double* S, double* F, int64_t m, int64_t n, double thr, const CqWs& 
 }  // namespace
 
 int chol_block(const double* S, int64_t ld, int64_t j0, int w, const double* delta, double* F,
-               double* X, hipStream_t st) {
+               double* X, hipStream_t st, const int* skip) {
   hipLaunchKernelGGL(cq_diag<true>, dim3(1), dim3(512), 0, st, S, ld, j0, w, delta, F, X,
-                     (int*)nullptr);
+                     (int*)nullptr, skip);
   TN_CHECK_LAUNCH();
   return TN_OK;
 }

@@ -20,6 +20,7 @@ Modes mk(std::initializer_list<int64_t> dims, std::initializer_list<int64_t> str
 // Householder QR internals (tn_qr.hip), reused by the QR-preconditioned SVD.
 struct QrWs {
   double *W, *tau, *V, *Tall, *G, *Y, *Y2, *Tp, *Qw, *part, *Ypart;
+  int* bad;  // device flag of tn_qr_hr.h
   size_t part_bytes;
 };
 // Carve the QR workspace for an m x n factorisation (base == nullptr: size query).
@@ -38,9 +39,10 @@ int qr_form_q(const double* W, int64_t m, int64_t n, const QrWs& ws, double* Qw,
 // Shifted Cholesky of the w x w diagonal block at (j0, j0) of the
 // column-major S (ld): L11 into F at the same position, L11^{-1} into X
 // (64 x 64, column-major); a pivot below delta/2 (delta on the device)
-// drops its column (zero L column, zero X row).  w <= 64.
+// drops its column (zero L column, zero X row).  w <= 64.  skip (on the
+// device, may be null): do nothing while *skip is not 0.
 int chol_block(const double* S, int64_t ld, int64_t j0, int w, const double* delta, double* F,
-               double* X, hipStream_t st);
+               double* X, hipStream_t st, const int* skip = nullptr);
 size_t cholqr_ws_bytes(int64_t m, int64_t n);
 int cholqr_run(const void* A, const Modes& rows, const Modes& cols, int64_t m, int64_t n,
                double* Q, int64_t q_rs, int64_t q_cs, double* R, double orth_tol,

@@ -13,6 +13,7 @@
 // Q is formed explicitly (orgqr order: blocks applied last to first to
 // [I; 0]).  Sign convention as LAPACK dlarfg: beta = -sign(alpha)*norm.
 #include "tn_internal.h"
+#include "tn_qr_hr.h"
 
 #include <vector>
 
@@ -70,7 +71,9 @@ template <int R, int W>
 __global__ void __launch_bounds__(PT) qr_panel_kernel(double* __restrict__ A, int64_t m,
                                                       int64_t ld, int64_t c0, int w,
                                                       double* __restrict__ tau,
-                                                      double* __restrict__ Tp) {
+                                                      double* __restrict__ Tp,
+                                                      const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   __shared__ double lds[2][NWAVE * W];
   int par = 0;
   __shared__ double piv[W];       // pivot value of each column (one slot each)
@@ -235,7 +238,9 @@ __device__ __forceinline__ double vref(const double* A, int64_t ld, int64_t c0, 
 template <int W>
 __global__ void __launch_bounds__(256) qr_panel_dots(const double* __restrict__ A, int64_t m,
                                                      int64_t ld, int64_t c0, int w, int64_t cb,
-                                                     int64_t ncol, double* __restrict__ Ypart) {
+                                                     int64_t ncol, double* __restrict__ Ypart,
+                                                     const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   __shared__ double Vs[QCH][W];
   __shared__ double red[4][W][QCOL];
   const int64_t r0 = c0 + (int64_t)blockIdx.y * QCH;
@@ -297,7 +302,9 @@ __global__ void __launch_bounds__(256) qr_panel_update(double* __restrict__ A, i
                                                        int64_t ld, int64_t c0, int w, int64_t cb,
                                                        int64_t ncol, int nchunk,
                                                        const double* __restrict__ Ypart,
-                                                       const double* __restrict__ Tp) {
+                                                       const double* __restrict__ Tp,
+                                                       const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   __shared__ double ys[W][QCOL];
   __shared__ double z[W][QCOL];
   const int64_t r0 = c0 + (int64_t)blockIdx.y * QCH;
@@ -354,7 +361,9 @@ __global__ void __launch_bounds__(256) qr_panel_update(double* __restrict__ A, i
 
 // Explicit V (mr x nb, column-major, ld = mr) of the outer block at j0.
 __global__ void qr_build_v_kernel(const double* __restrict__ A, int64_t m, int64_t ld,
-                                  int64_t j0, int nb, double* __restrict__ V) {
+                                  int64_t j0, int nb, double* __restrict__ V,
+                                  const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   const int64_t mr = m - j0;
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= mr * nb) return;
@@ -374,7 +383,9 @@ __global__ void qr_build_v_kernel(const double* __restrict__ A, int64_t m, int64
 // G = 0, so their rows and columns of T are zero.
 __global__ void __launch_bounds__(256) qr_larft_kernel(const double* __restrict__ G, int nb,
                                                        const double* __restrict__ tau,
-                                                       double* __restrict__ T) {
+                                                       double* __restrict__ T,
+                                                       const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   __shared__ double Gs[QR_NB][QR_NB + 1];
   __shared__ double Ts[QR_NB][QR_NB + 1];
   __shared__ double Ms[QR_NB][QR_NB + 1];
@@ -508,6 +519,7 @@ size_t qr_layout(int64_t m, int64_t n, char* base, size_t cap, QrWs* ws) {
   w.Y2 = a.take<double>((size_t)(QR_NB * wn));
   w.Tp = a.take<double>(64);
   w.Ypart = a.take<double>((size_t)ceil_div(m, QCH) * 8 * QR_NB);
+  w.bad = a.take<int>(1);
   w.Qw = a.take<double>((size_t)(m * k));
   w.part_bytes = (size_t)16 * QR_NB * wn * sizeof(double);
   w.part = a.take<double>((size_t)16 * QR_NB * wn);
@@ -532,7 +544,9 @@ __device__ __forceinline__ double block_sum256(double s, double* red) {
 
 __global__ void __launch_bounds__(256) qr_tall_sumsq(const double* __restrict__ A, int64_t m,
                                                       int64_t ld, int64_t c0,
-                                                      double* __restrict__ part) {
+                                                      double* __restrict__ part,
+                                                      const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   __shared__ double red[4];
   const int64_t r0 = c0 + 1 + (int64_t)blockIdx.x * QTALL;
   const int64_t r1 = r0 + QTALL < m ? r0 + QTALL : m;
@@ -546,7 +560,9 @@ __global__ void __launch_bounds__(256) qr_tall_sumsq(const double* __restrict__ 
 __global__ void __launch_bounds__(256) qr_tall_reflector(double* __restrict__ A, int64_t ld,
                                                           int64_t c0, double* __restrict__ part,
                                                           int nchunk, double* __restrict__ tau,
-                                                          double* __restrict__ Tp) {
+                                                          double* __restrict__ Tp,
+                                                          const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   __shared__ double red[4];
   double s = 0.0;
   for (int i = threadIdx.x; i < nchunk; i += 256) s += part[i];
@@ -570,7 +586,8 @@ __global__ void __launch_bounds__(256) qr_tall_reflector(double* __restrict__ A,
 
 __global__ void __launch_bounds__(256) qr_tall_scale(double* __restrict__ A, int64_t m, int64_t ld,
                                                       int64_t c0, const double* __restrict__ part,
-                                                      int nchunk) {
+                                                      int nchunk, const int* __restrict__ guard) {
+  if (guard && *guard == 0) return;
   const double scale = part[nchunk];
   const int64_t r0 = c0 + 1 + (int64_t)blockIdx.x * QTALL;
   const int64_t r1 = r0 + QTALL < m ? r0 + QTALL : m;
@@ -579,33 +596,29 @@ __global__ void __launch_bounds__(256) qr_tall_scale(double* __restrict__ A, int
 }
 
 static int run_tall_column(double* A, int64_t m, int64_t ld, int64_t c0, double* tau, double* Tp,
-                           double* part, hipStream_t st) {
+                           double* part, const int* guard, hipStream_t st) {
   const int nchunk = (int)ceil_div(std::max<int64_t>(m - c0 - 1, 0), QTALL);
   if (nchunk > 0) {
-    hipLaunchKernelGGL(qr_tall_sumsq, dim3((unsigned)nchunk), dim3(256), 0, st, A, m, ld, c0, part);
+    hipLaunchKernelGGL(qr_tall_sumsq, dim3((unsigned)nchunk), dim3(256), 0, st, A, m, ld, c0, part,
+                       guard);
     TN_CHECK_LAUNCH();
   }
-  hipLaunchKernelGGL(qr_tall_reflector, dim3(1), dim3(256), 0, st, A, ld, c0, part, nchunk, tau, Tp);
+  hipLaunchKernelGGL(qr_tall_reflector, dim3(1), dim3(256), 0, st, A, ld, c0, part, nchunk, tau, Tp,
+                     guard);
   TN_CHECK_LAUNCH();
   if (nchunk > 0) {
     hipLaunchKernelGGL(qr_tall_scale, dim3((unsigned)nchunk), dim3(256), 0, st, A, m, ld, c0, part,
-                       nchunk);
+                       nchunk, guard);
     TN_CHECK_LAUNCH();
   }
   return TN_OK;
 }
 
-typedef void (*PanelFn)(double*, int64_t, int64_t, int64_t, int, double*, double*);
-
-struct PanelChoice {
-  int R, W;
-  const void* fn;
-};
-
 template <int R, int W>
 static int launch_panel(double* A, int64_t m, int64_t ld, int64_t c0, int w, double* tau,
-                        double* Tp, hipStream_t st) {
-  hipLaunchKernelGGL((qr_panel_kernel<R, W>), dim3(1), dim3(PT), 0, st, A, m, ld, c0, w, tau, Tp);
+                        double* Tp, const int* guard, hipStream_t st) {
+  hipLaunchKernelGGL((qr_panel_kernel<R, W>), dim3(1), dim3(PT), 0, st, A, m, ld, c0, w, tau, Tp,
+                     guard);
   TN_CHECK_LAUNCH();
   return TN_OK;
 }
@@ -620,40 +633,92 @@ static int panel_width(int64_t mrem) {
 }
 
 static int run_panel(double* A, int64_t m, int64_t ld, int64_t c0, int w, double* tau, double* Tp,
-                     double* part, hipStream_t st) {
+                     double* part, const int* guard, hipStream_t st) {
   int64_t R = ceil_div(m - c0, PT);
-  if (R <= 1) return launch_panel<1, 8>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 2) return launch_panel<2, 8>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 4) return launch_panel<4, 8>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 6) return launch_panel<6, 8>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 8) return launch_panel<8, 8>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 10) return launch_panel<10, 8>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 14) return launch_panel<14, 4>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 24) return launch_panel<24, 2>(A, m, ld, c0, w, tau, Tp, st);
-  if (R <= 48) return launch_panel<48, 1>(A, m, ld, c0, w, tau, Tp, st);
+  if (R <= 1) return launch_panel<1, 8>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 2) return launch_panel<2, 8>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 4) return launch_panel<4, 8>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 6) return launch_panel<6, 8>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 8) return launch_panel<8, 8>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 10) return launch_panel<10, 8>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 14) return launch_panel<14, 4>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 24) return launch_panel<24, 2>(A, m, ld, c0, w, tau, Tp, guard, st);
+  if (R <= 48) return launch_panel<48, 1>(A, m, ld, c0, w, tau, Tp, guard, st);
   TN_REQUIRE(w == 1, "tn_qr: tall panel of width %d", w);
-  return run_tall_column(A, m, ld, c0, tau, Tp, part, st);
+  return run_tall_column(A, m, ld, c0, tau, Tp, part, guard, st);
 }
 
 static int run_apply_panel(double* A, int64_t m, int64_t ld, int64_t c0, int w, const double* Tp,
-                           int64_t cb, int64_t ce, double* Ypart, hipStream_t st) {
+                           int64_t cb, int64_t ce, double* Ypart, const int* guard,
+                           hipStream_t st) {
   if (ce <= cb) return TN_OK;
   const int64_t ncol = ce - cb;
   const int nchunk = (int)ceil_div(m - c0, QCH);
   dim3 grid((unsigned)ceil_div(ncol, QCOL), (unsigned)nchunk);
   if (w > 4) {
-    hipLaunchKernelGGL(qr_panel_dots<8>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol, Ypart);
+    hipLaunchKernelGGL(qr_panel_dots<8>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol, Ypart,
+                       guard);
     hipLaunchKernelGGL(qr_panel_update<8>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol,
-                       nchunk, Ypart, Tp);
+                       nchunk, Ypart, Tp, guard);
   } else if (w > 2) {
-    hipLaunchKernelGGL(qr_panel_dots<4>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol, Ypart);
+    hipLaunchKernelGGL(qr_panel_dots<4>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol, Ypart,
+                       guard);
     hipLaunchKernelGGL(qr_panel_update<4>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol,
-                       nchunk, Ypart, Tp);
+                       nchunk, Ypart, Tp, guard);
   } else {
-    hipLaunchKernelGGL(qr_panel_dots<2>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol, Ypart);
+    hipLaunchKernelGGL(qr_panel_dots<2>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol, Ypart,
+                       guard);
     hipLaunchKernelGGL(qr_panel_update<2>, grid, dim3(256), 0, st, A, m, ld, c0, w, cb, ncol,
-                       nchunk, Ypart, Tp);
+                       nchunk, Ypart, Tp, guard);
   }
+  TN_CHECK_LAUNCH();
+  return TN_OK;
+}
+
+// The block's scratch lies in buffers that only later steps use: the chunks'
+// sums in the split-K one (16 x 64 x max(n, 64) doubles), the 64 x 64 matrices
+// in the one Q is formed in (m k >= 256 x 64), the scales in the panels' T.
+static HrWs hr_carve(const QrWs& ws) {
+  HrWs h{};
+  h.part = ws.part;
+  h.G = ws.Qw;
+  h.F = h.G + HB * HB;
+  h.X = h.F + HB * HB;
+  h.M = h.X + HB * HB;
+  h.d = ws.Tp;
+  h.bad = ws.bad;
+  return h;
+}
+
+static int hr_chunks(int64_t rows) { return (int)std::min<int64_t>(HCH, ceil_div(rows, 64)); }
+
+// One 64-column block (mr x 64 at P, ld) through its orthonormal factor: P
+// becomes S R over the reflectors, V (ld mr) the explicit reflectors, T their
+// compact-WY factor; nothing is touched when *h.bad is or gets raised.
+static int hr_block(double* P, int64_t mr, int64_t ld, double* V, double* T, const HrWs& h,
+                    hipStream_t st) {
+  const int nc = hr_chunks(mr);
+  hipLaunchKernelGGL(hr_gram, dim3(nc), dim3(256), 0, st, P, mr, ld, nc, h.part, h.bad, 0);
+  hipLaunchKernelGGL(hr_scale, dim3(16), dim3(256), 0, st, h.part, nc, h.G, h.d, h.delta, h.bad);
+  TN_CHECK_LAUNCH();
+  TN_TRY(chol_block(h.G, HB, 0, HB, h.delta, h.F, h.X, st, h.bad));
+  hipLaunchKernelGGL(hr_apply, dim3((unsigned)ceil_div(mr, HROWS)), dim3(256), 0, st, P, mr, ld,
+                     h.X, h.d, V, mr, (double*)nullptr, (int64_t)0, h.bad);
+  hipLaunchKernelGGL(hr_gram, dim3(nc), dim3(256), 0, st, V, mr, mr, nc, h.part, h.bad, 0);
+  hipLaunchKernelGGL(hr_reflect, dim3(1), dim3(512), 0, st, h.part, nc, h.F, h.d, V, mr, P, ld,
+                     h.M, T, h.bad);
+  hipLaunchKernelGGL(hr_apply, dim3((unsigned)ceil_div(mr - HB, HROWS)), dim3(256), 0, st, V + HB,
+                     mr - HB, mr, h.M, (const double*)nullptr, V + HB, mr, P + HB, ld, h.bad);
+  TN_CHECK_LAUNCH();
+  return TN_OK;
+}
+
+// G (64 x 64) = V^T V (mr x 64), only while *guard is raised.
+static int gram_guarded(const double* V, int64_t mr, const HrWs& h, double* G, const int* guard,
+                        hipStream_t st) {
+  const int nc = hr_chunks(mr);
+  hipLaunchKernelGGL(hr_gram, dim3(nc), dim3(256), 0, st, V, mr, mr, nc, h.part, guard, 1);
+  hipLaunchKernelGGL(hr_gram_sum, dim3(16), dim3(256), 0, st, h.part, nc, G, guard);
   TN_CHECK_LAUNCH();
   return TN_OK;
 }
@@ -661,27 +726,40 @@ static int run_apply_panel(double* A, int64_t m, int64_t ld, int64_t c0, int w, 
 // Factor W (m x n column-major, ld=m) in place; fills tau and the per-block T.
 int qr_factor(double* W, int64_t m, int64_t n, const QrWs& ws, hipStream_t st) {
   const int64_t k = std::min(m, n);
+  HrWs h = hr_carve(ws);
+  if (k >= HB && m >= HR_MIN_ROWS) hipLaunchKernelGGL(hr_reset, dim3(1), dim3(1), 0, st, h.bad);
   for (int64_t j0 = 0; j0 < k; j0 += QR_NB) {
     const int nbo = (int)std::min<int64_t>(QR_NB, k - j0);
+    const int64_t mr = m - j0;
+    double* T = ws.Tall + (j0 / QR_NB) * QR_NB * QR_NB;
+    // whole blocks with rows enough to pay: through the orthonormal factor
+    // (tn_qr_hr.h), the panels below then only run if it gave up
+    const bool hr = nbo == HB && mr >= HR_MIN_ROWS;
+    const int* guard = hr ? h.bad : nullptr;
+    h.delta = ws.tau + j0;  // (the panels' taus come after)
+    if (hr) TN_TRY(hr_block(W + j0 + j0 * m, mr, m, ws.V, T, h, st));
     // inner panels inside the outer block
     for (int64_t jj = j0; jj < j0 + nbo;) {
       int wmax = panel_width(m - jj);
       int w = (int)std::min<int64_t>(wmax, j0 + nbo - jj);
-      TN_TRY(run_panel(W, m, m, jj, w, ws.tau, ws.Tp, ws.Ypart, st));
-      TN_TRY(run_apply_panel(W, m, m, jj, w, ws.Tp, jj + w, j0 + nbo, ws.Ypart, st));
+      TN_TRY(run_panel(W, m, m, jj, w, ws.tau, ws.Tp, ws.Ypart, guard, st));
+      TN_TRY(run_apply_panel(W, m, m, jj, w, ws.Tp, jj + w, j0 + nbo, ws.Ypart, guard, st));
       jj += w;
     }
     // compact-WY for the whole outer block (also used to form Q)
-    const int64_t mr = m - j0;
     hipLaunchKernelGGL(qr_build_v_kernel, dim3((unsigned)ceil_div(mr * nbo, 256)), dim3(256), 0,
-                       st, W, m, m, j0, nbo, ws.V);
+                       st, W, m, m, j0, nbo, ws.V, guard);
     TN_CHECK_LAUNCH();
-    // G = V^T V
-    TN_TRY(contract_launch(ws.V, mk({nbo}, {mr}), mk({mr}, {1}), ws.V, mk({mr}, {1}),
-                           mk({nbo}, {mr}), ws.G, mk({nbo}, {nbo}), mk({nbo}, {1}), TN_F64,
-                           TN_PREC_NATIVE, 1.0, 0.0, ws.part, ws.part_bytes, st));
-    double* T = ws.Tall + (j0 / QR_NB) * QR_NB * QR_NB;
-    hipLaunchKernelGGL(qr_larft_kernel, dim3(1), dim3(256), 0, st, ws.G, nbo, ws.tau + j0, T);
+    // G = V^T V, T from it
+    if (hr) {
+      TN_TRY(gram_guarded(ws.V, mr, h, ws.G, guard, st));
+    } else {
+      TN_TRY(contract_launch(ws.V, mk({nbo}, {mr}), mk({mr}, {1}), ws.V, mk({mr}, {1}),
+                             mk({nbo}, {mr}), ws.G, mk({nbo}, {nbo}), mk({nbo}, {1}), TN_F64,
+                             TN_PREC_NATIVE, 1.0, 0.0, ws.part, ws.part_bytes, st));
+    }
+    hipLaunchKernelGGL(qr_larft_kernel, dim3(1), dim3(256), 0, st, ws.G, nbo, ws.tau + j0, T,
+                       guard);
     TN_CHECK_LAUNCH();
     const int64_t nt = n - (j0 + nbo);
     if (nt > 0) {
@@ -725,7 +803,7 @@ int qr_form_q(const double* W, int64_t m, int64_t n, const QrWs& ws, double* Qw,
     const int64_t c0 = init == nullptr ? j0 : 0;
     const int64_t mr = m - j0, nc = k - c0;
     hipLaunchKernelGGL(qr_build_v_kernel, dim3((unsigned)ceil_div(mr * nbo, 256)), dim3(256), 0,
-                       st, W, m, m, j0, nbo, ws.V);
+                       st, W, m, m, j0, nbo, ws.V, (const int*)nullptr);
     TN_CHECK_LAUNCH();
     const double* T = ws.Tall + b * QR_NB * QR_NB;
     double* Qs = Qw + j0 + c0 * m;

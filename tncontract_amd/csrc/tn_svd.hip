@@ -346,7 +346,7 @@ __global__ void init_identity(double* __restrict__ Z, int64_t k) {
 
 struct SvdWs {
   double *Wv, *Z, *Gpart, *sig, *S, *R, *QZ, *Rtmp;
-  int *skip, *perm, *vp;
+  int *perm, *vp;
   unsigned long long* off;
   QrWs qr;
   char* cq;  // Cholesky QR workspace
@@ -375,7 +375,6 @@ static size_t svd_layout(int64_t m, int64_t n, char* base, size_t cap, SvdWs* ou
   w.Gpart = a.take<double>((size_t)npairs * ceil_div(Lj, GCH) * J2 * J2);
   w.sig = a.take<double>((size_t)k);
   w.S = a.take<double>((size_t)k);
-  w.skip = a.take<int>((size_t)npairs);
   w.perm = a.take<int>((size_t)k);
   w.off = a.take<unsigned long long>(4);
   if (w.precond) {
@@ -833,7 +832,6 @@ static size_t eig_layout(int64_t n, char* base, size_t cap, EigWs* out) {
   e.jw.Gpart = a.take<double>((size_t)npairs * ceil_div(n, GCH) * J2 * J2);
   e.jw.sig = a.take<double>((size_t)n);
   e.jw.S = a.take<double>((size_t)n);
-  e.jw.skip = a.take<int>((size_t)npairs);
   e.jw.perm = a.take<int>((size_t)n);
   e.jw.off = a.take<unsigned long long>(4);
   if (out) *out = e;
