@@ -118,11 +118,12 @@ __device__ __forceinline__ double hr_sum(const double* __restrict__ part, int nc
   return s;
 }
 
-// G (64 x 64) from the chunks' sums, when *bad is raised.
+// G (64 x 64) from the chunks' sums, over 16 CUs (one workgroup reading them
+// all took 24 us).
 __global__ void __launch_bounds__(256) hr_gram_sum(const double* __restrict__ part, int nchunk,
                                                    double* __restrict__ G,
-                                                   const int* __restrict__ bad) {
-  if (*bad == 0) return;
+                                                   const int* __restrict__ bad, int when) {
+  if (*bad != when) return;
   const int e = blockIdx.x * 256 + threadIdx.x, c = e >> 6, r = e & 63;
   G[e] = r >= c ? hr_sum(part, nchunk, r, c) : hr_sum(part, nchunk, c, r);
 }
@@ -212,7 +213,7 @@ __global__ void __launch_bounds__(256) hr_apply(const double* In, int64_t rows, 
 // readlane), the later waves then take its columns; the same column
 // operations turn I - N into M.
 constexpr int HC = 8;
-__global__ void __launch_bounds__(512) hr_reflect(const double* __restrict__ part, int nchunk,
+__global__ void __launch_bounds__(512) hr_reflect(const double* __restrict__ G,
                                                   const double* __restrict__ F,
                                                   const double* __restrict__ d,
                                                   double* __restrict__ V, int64_t ldv,
@@ -220,7 +221,7 @@ __global__ void __launch_bounds__(512) hr_reflect(const double* __restrict__ par
                                                   double* __restrict__ M, double* __restrict__ T,
                                                   int* bad) {
   if (*bad) return;
-  __shared__ double As[HB][HB + 1];   // [row][column]: N, later L^T D^{-1}
+  __shared__ __attribute__((aligned(16))) double As[HB][HB + 2];  // [row][column]: N, then L^T D^{-1}
   __shared__ double Bs[HB][HB + 1];   // [column][row]: Q1's top rows, later N's rows
   __shared__ double Ls[HB][HB];       // columns of Y_t, zero on and above the diagonal
   __shared__ double Xs[2][HC][HB];    // a panel's columns of M, then of T
@@ -235,8 +236,7 @@ __global__ void __launch_bounds__(512) hr_reflect(const double* __restrict__ par
   for (int k = 0; k < HC; ++k) {
     const int c = HC * q + k;
     Bs[c][t] = V[(int64_t)c * ldv + t];
-    // E's entry (t, c) is its entry (c, t)
-    const double e = hr_sum(part, nchunk, t > c ? t : c, t > c ? c : t) - (t == c ? 1.0 : 0.0);
+    const double e = G[c * HB + t] - (t == c ? 1.0 : 0.0);
     fine = fine && fabs(e) <= 1e-9;   // false for NaN
     As[t][c] = t < c ? e : (t == c ? 0.5 * e : 0.0);
   }
@@ -250,10 +250,16 @@ __global__ void __launch_bounds__(512) hr_reflect(const double* __restrict__ par
     x[k] = (t == c ? 1.0 : 0.0) - As[t][c];
     acc[k] = 0.0;
   }
+#pragma unroll 4
   for (int i = 0; i < HC * q + HC; ++i) {
     const double v = Bs[i][t];
+    const double2* n = (const double2*)&As[i][HC * q];
 #pragma unroll
-    for (int k = 0; k < HC; ++k) acc[k] = fma(v, As[i][HC * q + k], acc[k]);
+    for (int k = 0; k < HC; k += 2) {
+      const double2 nk = n[k / 2];
+      acc[k] = fma(v, nk.x, acc[k]);
+      acc[k + 1] = fma(v, nk.y, acc[k + 1]);
+    }
   }
 #pragma unroll
   for (int k = 0; k < HC; ++k) a[k] -= acc[k];
@@ -271,10 +277,16 @@ __global__ void __launch_bounds__(512) hr_reflect(const double* __restrict__ par
 #pragma unroll
   for (int k = 0; k < HC; ++k) As[t][HC * q + k] = rr[k];
   __syncthreads();
+#pragma unroll 4
   for (int i = 0; i < HC * q + HC; ++i) {
     const double v = Bs[i][t];                     // N[t][i]
+    const double2* n = (const double2*)&As[i][HC * q];
 #pragma unroll
-    for (int k = 0; k < HC; ++k) rr[k] = fma(v, As[i][HC * q + k], rr[k]);
+    for (int k = 0; k < HC; k += 2) {
+      const double2 nk = n[k / 2];
+      rr[k] = fma(v, nk.x, rr[k]);
+      rr[k + 1] = fma(v, nk.y, rr[k + 1]);
+    }
   }
   // LU of Q_t - S with S chosen on the way
   double sgn[HC];
