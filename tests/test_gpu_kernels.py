@@ -303,3 +303,35 @@ def test_qr_blocks_leave_special_inputs_to_the_panels(L, case):
         ref = np.linalg.qr(a)[1]
         keep = 70 if case == "zero_column" else n  # (past it the signs are rounding's)
         assert np.abs(r[:keep] - ref[:keep]).max() <= 1e-11 * np.abs(ref).max()
+
+
+# SVDs that one workgroup does in one launch (at most 32 vectors of at most
+# 256), at both limits and just past them, full, graded and rank-deficient,
+# FP64 and FP32 in; bounds as for test_svd_matches_lapack's sizes: k eps for
+# the values, a few sweeps' rounding for the factors.
+@pytest.mark.parametrize("m,n", [(1, 7), (2, 2), (15, 256), (256, 16), (17, 257), (31, 31),
+                                 (32, 32), (32, 33), (256, 32), (257, 32), (32, 256)])
+@pytest.mark.parametrize("case", ["full", "graded", "rank", "zero_vectors"])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_svd_in_one_workgroup(L, m, n, case, dtype):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(m * 300 + n)
+    a, k = rng.standard_normal((m, n)), min(m, n)
+    if case == "graded":
+        a = (a[:, :1] if n == 1 else a) * (10.0 ** -np.linspace(0, 12, n))
+    elif case == "rank":
+        r = max(1, k // 3)
+        a = a[:, :r] @ rng.standard_normal((r, n))
+    elif case == "zero_vectors":
+        a[:, ::2] = 0.0
+    a = a.astype(dtype)
+    u, s, vt = (x.cpu().numpy().astype(np.float64) for x in T._svd_device(dev(a), 1))
+    a = a.astype(np.float64)
+    ref = np.linalg.svd(a, compute_uv=False)
+    eps = 2e-13 if dtype == np.float64 else 2e-6
+    assert np.abs(s - ref).max() <= 1e-13 * max(ref[0], 1e-300)
+    assert np.all(np.diff(s) <= 0)
+    assert np.linalg.norm((u * s) @ vt - a) <= eps * max(ref[0], 1e-300) * np.sqrt(k)
+    big = int(np.count_nonzero(ref > 1e-10 * ref[0]))
+    assert np.abs(u[:, :big].T @ u[:, :big] - np.eye(big)).max() <= eps
+    assert np.abs(vt[:big] @ vt[:big].T - np.eye(big)).max() <= eps

@@ -19,7 +19,8 @@
 // and replayed.
 // A sweep is nblk-1 steps; sweeps repeat until the largest normalised
 // off-diagonal of a whole sweep is <= tol.  Singular values are the vector
-// norms; they are sorted descending on the device.
+// norms; they are sorted descending on the device.  At most 32 vectors of
+// length at most 256 are done by one workgroup in one launch (jac_small).
 #include "tn_internal.h"
 #include "tn_jacobi.h"
 #include "tn_prof.h"
@@ -181,6 +182,226 @@ __global__ void __launch_bounds__(EIG_NT) jac_eig_apply(double* __restrict__ Wv,
   apply_rows_finish<NT, EIG_NW>(base, ld, nv, rs, re, I, J, x, sm.Q);
 }
 
+// At most 32 vectors of length at most kSmallLen (one block pair, so a sweep
+// is one step): everything from the vectors to the rotated ones by one
+// workgroup in one launch, in LDS and registers; the host is told the outcome
+// once.  Two launches and a read-back per sweep, and a factorisation of some
+// thirty launches before them, spent most of a small SVD waiting (32 x 32: 618
+// -> 212 us a call, 31 x 31: 480 -> 209, a 16 x 16 eigensolve 389 -> 168).
+// QR = false: one-sided Jacobi of the vectors in Wv (in place).  QR = true,
+// the preconditioned SVD: the vectors by descending norm (order in vp),
+// X' = Q R by Householder's method, Jacobi on the rows of R (rotated rows to
+// R, vector-contiguous) and Q Z to QZ.  info = {sweeps, converged}.
+constexpr int kSmallLen = 256;
+
+// NaN ranks as -inf so that ranks stay a permutation of 0..k-1.
+__device__ __forceinline__ double rank_key(double x) { return x == x ? x : -INFINITY; }
+
+// Sum over the lane's row of 16.
+__device__ __forceinline__ double row16_sum(double v) {
+  v += dpp_f64<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
+  v += dpp_f64<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
+  v += dpp_f64<0x141, 0xF>(v);  // row_half_mirror
+  v += dpp_f64<0x140, 0xF>(v);  // row_mirror
+  return v;
+}
+
+template <bool QR>
+__global__ void __launch_bounds__(EIG_NT) jac_small(double* __restrict__ Wv, int L, int k,
+                                                    double tol, int max_sweeps,
+                                                    double* __restrict__ R,
+                                                    double* __restrict__ QZ, int* __restrict__ vp,
+                                                    int* __restrict__ info) {
+  constexpr int LW = kSmallLen + 4, LZ = J2 + 4, NI = kSmallLen / 16;
+  __shared__ double W[J2][LW];
+  __shared__ double Zs[QR ? J2 : 1][LZ], Rv[QR ? J2 : 1][LZ];
+  __shared__ double vcol[QR ? 2 : 1][QR ? kSmallLen : 1], nrm[J2], taus[J2];
+  __shared__ EigLds sm;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  const int q = tid >> 4, l = tid & 15;  // QR: this thread's column and first row (every 16th)
+  const int ni = (L + 15) >> 4;
+  if constexpr (!QR) {
+    for (int e = tid; e < J2 * 16 * ni; e += EIG_NT) {
+      const int v = e / (16 * ni), r = e - v * 16 * ni;
+      W[v][r] = (v < k && r < L) ? Wv[(int64_t)v * L + r] : 0.0;
+    }
+    lds_barrier();
+  } else {
+    double x[NI];
+    double s2 = 0.0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = l + 16 * i;
+      x[i] = (q < k && r < L) ? Wv[(int64_t)q * L + r] : 0.0;
+      s2 = fma(x[i], x[i], s2);
+    }
+    s2 = row16_sum(s2);
+    if (l == 0) nrm[q] = rank_key(s2);
+    lds_barrier();
+    // the columns by descending norm (ties and the zero padding in order)
+    int rank = 0;
+    if (q < k) {
+      const double mine = rank_key(s2);
+      for (int i = 0; i < k; ++i) rank += (nrm[i] > mine || (nrm[i] == mine && i < q)) ? 1 : 0;
+    } else {
+      rank = q;
+    }
+    if (l == 0 && q < k) vp[rank] = q;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (i < ni) W[rank][l + 16 * i] = x[i];
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x[i] = i < ni ? W[q][l + 16 * i] : 0.0;
+    // Householder (dlarfg's convention), one barrier a column: column j goes
+    // to LDS, and every column sums its own dot below the pivot and the
+    // norm; v . x_q = x_q[j] + scale S_q
+    for (int j = 0; j < k; ++j) {
+      double* vc = vcol[j & 1];
+      if (q == j) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          if (i < ni) vc[l + 16 * i] = x[i];
+      }
+      lds_barrier();
+      double v[NI], n2 = 0.0, dot = 0.0;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int r = l + 16 * i;
+        v[i] = (i < ni && r > j) ? vc[r] : 0.0;
+        n2 = fma(v[i], v[i], n2);
+        dot = fma(v[i], x[i], dot);
+      }
+      n2 = row16_sum(n2);
+      dot = row16_sum(dot);
+      const double alpha = vc[j];
+      // this column's pivot-row entry, held by lane j % 16 of its row
+      const double pv = __shfl(j < 16 ? x[0] : x[1], (lane & 48) | (j & 15), 64);
+      double tj = 0.0, scale = 0.0, beta = alpha;
+      if (n2 != 0.0) {  // NaN too: it has to reach R
+        const double h = sqrt(alpha * alpha + n2);
+        beta = alpha >= 0.0 ? -h : h;
+        tj = (beta - alpha) / beta;
+        scale = 1.0 / (alpha - beta);
+      }
+      if (q == j) {
+        if (l == 0) taus[j] = tj;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int r = l + 16 * i;
+          x[i] = r > j ? x[i] * scale : (r == j ? beta : x[i]);
+        }
+      } else if (q > j) {
+        const double w = tj * fma(scale, dot, pv), ws = w * scale;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int r = l + 16 * i;
+          x[i] = r == j ? x[i] - w : fma(-ws, v[i], x[i]);
+        }
+      }
+    }
+    // reflectors to W, the rows of R to Rv, Z = I
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (i < ni) W[q][l + 16 * i] = x[i];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = l + 16 * i;
+      Rv[r][q] = (r <= q && r < k && q < k) ? x[i] : 0.0;
+      Zs[q][r] = r == q ? 1.0 : 0.0;
+    }
+    lds_barrier();
+  }
+  double* const V = QR ? &Rv[0][0] : &W[0][0];
+  constexpr int LV = QR ? LZ : LW;
+  const int nt = QR ? 2 : ni;  // 16-row tiles of the Jacobi vectors
+  // rows 16 t .. 16 t + 15 of the vectors at B (row pitch ld) <- rows . Q
+  auto apply = [&](double* B, int ld, int t) {
+    double x[8];
+    double* p = B + 16 * t + lr;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) x[ks] = p[(4 * ks + lk) * ld];
+    f64x4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+        acc[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(sm.Q[4 * ks + lk][16 * mt + lr], x[ks],
+                                                       acc[mt], 0, 0, 0);
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[(16 * mt + lk + 4 * e) * ld] = acc[mt][e];
+  };
+  const int ti = (wave >> 1) & 1, tj = wave & 1;
+  int sweep = 0, done = 0;
+  while (sweep < max_sweeps) {
+    // Gram: wave w the quarter w % 4 over every other group of four rows
+    f64x4 acc = {0, 0, 0, 0};
+    for (int r = 4 * (wave >> 2); r < 16 * nt; r += 8)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(V[(16 * ti + lr) * LV + r + lk],
+                                                 V[(16 * tj + lr) * LV + r + lk], acc, 0, 0, 0);
+    const int gc = eig_pos(16 * tj + lr);
+    if (wave >= 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sm.G[1][eig_pos(16 * ti + lk + 4 * e)][gc] = acc[e];
+    }
+    lds_barrier();
+    if (wave < 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int gr = eig_pos(16 * ti + lk + 4 * e);
+        sm.G[0][gr][gc] = acc[e] + sm.G[1][gr][gc];
+      }
+    }
+    lds_barrier();
+    ++sweep;
+    if (eig_off(sm, tol) <= tol) {
+      done = 1;
+      break;
+    }
+    eig_rotate(sm, tol);
+    for (int t = wave; t < nt + (QR ? 2 : 0); t += EIG_NW) {
+      if (t < nt) apply(V, LV, t);
+      else apply(&Zs[0][0], LZ, t - nt);
+    }
+    lds_barrier();
+  }
+  if (tid == 0) {
+    info[0] = sweep;
+    info[1] = done;
+  }
+  if constexpr (!QR) {
+    for (int e = tid; e < k * L; e += EIG_NT) {
+      const int v = e / L, r = e - v * L;
+      Wv[e] = W[v][r];
+    }
+  } else {
+    for (int e = tid; e < k * k; e += EIG_NT) R[e] = Rv[e / k][e % k];
+    // column q of Q [Z; 0]: the reflectors in reverse, within the row of 16
+    double x[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x[i] = i < 2 ? Zs[q][l + 16 * i] : 0.0;
+    for (int j = k - 1; j >= 0; --j) {
+      double v[NI], dot = 0.0;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int r = l + 16 * i;
+        v[i] = (i < ni && r > j) ? W[j][r] : (r == j ? 1.0 : 0.0);
+        dot = fma(v[i], x[i], dot);
+      }
+      const double w = taus[j] * row16_sum(dot);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) x[i] = fma(-w, v[i], x[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = l + 16 * i;
+      if (q < k && r < L) QZ[(int64_t)q * L + r] = x[i];
+    }
+  }
+}
+
 // Convergence of the whole vector set from its Gram matrix G = Wv^T Wv
 // (k x k, either triangle): eig_off's measure over every pair (p < q), so
 // "off <= tol" holds exactly when a sweep would rotate no pair of G.
@@ -220,7 +441,6 @@ __global__ void __launch_bounds__(256) vec_norms(const double* __restrict__ Wv, 
 
 // perm[rank] = j with rank = #{i : s_i > s_j or (s_i == s_j and i < j)};
 // NaN ranks as -inf so that the ranks stay a permutation of 0..k-1.
-__device__ __forceinline__ double rank_key(double x) { return x == x ? x : -INFINITY; }
 
 // 64 elements j per block of 256 threads (k = 1024 spreads over 16 CUs;
 // 1024-thread blocks of 256 elements kept it on 4 and took 15.5 us): the
@@ -354,13 +574,28 @@ struct SvdWs {
   int precond;
 };
 
+// One workgroup and one launch (jac_small).
+static bool small_jacobi(int64_t L, int64_t k) { return k <= J2 && L <= kSmallLen; }
+
+// Reads back jac_small's outcome.
+static int small_outcome(int* info, int* sweeps_out, bool* converged, hipStream_t st) {
+  int h[2] = {0, 0};
+  TN_HIP(hipMemcpyAsync(h, info, sizeof(h), hipMemcpyDeviceToHost, st));
+  TN_HIP(hipStreamSynchronize(st));
+  if (sweeps_out) *sweeps_out = h[0];
+  *converged = h[1] != 0;
+  return TN_OK;
+}
+
 // Precondition with a QR (static norm pivot, then Jacobi on the rows of R)
 // whenever there are at least 32 vectors: besides shortening long vectors, it
 // grades the problem, so square matrices with spread spectra (bond matrices)
 // need far fewer sweeps (22 -> 8 for a 128 x 128 matrix with singular values
 // from 1 to 1e-6, 10 -> 9 for a Gaussian one, in a simulation of this block
-// Jacobi).
-static bool use_precond(int64_t L, int64_t k) { return k >= 32 && L >= k; }
+// Jacobi).  What one workgroup does alone (jac_small) is preconditioned at
+// every size: without it the rounding-level vectors of a rank-deficient
+// matrix keep being rotated.
+static bool use_precond(int64_t L, int64_t k) { return k >= 32 || small_jacobi(L, k); }
 
 static size_t svd_layout(int64_t m, int64_t n, char* base, size_t cap, SvdWs* out) {
   const int64_t k = std::min(m, n), L = std::max(m, n);
@@ -382,6 +617,8 @@ static size_t svd_layout(int64_t m, int64_t n, char* base, size_t cap, SvdWs* ou
     w.Rtmp = a.take<double>((size_t)(k * k));
     w.QZ = a.take<double>((size_t)(L * k));
     w.vp = a.take<int>((size_t)k);
+  }
+  if (w.precond && !small_jacobi(L, k)) {
     size_t qbytes = qr_layout(L, k, nullptr, 0, nullptr) + 256;
     char* qbase = a.take<char>(qbytes);
     if (base) qr_layout(L, k, qbase, qbytes, &w.qr);
@@ -407,6 +644,13 @@ __global__ void copy_f64(const double* __restrict__ src, double* __restrict__ ds
 static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& w, double tol,
                       int max_sweeps, int* sweeps_out, bool* converged, hipStream_t st,
                       bool allow_graph = true, double* sort_tmp = nullptr) {
+  *converged = false;
+  if (Z == nullptr && small_jacobi(L, k)) {
+    hipLaunchKernelGGL(jac_small<false>, dim3(1), dim3(EIG_NT), 0, st, Wv, (int)L, (int)k, tol,
+                       max_sweeps, (double*)nullptr, (double*)nullptr, (int*)nullptr, (int*)w.off);
+    TN_CHECK_LAUNCH();
+    return small_outcome((int*)w.off, sweeps_out, converged, st);
+  }
   int nblk = (int)ceil_div(std::max<int64_t>(k, 1), JB);
   if (nblk % 2) nblk += 1;
   const int npairs = nblk / 2;
@@ -420,7 +664,6 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
     hipLaunchKernelGGL(init_identity, dim3((unsigned)ceil_div(k * k, 256)), dim3(256), 0, st, Z, k);
   TN_CHECK_LAUNCH();
   int sweep = 0;
-  *converged = false;
   // algorithmic work per step: Gram 2 L (2b)^2 per pair, apply 2 (L + k) (2b)^2 per pair
   const double gram_fl = 2.0 * (double)L * J2 * J2 * npairs;
   const double apply_fl = 2.0 * (double)(L + kz) * J2 * J2 * npairs;
@@ -604,7 +847,17 @@ static int svd_impl(const void* A, const tn_modes* a_rows, const tn_modes* a_col
   int64_t orth_len;
   const int* upm = nullptr;
   const int* vpm = nullptr;
-  if (w.precond) {
+  if (w.precond && small_jacobi(L, k)) {
+    if (tol <= 0.0) tol = std::max(1e-15, (double)k * 2.220446049250313e-16);
+    hipLaunchKernelGGL(jac_small<true>, dim3(1), dim3(EIG_NT), 0, st, w.Wv, (int)L, (int)k, tol,
+                       max_sweeps, w.R, w.QZ, w.vp, (int*)w.off);
+    TN_CHECK_LAUNCH();
+    TN_TRY(small_outcome((int*)w.off, sweeps_out, &converged, st));
+    orth_src = w.R;
+    orth_len = k;
+    if (tall) { Uvec = w.QZ; ldu = L; u_scaled = 0; Vvec = w.R; ldv = k; v_scaled = 1; vpm = w.vp; }
+    else { Uvec = w.R; ldu = k; u_scaled = 1; Vvec = w.QZ; ldv = L; v_scaled = 0; upm = w.vp; }
+  } else if (w.precond) {
     // Static pivot: X' = X P with the vectors by descending norm (R R^T is
     // then closer to diagonal and the Jacobi needs fewer sweeps).
     // X' = Q R; one-sided Jacobi on the rows of R (R^T Z = W''), then
