@@ -335,3 +335,31 @@ def test_svd_in_one_workgroup(L, m, n, case, dtype):
     big = int(np.count_nonzero(ref > 1e-10 * ref[0]))
     assert np.abs(u[:, :big].T @ u[:, :big] - np.eye(big)).max() <= eps
     assert np.abs(vt[:big] @ vt[:big].T - np.eye(big)).max() <= eps
+
+
+# Jacobi with the inner pairs at every fourth step (more than four blocks of
+# 16 vectors), from the last size without to a few past a whole block: the SVD
+# (rotations accumulated) and the PSD eigensolver; bounds as above.
+@pytest.mark.parametrize("n", [64, 65, 96, 97, 130, 257])
+@pytest.mark.parametrize("case", ["full", "graded", "clusters", "rank"])
+def test_jacobi_inner_pairs_every_fourth_step(L, n, case):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n))
+    if case != "full":
+        u, v = np.linalg.qr(a)[0], np.linalg.qr(rng.standard_normal((n, n)))[0]
+        s = {"graded": np.logspace(0, -12, n), "clusters": 10.0 ** -(np.arange(n) % 3),
+             "rank": np.where(np.arange(n) < n // 3, 1.0, 0.0)}[case]
+        a = (u * s) @ v
+    ref = np.linalg.svd(a, compute_uv=False)
+    u, s, vt = (x.cpu().numpy() for x in T._svd_device(dev(a), 1))
+    assert np.abs(s - ref).max() <= 2e-13 * ref[0]
+    assert np.linalg.norm((u * s) @ vt - a) <= 4e-13 * ref[0] * np.sqrt(n)
+    big = int(np.count_nonzero(ref > 1e-10 * ref[0]))
+    assert np.abs(u[:, :big].T @ u[:, :big] - np.eye(big)).max() <= 4e-13
+    assert np.abs(vt[:big] @ vt[:big].T - np.eye(big)).max() <= 4e-13
+    K = a.T @ a
+    w, lam = (x.cpu().numpy() for x in T._eigh_psd_device(dev(K), 1)[:2])
+    assert np.linalg.norm((w * lam) @ w.T - K) <= 4e-13 * ref[0] ** 2 * np.sqrt(n)
+    big = int(np.count_nonzero(ref > 1e-5 * ref[0]))
+    assert np.abs(w[:, :big].T @ w[:, :big] - np.eye(big)).max() <= 4e-13

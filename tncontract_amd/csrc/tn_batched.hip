@@ -259,6 +259,12 @@ __global__ void __launch_bounds__(256) bjac_gram(double* __restrict__ Wv, const 
   }
 }
 
+// a pair eigensolve in the work counter: the number in the low half, the
+// rounds in the high one
+__device__ __forceinline__ unsigned long long eig_count(bool inner) {
+  return 1ull + ((unsigned long long)step_rounds(inner) << 32);
+}
+
 // eig items are (job, pair) in job-major order; Gpart items for (job, pair,
 // chunk) start at gram_base + pair * nch.
 __global__ void __launch_bounds__(EIG_NT) bjac_eig(const double* __restrict__ Gpart,
@@ -266,6 +272,7 @@ __global__ void __launch_bounds__(EIG_NT) bjac_eig(const double* __restrict__ Gp
                                                 const int* __restrict__ e_job,
                                                 const int* __restrict__ e_pair,
                                                 const int* __restrict__ done,
+                                                const int* __restrict__ gbase, int goff,
                                                 double* __restrict__ Qall, int* __restrict__ skip,
                                                 unsigned long long* __restrict__ offmax,
                                                 unsigned long long* __restrict__ work) {
@@ -309,15 +316,16 @@ __global__ void __launch_bounds__(EIG_NT) bjac_eig(const double* __restrict__ Gp
     }
   }
   __syncthreads();
-  const double off = eig_off(sm, J.tol, J.neg2);
+  const bool inner = inner_step((*gbase + goff) % (J.nblk - 1), J.nblk);
+  const double off = eig_off(sm, J.tol, J.neg2, inner);
   if (tid == 0) atomicMax(offmax + j, dbits(off));
   if (off <= J.tol) {
     if (tid == 0) skip[item] = 1;
     return;
   }
   if (tid == 0) skip[item] = 0;
-  if (work && tid == 0) atomicAdd(work + 1, 1ull);
-  eig_rotate(sm, J.tol, J.neg2);
+  if (work && tid == 0) atomicAdd(work + 1, eig_count(inner));
+  eig_rotate(sm, J.tol, J.neg2, inner);
   double* out = Qall + (int64_t)item * (BJ2 * BJ2);
   for (int e = tid; e < BJ2 * BJ2; e += EIG_NT) out[e] = sm.Q[e / BJ2][e % BJ2];
 }
@@ -414,15 +422,16 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
     for (int e = 0; e < 4; ++e) sm.G[0][gr[e]][gc] = acc[e] + sm.G[1][gr[e]][gc];
   }
   lds_barrier();
-  const double off = eig_off(sm, J.tol, J.neg2);
+  const bool inner = inner_step(s, J.nblk);
+  const double off = eig_off(sm, J.tol, J.neg2, inner);
   if (tid == 0) atomicMax(offmax + j, dbits(off));
   if (off <= J.tol) return;
   if (work && tid == 0) {
     atomicAdd(work, (unsigned long long)J.L);
-    atomicAdd(work + 1, 1ull);
+    atomicAdd(work + 1, eig_count(inner));
     atomicAdd(work + 2, (unsigned long long)(J.L + J.k));
   }
-  eig_rotate(sm, J.tol, J.neg2);
+  eig_rotate(sm, J.tol, J.neg2, inner);
   apply_rows_finish<2, EIG_NW>(W, J.L, J.k, 0, J.L, I, K2, x, sm.Q);
   apply_rows_finish<2, EIG_NW>(Z, J.k, J.k, 0, J.k, I, K2, z, sm.Q);
 }
@@ -1067,7 +1076,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
         {
           ProfScope p(PROF_JAC_EIG, st, 0.0, 0.0);
           hipLaunchKernelGGL(bjac_eig, dim3(nei), dim3(EIG_NT), 0, st, dG, dbj, det, det + nei, ddone,
-                             dQ, dskip, doff, cnt);
+                             dgbase, o, dQ, dskip, doff, cnt);
         }
         {
           ProfScope p(PROF_JAC_APPLY, st, 0.0, 0.0);
@@ -1172,9 +1181,10 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   if (cnt) {
     // a Gram row of a 32-column block pair: 32 x 32 multiply-adds, 32 values
     // read; a rotated row: the same product, 32 values read and written; a
-    // 32 x 32 eigensolve: 31 rotation rounds of about 9216 flops
+    // round of a 32 x 32 eigensolve: about 9216 flops
     prof_add(PROF_JAC_GRAM, 2.0 * BJ2 * BJ2 * (double)hw[0], 8.0 * BJ2 * (double)hw[0]);
-    prof_add(PROF_JAC_EIG, 31.0 * 9216.0 * (double)hw[1], 16.0 * BJ2 * BJ2 * (double)hw[1]);
+    prof_add(PROF_JAC_EIG, 9216.0 * (double)(hw[1] >> 32),
+             16.0 * BJ2 * BJ2 * (double)(hw[1] & 0xffffffffu));
     prof_add(PROF_JAC_APPLY, 2.0 * BJ2 * BJ2 * (double)hw[2], 16.0 * BJ2 * (double)hw[2]);
   }
   for (int j = 0; j < njobs; ++j)

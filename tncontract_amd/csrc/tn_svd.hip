@@ -12,7 +12,8 @@
 //   2. jac_eig_apply: every block of a pair sums the partials, records the
 //                 largest normalised off-diagonal |G_pq|/sqrt(G_pp G_qq),
 //                 runs one cyclic sweep of two-sided Jacobi on the 32x32 G
-//                 in LDS accumulating Q (the same Q in every block), and
+//                 (at most steps the pairs across the two blocks only) in
+//                 LDS accumulating Q (the same Q in every block), and
 //                 applies [W_I W_J] <- [W_I W_J] Q (or [Z_I Z_J] Q) to its
 //                 row chunk by MFMA (grid: pairs x row chunks).
 // The two kernels of every step of a sweep are captured once as a HIP graph
@@ -175,10 +176,11 @@ __global__ void __launch_bounds__(EIG_NT) jac_eig_apply(double* __restrict__ Wv,
   eig_load(sm, Gpart + (int64_t)pi * nchG * (J2 * J2), nchG);
   double x[8][NT];
   apply_rows_fetch<NT, EIG_NW>(base, ld, nv, rs, re, I, J, x);   // in flight during the rounds
-  const double off = eig_off(sm, tol);
+  const bool inner = inner_step(s, nblk);
+  const double off = eig_off(sm, tol, 0.0, inner);
   if (ch == 0 && threadIdx.x == 0) atomicMax(offmax, dbits(off));
   if (off <= tol) return;
-  eig_rotate(sm, tol);
+  eig_rotate(sm, tol, 0.0, inner);
   apply_rows_finish<NT, EIG_NW>(base, ld, nv, rs, re, I, J, x, sm.Q);
 }
 
@@ -694,11 +696,12 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
       {
         // a kernel boundary between the partials and the pair eigensolve is
         // cheaper than a device-scope fence + arrival counter in the Gram
-        // kernel (measured).  Work: the inner sweep (31 rounds x 9216 flops)
+        // kernel (measured).  Work: the inner sweep (31 or 16 rounds x 9216 flops)
         // once per pair plus the apply; HBM bytes: each pair's partials once
         // (the other row blocks of the pair re-read them from L2) + the
         // chunks read and written
-        ProfScope p(PROF_JAC_EIG, st, 31.0 * 9216.0 * npairs + apply_fl,
+        ProfScope p(PROF_JAC_EIG, st,
+                    step_rounds(inner_step(s, nblk)) * 9216.0 * npairs + apply_fl,
                     8.0 * (double)nchG * J2 * J2 * npairs + 16.0 * (double)(L + kz) * J2 * npairs);
         const dim3 eg(npairs, nchW + nchZ);
         if (ent == 1)
