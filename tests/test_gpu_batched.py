@@ -99,3 +99,23 @@ def test_batched_svd_qr_preconditioned_edges(tn):
         np.testing.assert_allclose(u[:, :r].T @ u[:, :r], np.eye(r), atol=1e-11)
         np.testing.assert_allclose(vt[:r] @ vt[:r].T, np.eye(r), atol=1e-11)
     assert sweeps.max() <= 20, sweeps
+
+
+# Products of low rank: the Jacobi first sweeps over the blocks of vectors
+# that are not negligible alone.  Ranks on both sides of a pair of blocks, with
+# the job's vectors within one row chunk (the one-launch step) and beyond it.
+@pytest.mark.parametrize("sizes", [[(40, 1, 40), (100, 31, 64), (100, 32, 70), (100, 33, 130),
+                                    (250, 64, 256), (96, 96, 96)],
+                                   [(300, 1, 290), (400, 32, 300), (64, 33, 500), (520, 65, 410),
+                                    (290, 280, 300)]])
+def test_batched_truncate_low_rank(tn, sizes):
+    from tncontract_amd.batched import batched_truncate
+    rng = np.random.default_rng(sum(s[0] for s in sizes))
+    jobs = [(rng.standard_normal((m, k)).astype(np.float32),
+             rng.standard_normal((k, n)).astype(np.float32)) for m, k, n in sizes]
+    U, S, Vt, kept, sweeps = batched_truncate([torch.from_numpy(a).cuda() for a, _ in jobs],
+                                              [torch.from_numpy(b).cuda() for _, b in jobs],
+                                              rel_threshold=1e-8)
+    for j, (Lm, Rm) in enumerate(jobs):
+        check_job(Lm, Rm, U[j], S[j], Vt[j], int(kept[j]), 1e-8, 0)
+    assert sweeps.max() < 60

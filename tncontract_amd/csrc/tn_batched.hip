@@ -178,7 +178,45 @@ struct BJob {
   // squared norm below which a vector is negligible (pairs of two such
   // vectors are not rotated; 0: none is)
   double neg2;
+  int32_t nact;   // blocks (even) up to the last one with a vector that is not negligible
 };
+
+// Where a job's Jacobi stands: step s of a sweep over its first nb blocks
+// (nb = 0: retired).  Kept twice, by the parity of the global step: a step's
+// kernels read one while the next step's is written.
+struct BState {
+  int32_t s, nb;
+};
+
+// The state after this step, by one thread per job once the step's measures
+// are in offmax.  A job first sweeps over its blocks up to nact alone, until it
+// is a sweep or two from convergence (the off-diagonal is about squared per
+// sweep, so at off <= 10 sqrt(tol)); then over all its blocks until a whole
+// sweep has nothing to rotate.  A product of rank r leaves the QR with r rows
+// and negligible ones: those then cost the last three sweeps instead of all
+// (32 products of ranks 22 .. 492 and sizes up to 1022: 46.0 -> 34.5 ms;
+// going over to all blocks a sweep later costs a sweep of the first ones).
+__device__ __forceinline__ void bstate_next(const BJob& J, int j, BState cur, int max_sweeps,
+                                            BState* __restrict__ next, int* __restrict__ done,
+                                            int* __restrict__ sweeps,
+                                            unsigned long long* __restrict__ offmax,
+                                            int* __restrict__ active) {
+  BState n{cur.s + 1, cur.nb};
+  if (cur.nb > 0 && n.s == cur.nb - 1) {
+    const double off = __longlong_as_double((long long)offmax[j]);
+    offmax[j] = 0ull;
+    const int sw = ++sweeps[j];
+    n.s = 0;
+    if (cur.nb < J.nblk) {
+      if (off * off <= 100.0 * J.tol || sw >= max_sweeps) n.nb = J.nblk;
+    } else if (off <= J.tol || sw >= max_sweeps + (J.nact < J.nblk ? 2 : 0)) {
+      done[j] = off <= J.tol ? 1 : 2;
+      atomicSub(active, 1);
+      n.nb = 0;
+    }
+  }
+  next[j] = n;
+}
 
 // acc += the 32 x 32 Gram of the pair's vectors (blocks I and K2 of the
 // job's k vectors of length L at W) over rows [r0, r1): tiles of 64 NG rows
@@ -232,18 +270,17 @@ __global__ void __launch_bounds__(256) bjac_gram(double* __restrict__ Wv, const 
                                                  const int* __restrict__ it_job,
                                                  const int* __restrict__ it_pair,
                                                  const int* __restrict__ it_chunk,
-                                                 const int* __restrict__ done,
-                                                 const int* __restrict__ gbase, int goff,
+                                                 const BState* __restrict__ state,
                                                  double* __restrict__ Gpart,
                                                  unsigned long long* __restrict__ work) {
   __shared__ double Ps[64][BJ2 + 1];
   const int item = blockIdx.x;
   const int j = it_job[item];
-  if (done[j]) return;
-  const BJob J = jobs[j];
-  const int s = (*gbase + goff) % (J.nblk - 1);
+  const BState S = state[j];
   const int pi = it_pair[item], ch = it_chunk[item];
-  const int I = brr(pi, s, J.nblk), K2 = brr(J.nblk - 1 - pi, s, J.nblk);
+  if (2 * pi >= S.nb) return;
+  const BJob J = jobs[j];
+  const int I = brr(pi, S.s, S.nb), K2 = brr(S.nb - 1 - pi, S.s, S.nb);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int ti = wave >> 1, tj = wave & 1;
   const int64_t r0 = (int64_t)ch * BCH, r1 = min((int64_t)J.L, r0 + BCH);
@@ -271,17 +308,17 @@ __global__ void __launch_bounds__(EIG_NT) bjac_eig(const double* __restrict__ Gp
                                                 const BJob* __restrict__ jobs,
                                                 const int* __restrict__ e_job,
                                                 const int* __restrict__ e_pair,
-                                                const int* __restrict__ done,
-                                                const int* __restrict__ gbase, int goff,
+                                                const BState* __restrict__ state,
                                                 double* __restrict__ Qall, int* __restrict__ skip,
                                                 unsigned long long* __restrict__ offmax,
                                                 unsigned long long* __restrict__ work) {
   __shared__ EigLds sm;
   const int item = blockIdx.x, tid = threadIdx.x;
   const int j = e_job[item];
-  if (done[j]) return;
-  const BJob J = jobs[j];
+  const BState S = state[j];
   const int pi = e_pair[item];
+  if (2 * pi >= S.nb) return;
+  const BJob J = jobs[j];
   {
     // every partial of a group of four chunks loaded before the first add
     constexpr int PER = BJ2 * BJ2 / EIG_NT;
@@ -316,7 +353,7 @@ __global__ void __launch_bounds__(EIG_NT) bjac_eig(const double* __restrict__ Gp
     }
   }
   __syncthreads();
-  const bool inner = inner_step((*gbase + goff) % (J.nblk - 1), J.nblk);
+  const bool inner = inner_step(S.s, S.nb);
   const double off = eig_off(sm, J.tol, J.neg2, inner);
   if (tid == 0) atomicMax(offmax + j, dbits(off));
   if (off <= J.tol) {
@@ -336,21 +373,26 @@ __global__ void __launch_bounds__(256) bjac_apply(double* __restrict__ Wv, doubl
                                                   const int* __restrict__ a_job,
                                                   const int* __restrict__ a_pair,
                                                   const int* __restrict__ a_chunk,
-                                                  const int* __restrict__ done,
-                                                  const int* __restrict__ gbase, int goff,
+                                                  const BState* __restrict__ state,
                                                   const double* __restrict__ Qall,
                                                   const int* __restrict__ skip,
-                                                  unsigned long long* __restrict__ work) {
+                                                  unsigned long long* __restrict__ work,
+                                                  BState* __restrict__ next, int max_sweeps,
+                                                  int* __restrict__ done, int* __restrict__ sweeps,
+                                                  unsigned long long* __restrict__ offmax,
+                                                  int* __restrict__ active) {
   __shared__ double Q[BJ2][BJ2 + 1];
   const int item = blockIdx.x;
   const int j = a_job[item];
-  if (done[j]) return;
-  const BJob J = jobs[j];
+  const BState S = state[j];
   const int pi = a_pair[item], ch = a_chunk[item];
+  const BJob J = jobs[j];
+  if (pi == 0 && ch == 0 && threadIdx.x == 0)
+    bstate_next(J, j, S, max_sweeps, next, done, sweeps, offmax, active);
+  if (2 * pi >= S.nb) return;
   const int eidx = J.eig_base + pi;
   if (skip[eidx]) return;
-  const int s = (*gbase + goff) % (J.nblk - 1);
-  const int I = brr(pi, s, J.nblk), K2 = brr(J.nblk - 1 - pi, s, J.nblk);
+  const int I = brr(pi, S.s, S.nb), K2 = brr(S.nb - 1 - pi, S.s, S.nb);
   const double* Qg = Qall + (int64_t)eidx * BJ2 * BJ2;
   const bool onW = ch < J.ncha;
   double* base = onW ? Wv + J.wv : Zb + J.z;
@@ -386,19 +428,18 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
                                                   const BJob* __restrict__ jobs,
                                                   const int* __restrict__ e_job,
                                                   const int* __restrict__ e_pair,
-                                                  const int* __restrict__ done,
-                                                  const int* __restrict__ gbase, int goff,
+                                                  const BState* __restrict__ state,
                                                   unsigned long long* __restrict__ offmax,
                                                   unsigned long long* __restrict__ work) {
   __shared__ double Ps[128][BJ2 + 1];
   __shared__ EigLds sm;
   const int item = blockIdx.x, tid = threadIdx.x;
   const int j = e_job[item];
-  if (done[j]) return;
-  const BJob J = jobs[j];
-  const int s = (*gbase + goff) % (J.nblk - 1);
+  const BState S = state[j];
   const int pi = e_pair[item];
-  const int I = brr(pi, s, J.nblk), K2 = brr(J.nblk - 1 - pi, s, J.nblk);
+  if (2 * pi >= S.nb) return;
+  const BJob J = jobs[j];
+  const int I = brr(pi, S.s, S.nb), K2 = brr(S.nb - 1 - pi, S.s, S.nb);
   const int wave = tid >> 6, lane = tid & 63;
   const int ti = (wave >> 1) & 1, tj = wave & 1;
   double* W = Wv + J.wv;
@@ -422,7 +463,7 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
     for (int e = 0; e < 4; ++e) sm.G[0][gr[e]][gc] = acc[e] + sm.G[1][gr[e]][gc];
   }
   lds_barrier();
-  const bool inner = inner_step(s, J.nblk);
+  const bool inner = inner_step(S.s, S.nb);
   const double off = eig_off(sm, J.tol, J.neg2, inner);
   if (tid == 0) atomicMax(offmax + j, dbits(off));
   if (off <= J.tol) return;
@@ -436,31 +477,18 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
   apply_rows_finish<2, EIG_NW>(Z, J.k, J.k, 0, J.k, I, K2, z, sm.Q);
 }
 
-// After global step g: retire jobs whose sweep just ended with off <= tol.
-__global__ void bjac_sweep_end(const BJob* __restrict__ jobs, int njobs,
-                               const int* __restrict__ gbase, int goff, int max_sweeps,
-                               int* __restrict__ done, int* __restrict__ sweeps,
-                               unsigned long long* __restrict__ offmax, int* __restrict__ active) {
-  int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= njobs || done[j]) return;
-  const BJob J = jobs[j];
-  if ((*gbase + goff + 1) % (J.nblk - 1) != 0) return;
-  double off = __longlong_as_double((long long)offmax[j]);
-  offmax[j] = 0ull;
-  int sw = ++sweeps[j];
-  if (off <= J.tol) {
-    done[j] = 1;
-    atomicSub(active, 1);
-  } else if (sw >= max_sweeps) {
-    done[j] = 2;
-    atomicSub(active, 1);
-  }
+// After a fused step (bjac_apply advances the jobs itself).
+__global__ void bjac_step_end(const BJob* __restrict__ jobs, int njobs,
+                              const BState* __restrict__ state, BState* __restrict__ next,
+                              int max_sweeps, int* __restrict__ done, int* __restrict__ sweeps,
+                              unsigned long long* __restrict__ offmax, int* __restrict__ active) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < njobs) bstate_next(jobs[j], j, state[j], max_sweeps, next, done, sweeps, offmax, active);
 }
 
-// The global step of a launch is *gbase + goff: a captured set of steps
-// (goff = 0 .. n-1) is replayed with the base advanced by n after each set.
-__global__ void badvance(int* __restrict__ gbase, int n) {
-  if (threadIdx.x == 0) *gbase += n;
+__global__ void binit_state(const BJob* __restrict__ jobs, int njobs, BState* __restrict__ state) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < njobs) state[j] = BState{0, jobs[j].nact};
 }
 
 __global__ void binit_identity(double* __restrict__ Zb, const BJob* __restrict__ jobs) {
@@ -476,23 +504,31 @@ __global__ void binit_identity(double* __restrict__ Zb, const BJob* __restrict__
 // the space those vectors span has singular values <= sqrt(k neg2) <=
 // thr F / (2 sqrt(k)) <= thr sigma_0 / 2 (F <= sqrt(k) sigma_0), so it lies
 // below the relative threshold thr whatever its internal orthogonality.
-__global__ void __launch_bounds__(256) bjob_neg2(const double* __restrict__ Wv,
+// Also nact, from the vectors' norms sig (one block per job summing the whole
+// matrix took 1.04 ms of 46).
+__global__ void __launch_bounds__(256) bjob_neg2(const double* __restrict__ sig,
+                                                 const int64_t* __restrict__ sbase,
                                                  BJob* __restrict__ jobs, double thr) {
   __shared__ double red[4];
+  __shared__ int last;
   BJob& J = jobs[blockIdx.x];
-  const int64_t tot = (int64_t)J.L * J.k;
+  const double* s = sig + sbase[blockIdx.x];
   double acc = 0.0;
-  for (int64_t e = threadIdx.x; e < tot; e += 256) {
-    const double x = Wv[J.wv + e];
-    acc = fma(x, x, acc);
-  }
+  for (int v = threadIdx.x; v < J.k; v += 256) acc = fma(s[v], s[v], acc);
   acc = wave_sum(acc);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  if (threadIdx.x == 0) last = 0;
+  __syncthreads();
+  const double q = thr / (2.0 * (double)J.k);
+  const double neg2 = q * q * (red[0] + red[1] + red[2] + red[3]);
+  int top = 0;
+  for (int v = threadIdx.x; v < J.k; v += 256)
+    if (s[v] * s[v] > neg2) top = v;
+  atomicMax(&last, top);
   __syncthreads();
   if (threadIdx.x == 0) {
-    const double f2 = red[0] + red[1] + red[2] + red[3];
-    const double q = thr / (2.0 * (double)J.k);
-    J.neg2 = q * q * f2;
+    J.neg2 = neg2;
+    J.nact = min(J.nblk, 2 * (last / BJ2 + 1));
   }
 }
 
@@ -761,7 +797,7 @@ static size_t batched_ws_bytes(const std::vector<int64_t>& ms, const std::vector
   a.take<double>(sv * 2);
   a.take<int>(sv);
   a.take<int64_t>((size_t)njobs);
-  a.take<int>(1);  // device step base
+  a.take<BState>((size_t)njobs * 2);
   return a.used + 4096;
 }
 
@@ -838,6 +874,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     b.tol = tj ? std::max(1e-8, (double)Lj * 2.220446049250313e-16)
                : (double)Lj * 2.220446049250313e-16;
     b.neg2 = 0.0;
+    b.nact = b.nblk;
     for (int p = 0; p < b.nblk / 2; ++p) {
       for (int c = 0; c < b.nch; ++c) { g_job.push_back(j); g_pair.push_back(p); g_chunk.push_back(c); }
       e_job.push_back(j);
@@ -932,8 +969,8 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   double* dS = a.take<double>((size_t)sv);
   int* dperm = a.take<int>((size_t)sv);
   int64_t* dsbase = a.take<int64_t>((size_t)njobs);
-  int* dgbase = a.take<int>(1);
-  TN_REQUIRE(dgbase != nullptr, "%s: workspace too small", who);
+  BState* dstate = a.take<BState>((size_t)njobs * 2);
+  TN_REQUIRE(dstate != nullptr, "%s: workspace too small", who);
   for (int j = 0; j < njobs; ++j) gj[j].C = dWv + xoff[j];
   for (const QJob& q : qj) oj[q.job].qz = dQZ + q.qz;
   std::vector<int> gt(ngi * 3), et(nei * 2), at(nai * 3);
@@ -961,7 +998,6 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   TN_HIP(hipMemsetAsync(ddone, 0, sizeof(int) * njobs, st));
   TN_HIP(hipMemsetAsync(dsweeps, 0, sizeof(int) * njobs, st));
   TN_HIP(hipMemsetAsync(doff, 0, sizeof(unsigned long long) * njobs, st));
-  TN_HIP(hipMemsetAsync(dgbase, 0, sizeof(int), st));
   // rows through the Gram and rotation kernels and eigensolves that rotated,
   // counted only while launch timing is on (they give the Jacobi rooflines)
   unsigned long long* cnt = prof_on() ? dwork : nullptr;
@@ -1047,47 +1083,55 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   hipLaunchKernelGGL(binit_identity, dim3((unsigned)ceil_div((int64_t)maxk * maxk, 256), njobs),
                      dim3(256), 0, st, dZ, dbj);
   // truncation jobs: vectors negligible against the keep threshold
-  if (tj && rel_threshold > 0.0)
-    hipLaunchKernelGGL(bjob_neg2, dim3((unsigned)njobs), dim3(256), 0, st, dWv, dbj, rel_threshold);
+  if (tj && rel_threshold > 0.0) {
+    hipLaunchKernelGGL(bvec_norms, dim3((unsigned)maxk, njobs), dim3(256), 0, st, dWv, dbj, dsig,
+                       dsbase);
+    hipLaunchKernelGGL(bjob_neg2, dim3((unsigned)njobs), dim3(256), 0, st, dsig, dsbase, dbj,
+                       rel_threshold);
+  }
+  const unsigned njb = (unsigned)ceil_div(njobs, 256);
+  hipLaunchKernelGGL(binit_state, dim3(njb), dim3(256), 0, st, dbj, njobs, dstate);
   TN_CHECK_LAUNCH();
   // every job within one row chunk: the one-launch step
   bool fused = true;
   for (int j = 0; j < njobs; ++j) fused = fused && bj[j].L <= BCH && bj[j].k <= BCH;
   // A step set of `period` steps is enqueued as one unit (captured once as a
   // HIP graph and replayed; launched kernel by kernel while launch timing is
-  // on); each set ends by advancing the device step base.  The host reads
-  // the active-job count of a set while the next set runs, so the GPU never
-  // waits for the host; a set enqueued after the last job retired exits at
-  // once in every block.
-  const int period = std::max(8, maxsteps);
+  // on).  The host reads the active-job count of a set while the next set
+  // runs, so the GPU never waits for the host; a set enqueued after the last
+  // job retired exits at once in every block.  Even (the parity of a step
+  // picks its state), and long enough that a set outlasts its launch.
+  constexpr int period = 16;
   auto enqueue_set = [&]() {
     for (int o = 0; o < period; ++o) {
+      const BState* cur = dstate + (o & 1) * njobs;
+      BState* next = dstate + (~o & 1) * njobs;
       // work is counted on the device (cnt) and added once at the end
       if (fused) {
         ProfScope p(PROF_JAC_EIG, st, 0.0, 0.0);
         hipLaunchKernelGGL(bjac_fused, dim3(nei), dim3(EIG_NT), 0, st, dWv, dZ, dbj, det, det + nei,
-                           ddone, dgbase, o, doff, cnt);
+                           cur, doff, cnt);
+        hipLaunchKernelGGL(bjac_step_end, dim3(njb), dim3(256), 0, st, dbj, njobs, cur, next,
+                           max_sweeps, ddone, dsweeps, doff, dactive);
       } else {
         {
           ProfScope p(PROF_JAC_GRAM, st, 0.0, 0.0);
           hipLaunchKernelGGL(bjac_gram, dim3(ngi), dim3(256), 0, st, dWv, dbj, dgt, dgt + ngi,
-                             dgt + 2 * ngi, ddone, dgbase, o, dG, cnt);
+                             dgt + 2 * ngi, cur, dG, cnt);
         }
         {
           ProfScope p(PROF_JAC_EIG, st, 0.0, 0.0);
-          hipLaunchKernelGGL(bjac_eig, dim3(nei), dim3(EIG_NT), 0, st, dG, dbj, det, det + nei, ddone,
-                             dgbase, o, dQ, dskip, doff, cnt);
+          hipLaunchKernelGGL(bjac_eig, dim3(nei), dim3(EIG_NT), 0, st, dG, dbj, det, det + nei, cur,
+                             dQ, dskip, doff, cnt);
         }
         {
           ProfScope p(PROF_JAC_APPLY, st, 0.0, 0.0);
           hipLaunchKernelGGL(bjac_apply, dim3(nai), dim3(256), 0, st, dWv, dZ, dbj, dat, dat + nai,
-                             dat + 2 * nai, ddone, dgbase, o, dQ, dskip, cnt);
+                             dat + 2 * nai, cur, dQ, dskip, cnt, next, max_sweeps, ddone, dsweeps,
+                             doff, dactive);
         }
       }
-      hipLaunchKernelGGL(bjac_sweep_end, dim3((unsigned)ceil_div(njobs, 256)), dim3(256), 0, st,
-                         dbj, njobs, dgbase, o, max_sweeps, ddone, dsweeps, doff, dactive);
     }
-    hipLaunchKernelGGL(badvance, dim3(1), dim3(64), 0, st, dgbase, period);
   };
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -1114,7 +1158,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     set_error(TN_ERR_HIP, "%s: host buffer or event creation failed", who);
     rc_loop = TN_ERR_HIP;
   }
-  const int nsets = (int)ceil_div((int64_t)maxsteps * max_sweeps, period);
+  const int nsets = (int)ceil_div((int64_t)maxsteps * (max_sweeps + 2), period);
   for (int p = 0; rc_loop == TN_OK && p < nsets; ++p) {
     if (exec) {
       if (hipGraphLaunch(exec, st) != hipSuccess) {
