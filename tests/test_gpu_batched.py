@@ -119,3 +119,27 @@ def test_batched_truncate_low_rank(tn, sizes):
     for j, (Lm, Rm) in enumerate(jobs):
         check_job(Lm, Rm, U[j], S[j], Vt[j], int(kept[j]), 1e-8, 0)
     assert sweeps.max() < 60
+
+
+# The preconditioning QR's row and column tiles: rows at the edges of a tile, of
+# a wave's rows and of a workgroup's (1024), odd column strides, last panels of
+# one and of a few columns.
+def test_batched_qr_tile_edges(tn):
+    from tncontract_amd.batched import batched_svd
+    rng = np.random.default_rng(5)
+    mats = [rng.standard_normal(s) for s in
+            [(33, 33), (34, 50), (64, 64), (127, 40), (129, 47), (256, 80), (65, 1023),
+             (1024, 49), (1024, 128), (900, 250)]]
+    mats.append(np.zeros((70, 40)))
+    mats.append(rng.standard_normal((200, 5)) @ rng.standard_normal((5, 90)))
+    mats[2][:, 7] = 0.0
+    mats[4][10:, 3] = 0.0
+    U, S, Vt, sweeps = batched_svd([torch.from_numpy(a).cuda() for a in mats])
+    for a, u, s, vt in zip(mats, U, S, Vt):
+        u, s, vt = u.cpu().numpy(), s.cpu().numpy(), vt.cpu().numpy()
+        ref = np.linalg.svd(a, compute_uv=False)
+        assert np.abs(s - ref).max() <= 1e-13 * ref[0]
+        assert np.linalg.norm((u * s) @ vt - a) <= 4e-13 * ref[0] * np.sqrt(len(ref))
+        k = int(np.count_nonzero(ref > 1e-10 * ref[0]))
+        assert np.abs(u[:, :k].T @ u[:, :k] - np.eye(k)).max(initial=0.0) <= 4e-13
+        assert np.abs(vt[:k] @ vt[:k].T - np.eye(k)).max(initial=0.0) <= 4e-13

@@ -737,13 +737,13 @@ static double time_grouped(int FR, const std::vector<int>& ids, const std::vecto
 static bool qr_precond(int64_t L, int64_t k) { return k > BJ2 && L <= kQrRows; }
 
 // Work items of a preconditioned job with k columns: one panel item per
-// panel; trailing-update groups of 64 columns after each panel; Q-apply
-// groups of 64 of the (at most k) kept columns per panel.
+// panel; trailing-update groups of QNB columns after each panel; Q-apply
+// groups of QNB of the (at most k) kept columns per panel.
 static void qr_item_counts(int64_t k, size_t* npan, size_t* ntrail, size_t* napply) {
   const int64_t np = ceil_div(k, QNB);
   *npan += (size_t)np;
-  for (int64_t p = 0; p < np; ++p) *ntrail += (size_t)ceil_div(std::max<int64_t>(k - (p + 1) * QNB, 0), 64);
-  *napply += (size_t)(np * ceil_div(k, 64));
+  for (int64_t p = 0; p < np; ++p) *ntrail += (size_t)ceil_div(std::max<int64_t>(k - (p + 1) * QNB, 0), QNB);
+  *napply += (size_t)(np * np);
 }
 
 static size_t batched_ws_bytes(const std::vector<int64_t>& ms, const std::vector<int64_t>& ns) {
@@ -936,9 +936,9 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
       const int k = qj[i].k;
       if (p * QNB >= k) continue;
       pan_items.push_back(i);
-      const int ng = (int)ceil_div(std::max(k - (p + 1) * QNB, 0), 64);
+      const int ng = (int)ceil_div(std::max(k - (p + 1) * QNB, 0), QNB);
       for (int g = 0; g < ng; ++g) trail_items.push_back(QItem{i, g});
-      for (int g = 0; g < (int)ceil_div(k, 64); ++g) apply_items.push_back(QItem{i, g});
+      for (int g = 0; g < (int)ceil_div(k, QNB); ++g) apply_items.push_back(QItem{i, g});
     }
   }
   pan_off[maxpan] = pan_items.size();
@@ -1071,9 +1071,9 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     for (int p = 0; p < maxpan; ++p) {
       const unsigned np_ = (unsigned)(pan_off[p + 1] - pan_off[p]);
       const unsigned nt_ = (unsigned)(trail_off[p + 1] - trail_off[p]);
-      hipLaunchKernelGGL(bqr_panel, dim3(np_), dim3(256), 0, st, dWv, dTf, dqj, dpan + pan_off[p], p);
+      hipLaunchKernelGGL(bqr_panel, dim3(np_), dim3(64 * QPW), 0, st, dWv, dTf, dqj, dpan + pan_off[p], p);
       if (nt_)
-        hipLaunchKernelGGL(bqr_trail, dim3(nt_), dim3(256), 0, st, dWv, dTf, dqj,
+        hipLaunchKernelGGL(bqr_trail, dim3(nt_), dim3(QNT), 0, st, dWv, dTf, dqj,
                            dtrail + trail_off[p], p);
     }
     hipLaunchKernelGGL(bqr_rvec, dim3(64, (unsigned)npre), dim3(256), 0, st, dWv, dqj);
@@ -1206,7 +1206,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
                        dperm, dsbase, dkept);
     for (int p = maxpan - 1; p >= 0; --p) {
       const unsigned na_ = (unsigned)(apply_off[p + 1] - apply_off[p]);
-      hipLaunchKernelGGL(bqr_apply, dim3(na_), dim3(256), 0, st, dWv, dTf, dqj,
+      hipLaunchKernelGGL(bqr_apply, dim3(na_), dim3(QNT), 0, st, dWv, dTf, dqj,
                          dapply + apply_off[p], dkept, p, dQZ);
     }
   }

@@ -9,24 +9,35 @@
 //
 // Per panel of QNB = 16 columns (LAPACK dgeqrf's steps with dlarfg's
 // reflector convention, beta = -sign(alpha) ||x||, and dlarft's forward
-// column-wise T), every job's panel in the same two launches:
-//   * bqr_panel, one workgroup per job: the panel's rows are held in
-//     registers, 4 rows per thread (rows tid, tid + 256, ...), and each
-//     reflector costs one block reduction of 16 dot products (the update of
-//     the panel's other columns and the new column of T from the same dots);
-//   * bqr_trail, one workgroup per 64 trailing columns of a job: C -= V T^T
-//     V^T C by v_mfma_f64_16x16x4, each wave a 16-column tile, V read back
-//     from the stored panel through LDS.  Few registers, so many waves per
-//     CU hide the loads' latency.
+// column-wise T), every job's panel in the same two launches, by workgroups
+// that hold all rows below the panel's first one in registers, as 16 x 16
+// tiles in the fragment layout of v_mfma_f64_16x16x4 (column lane % 16; rows
+// 4 (lane / 16) + e, e = 0 .. 3: 32 contiguous bytes a lane):
+//   * bqr_panel, one workgroup per job, one barrier per reflector: a column
+//     reaches the others by DPP, and one exchange through LDS sums its dots
+//     with all 16 columns (its norm, the update of the later columns and the
+//     earlier reflectors' products that T is made of);
+//   * bqr_trail, one workgroup per 16 trailing columns of a job: C -= V T^T
+//     V^T C, C read once and written once.
+// What bounds both is latency: few workgroups run once the small jobs are
+// done, so the rows are spread over all waves of a workgroup (the panel's over
+// 8, whose reflectors' scalar work is repeated in every wave) and every load of
+// a tile is issued at once.  Averaged over the panels of 32 jobs of sizes up to
+// 1022, the trailing update takes 18.5 us, the application of Q 17.5 and the
+// panel 27.8; with 4 waves per 64 columns staging V through LDS 64 rows at a
+// time, and two barriered block sums per reflector, 79, 79 and 47.5.
 #pragma once
 #include "tn_common.h"
+#include "tn_jacobi.h"
 
 #include <utility>
 
 namespace tn {
 
 constexpr int QNB = 16;         // reflectors per panel (T is QNB x QNB)
-constexpr int kQrRows = 1024;   // rows a workgroup holds in registers (4 per thread)
+constexpr int kQrRows = 1024;   // rows a workgroup holds in registers (64 per wave)
+constexpr int QNW = kQrRows / 64;
+constexpr int QNT = 64 * QNW;
 
 typedef double f64x4q __attribute__((ext_vector_type(4)));
 
@@ -42,235 +53,300 @@ struct QJob {
   int32_t pad;
 };
 
-// v[0..N) summed over the block's 256 threads; every thread gets the sums
-// (bit-identical in all of them): each wave's values by DPP, the four waves'
-// partials one per lane from LDS, summed by two shuffles and read back by
-// readlane.
-template <int N>
-__device__ __forceinline__ void qr_block_sum(double (&v)[N], double (*red)[QNB]) {
-  static_assert(4 * N <= 64, "one partial per lane");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int c = 0; c < N; ++c) v[c] = wave_sum_dpp(v[c]);
-  if (lane == 0) {
-#pragma unroll
-    for (int c = 0; c < N; ++c) red[wave][c] = v[c];
-  }
-  __syncthreads();
-  double p = lane < 4 * N ? red[lane / N][lane % N] : 0.0;
-#pragma unroll
-  for (int sh = N; sh < 4 * N; sh <<= 1) p += __shfl_xor(p, sh, 64);
-  const long long u = __double_as_longlong(p);
-#pragma unroll
-  for (int c = 0; c < N; ++c) {
-    const int lo = __builtin_amdgcn_readlane((int)u, c);
-    const int hi = __builtin_amdgcn_readlane((int)(u >> 32), c);
-    v[c] = __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-  }
-  __syncthreads();
+// A pair of neighbouring doubles, 8-byte aligned (odd column strides).
+typedef double f64x2q __attribute__((ext_vector_type(2), aligned(8)));
+
+// Value of lane LANE of this lane's row of 16 (DPP row_newbcast).
+template <int LANE>
+__device__ __forceinline__ double dpp_row_bcast(double v) {
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(
+      0ll, __double_as_longlong(v), 0x150 + LANE, 0xf, 0xf, true));
 }
 
-// C[p0:L, c0:c1) -= V op(T) V^T C[p0:L, c0:c1) for c1 - c0 <= 64 (column-
-// major C, ld = ldc; called by the whole block: wave w takes the 16-column
-// tile at c0 + 16 w), V the nb reflectors of the panel at column p0 of X
-// (ld = L; unit diagonal, zero above it), op(T) = T^T if trans (applying
-// Q^T) else T.  V is staged through LDS (Vs) 64 rows at a time with
-// coalesced loads shared by the four waves; each wave's C loads of a chunk
-// are issued together.  MFMA operand layouts (16x16x4 f64): A[m][k] in lane
-// m + 16 k, B[k][n] in lane n + 16 k, D[k + 4 e][n] in element e of lane
-// n + 16 k.
+// Sum over the four lanes lane % 16 + 16 k (the same bits in all four):
+// swapping the odd rows of 16 (then the upper half) of one copy with the even
+// rows (lower half) of another leaves the two values to add in every lane.
+__device__ __forceinline__ double column_sum(double v) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  long long u = __double_as_longlong(v);
+  u2 lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
+  u2 hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+  v = __longlong_as_double(((long long)hi[0] << 32) | lo[0]) +
+      __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+  u = __double_as_longlong(v);
+  lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+  hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+  return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) +
+         __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+
+// C[p0:L, c0:c1) -= V op(T) V^T C[p0:L, c0:c1) for c1 - c0 <= 16 (column-
+// major C, ld = ldc; called by the whole workgroup of 16 waves), V the nb
+// reflectors of the panel at column p0 of X (ld = L; unit diagonal, zero above
+// it), op(T) = T^T if trans (applying Q^T) else T.  A[m][k] of the MFMA is in
+// lane m + 16 k, B[k][n] in lane n + 16 k, D[k + 4 e][n] in element e of lane
+// n + 16 k; the update's A rows are permuted so that D's rows are C's.
 __device__ __forceinline__ void qr_block_reflect(const double* __restrict__ X, int L, int p0,
                                                  int nb, const double (*Ts)[QNB + 1], bool trans,
                                                  double* __restrict__ C, int64_t ldc, int c0,
-                                                 int c1, double (*Vs)[QNB + 1]) {
+                                                 int c1, double (*part)[256]) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int lr = lane & 15, lk = lane >> 4;
-  const int cc = c0 + 16 * wave + lr;
-  const bool cok = cc < c1;
-  double* Cc = C + (int64_t)(cok ? cc : c0) * ldc;
-  // V rows r0 .. r0 + 63 into Vs (zero past L, above the diagonal and past nb)
-  auto stage = [&](int r0) {
-    __syncthreads();
+  const int R0 = p0 + 64 * wave, rb = R0 + 4 * lk;
+  const bool act = R0 < L;
+  const bool cok = c0 + lr < c1;
+  double* Cc = C + (int64_t)(cok ? c0 + lr : c0) * ldc;
+  // every row of the wave's exists, below the panel's triangle, for 16
+  // columns and reflectors: no bounds test
+  const bool full = wave > 0 && R0 + 64 <= L && c1 - c0 == 16 && nb == QNB;
+  double c[4][4], w[4][4];
+  f64x4q y = {0.0, 0.0, 0.0, 0.0}, y1 = {0.0, 0.0, 0.0, 0.0};
+  if (act) {
+    double v[4][4];
+    const double* Vc = X + (int64_t)(p0 + min(lr, nb - 1)) * L;
+    if (full) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+          const f64x2q a = *(const f64x2q*)(Vc + rb + 16 * t + e);
+          const f64x2q b = *(const f64x2q*)(Cc + rb + 16 * t + e);
+          v[t][e] = a[0];
+          v[t][e + 1] = a[1];
+          c[t][e] = b[0];
+          c[t][e + 1] = b[1];
+        }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = rb + 16 * t + e, d = row - p0 - lr;
+          v[t][e] = (lr < nb && row < L && d >= 0) ? (d == 0 ? 1.0 : Vc[row]) : 0.0;
+          c[t][e] = (cok && row < L) ? Cc[row] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        y = __builtin_amdgcn_mfma_f64_16x16x4f64(v[t][e], c[t][e], y, 0, 0, 0);
+        y1 = __builtin_amdgcn_mfma_f64_16x16x4f64(v[t][e + 1], c[t][e + 1], y1, 0, 0, 0);
+      }
+    // V again, as the update's operand: row R0 + 16 t + 4 (lr % 4) + lr / 4 of
+    // reflector lk + 4 u (in flight across the reduction)
+    const int r2 = R0 + 4 * (lr & 3) + (lr >> 2);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int e = tid + 256 * u, i = e & 63, c = e >> 6, row = r0 + i, dr = p0 + c;
-      double v = 0.0;
-      if (c < nb && row < L && row >= dr) v = row == dr ? 1.0 : X[(int64_t)dr * L + row];
-      Vs[i][c] = v;
-    }
-    __syncthreads();
-  };
-  // Y = V^T C_tile (16 x 16), summed over the rows p0 .. L-1
-  f64x4q y = {0.0, 0.0, 0.0, 0.0};
-  for (int r0 = p0; r0 < L; r0 += 64) {
-    stage(r0);
-    double b[16];
+      const int q = lk + 4 * u;
+      const double* Vq = X + (int64_t)(p0 + min(q, nb - 1)) * L;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = r0 + 4 * i + lk;
-      b[i] = (cok && row < L) ? Cc[row] : 0.0;
+      for (int t = 0; t < 4; ++t) {
+        const int row = r2 + 16 * t, d = row - p0 - q;
+        if (full)
+          w[t][u] = Vq[row];
+        else
+          w[t][u] = (q < nb && row < L && d >= 0) ? (d == 0 ? 1.0 : Vq[row]) : 0.0;
+      }
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      y = __builtin_amdgcn_mfma_f64_16x16x4f64(Vs[4 * i + lk][lr], b[i], y, 0, 0, 0);
+    for (int e = 0; e < 4; ++e) part[wave][64 * e + lane] = y[e] + y1[e];
   }
+  lds_barrier();
+  // Y summed over the waves: four threads an element, four partials each
+  {
+    const int q = tid & 255, g = tid >> 8, nw = min((L - p0 + 63) >> 6, QNW);
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * g + i < nw) s += part[4 * g + i][q];
+    lds_barrier();
+    part[g][q] = s;
+  }
+  lds_barrier();
+  if (!act) return;
   // Y2 = op(T) Y: element u of y holds Y[lk + 4u][lr], the B operand of
   // the k-step whose summation indices are lk + 4u
   f64x4q y2 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const int kk = lk + 4 * u;
+    const int kk = lk + 4 * u, q = 64 * u + lane;
+    const double yu = (part[0][q] + part[1][q]) + (part[2][q] + part[3][q]);
     const double a = trans ? Ts[kk][lr] : Ts[lr][kk];
-    y2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, y[u], y2, 0, 0, 0);
+    y2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, yu, y2, 0, 0, 0);
   }
-  // C_tile -= V Y2, 16 rows at a time
-  for (int r0 = p0; r0 < L; r0 += 64) {
-    stage(r0);
 #pragma unroll
-    for (int s16 = 0; s16 < 4; ++s16) {
-      const int R0 = r0 + 16 * s16;
-      f64x4q d = {0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < 4; ++t) {
+    f64x4q d = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        d = __builtin_amdgcn_mfma_f64_16x16x4f64(Vs[16 * s16 + lr][lk + 4 * u], y2[u], d, 0, 0, 0);
-      if (cok) {
+    for (int u = 0; u < 4; ++u)
+      d = __builtin_amdgcn_mfma_f64_16x16x4f64(w[t][u], y2[u], d, 0, 0, 0);
+    if (full) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = R0 + lk + 4 * e;
-          if (row < L) Cc[row] -= d[e];
-        }
-      }
+      for (int e = 0; e < 4; e += 2)
+        *(f64x2q*)(Cc + rb + 16 * t + e) = f64x2q{c[t][e] - d[e], c[t][e + 1] - d[e + 1]};
+    } else if (cok) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (rb + 16 * t + e < L) Cc[rb + 16 * t + e] = c[t][e] - d[e];
     }
   }
 }
 
-// Reflector JJ of the panel at column p0 (nb columns; JJ a compile-time
-// index, so that the panel stays in registers): forms it from column JJ,
-// applies it to the panel's later columns and adds column JJ of T.
+constexpr int QPW = 8;                        // waves of bqr_panel
+constexpr int QPT = kQrRows / (16 * QPW);     // 16-row tiles a wave holds
+
+struct QPanelLds {
+  double part[2][QPW][QNB];   // the waves' dots of a column with all 16
+  double row[2][QNB];         // the panel's row at the pivot
+  double dots[QNB][QNB];      // [JJ][c] = v_JJ . (column c): T's inner products for c < JJ
+  double tau[QNB];
+};
+
+// Reflector JJ of the panel (nb columns; JJ a compile-time index: the lane a
+// column is broadcast from): formed from column JJ, applied to the later
+// columns.  P[t][e]: the lane's rows of column lane % 16, nt tiles of which
+// exist.  x . P_c below the pivot comes from one exchange for every column c,
+// and the reflector v = (1; scal x) gives v . P_c = P[JJ][c] + scal x . P_c.
+// Columns keep x; myscal is the scal of this lane's column once it is a
+// reflector, 1 before.
 template <int JJ>
-__device__ __forceinline__ void qr_panel_step(double (&P)[4][QNB], int p0, int nb,
-                                              double (*red)[QNB], double (*Ts)[QNB + 1]) {
+__device__ __forceinline__ void qr_panel_step(double (&P)[QPT][4], int nt, int nb, QPanelLds& sm,
+                                              double& myscal) {
   if (JJ >= nb) return;  // block-uniform
-  const int tid = threadIdx.x, col = p0 + JJ;
-  double sa[2] = {0.0, 0.0};  // squared norm below the diagonal, alpha
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  double x[QPT][4], acc[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = tid + 256 * q;
-    if (r > col) sa[0] = fma(P[q][JJ], P[q][JJ], sa[0]);
-    if (r == col) sa[1] = P[q][JJ];
+  for (int t = 0; t < QPT; ++t) {
+    if (t >= nt) break;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[t][e] = dpp_row_bcast<JJ>(P[t][e]);
+    if (t == 0 && wave == 0) {
+      // the panel's triangle: rows 4 lk + e <= JJ of the first tile
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (4 * lk + e <= JJ) x[0][e] = 0.0;
+      if (lk == JJ / 4) sm.row[JJ & 1][lr] = P[0][JJ & 3] * myscal;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = fma(x[t][e], P[t][e], acc[e]);
   }
-  qr_block_sum<2>(sa, red);
-  const double s = sa[0], alpha = sa[1];
+  const double a = column_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+  if (lk == 0) sm.part[JJ & 1][wave][lr] = a;
+  lds_barrier();
+  double d = column_sum(sm.part[JJ & 1][2 * lk][lr] + sm.part[JJ & 1][2 * lk + 1][lr]);
+  const double prow = sm.row[JJ & 1][lr];
+  const double s = dpp_row_bcast<JJ>(d), alpha = dpp_row_bcast<JJ>(prow);
   double beta = alpha, tau = 0.0, scal = 1.0;
   if (s != 0.0) {
     beta = -copysign(sqrt(fma(alpha, alpha, s)), alpha);
     tau = (beta - alpha) / beta;
     scal = 1.0 / (alpha - beta);
   }
-  double v[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = tid + 256 * q;
-    v[q] = r > col ? P[q][JJ] * scal : (r == col ? 1.0 : 0.0);
-    if (r > col) P[q][JJ] = v[q];
+  const double vp = fma(scal * myscal, d, prow);  // v . (column c, or reflector c)
+  if (wave == 0 && lk == 0) {
+    sm.dots[JJ][lr] = vp;
+    sm.tau[JJ] = tau;
   }
-  // d_c = v^T P[:, c]: for c > JJ the update of column c, for c < JJ (the
-  // reflectors already formed) the new column of T
-  double d[QNB];
+  const double f = lr > JJ ? -tau * vp : 0.0, g = f * scal;
 #pragma unroll
-  for (int c = 0; c < QNB; ++c) {
-    double acc = 0.0;
+  for (int t = 0; t < QPT; ++t) {
+    if (t >= nt) break;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc = fma(v[q], P[q][c], acc);
-    d[c] = acc;
+    for (int e = 0; e < 4; ++e) P[t][e] = fma(g, x[t][e], P[t][e]);
   }
-  qr_block_sum<QNB>(d, red);
-#pragma unroll
-  for (int c = JJ + 1; c < QNB; ++c) {
-    const double f = -tau * d[c];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) P[q][c] = fma(f, v[q], P[q][c]);
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    if (tid + 256 * q == col) P[q][JJ] = beta;
-  // T[0:JJ, JJ] = -tau T[0:JJ, 0:JJ] d[0:JJ], T[JJ][JJ] = tau: thread i owns
-  // row i of T (its earlier entries are its own writes)
-  if (tid < JJ) {
-    double t = 0.0;
-#pragma unroll
-    for (int l = 0; l < JJ; ++l) t = fma(Ts[tid][l], d[l], t);
-    Ts[tid][JJ] = -tau * t;
-  }
-  if (tid == JJ) Ts[JJ][JJ] = tau;
+  if (lr == JJ) myscal = scal;
+  if (wave == 0 && lk == JJ / 4) P[0][JJ & 3] = lr == JJ ? beta : P[0][JJ & 3] + f;
 }
 
 template <int... J>
-__device__ __forceinline__ void qr_panel(std::integer_sequence<int, J...>, double (&P)[4][QNB],
-                                         int p0, int nb, double (*red)[QNB],
-                                         double (*Ts)[QNB + 1]) {
-  (qr_panel_step<J>(P, p0, nb, red, Ts), ...);
+__device__ __forceinline__ void qr_panel(std::integer_sequence<int, J...>, double (&P)[QPT][4],
+                                         int nt, int nb, QPanelLds& sm, double& myscal) {
+  (qr_panel_step<J>(P, nt, nb, sm, myscal), ...);
+}
+
+// T of the panel's nb reflectors (zero past them), row-major at out, by wave 0
+// (lane i: row i): T[0:j, j] = -tau_j T[0:j, 0:j] (V^T v_j)[0:j], T[j][j] =
+// tau_j.
+__device__ __forceinline__ void qr_panel_t(const QPanelLds& sm, int nb, double* __restrict__ out) {
+  const int i = threadIdx.x & 15;
+  double T[QNB];
+#pragma unroll
+  for (int c = 0; c < QNB; ++c) T[c] = 0.0;
+#pragma unroll 1
+  for (int j = 0; j < nb; ++j) {
+    double t = 0.0;
+#pragma unroll
+    for (int c = 0; c < QNB; ++c) t = fma(T[c], c < j ? sm.dots[j][c] : 0.0, t);
+    const double tau = sm.tau[j], v = i < j ? -tau * t : (i == j ? tau : 0.0);
+#pragma unroll
+    for (int c = 0; c < QNB; ++c) T[c] = c == j ? v : T[c];
+  }
+  if (threadIdx.x < 16) {
+#pragma unroll
+    for (int c = 0; c < QNB; ++c) out[i * QNB + c] = T[c];
+  }
 }
 
 // Panel p of every job (one workgroup per job that has it; items: the
 // indices into qjobs): the panel's QNB columns factored in registers, the
 // reflectors and R's entries stored back, T into Tf.
-__global__ void __launch_bounds__(256) bqr_panel(double* __restrict__ Wv, double* __restrict__ Tf,
-                                                 const QJob* __restrict__ qjobs,
-                                                 const int* __restrict__ items, int p) {
-  __shared__ double red[4][QNB];
-  __shared__ double Ts[QNB][QNB + 1];
+__global__ void __launch_bounds__(64 * QPW) bqr_panel(double* __restrict__ Wv,
+                                                      double* __restrict__ Tf,
+                                                      const QJob* __restrict__ qjobs,
+                                                      const int* __restrict__ items, int p) {
+  __shared__ QPanelLds sm;
   const QJob Q = qjobs[items[blockIdx.x]];
-  double* X = Wv + Q.x;
-  const int L = Q.L, k = Q.k, tid = threadIdx.x;
-  const int p0 = p * QNB, nb = min(QNB, k - p0);
-  double P[4][QNB];
+  const int L = Q.L, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15;
+  const int p0 = p * QNB, nb = min(QNB, Q.k - p0), nt = (L - p0 + 16 * QPW - 1) / (16 * QPW);
+  double* Xc = Wv + Q.x + (int64_t)(p0 + min(lr, nb - 1)) * L;
+  const int rb = p0 + 16 * wave + 4 * (lane >> 4);  // tile t: 16 QPW t rows on
+  double P[QPT][4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = tid + 256 * q;
+  for (int t = 0; t < QPT; ++t)
 #pragma unroll
-    for (int c = 0; c < QNB; ++c)
-      P[q][c] = (r >= p0 && r < L && c < nb) ? X[(int64_t)(p0 + c) * L + r] : 0.0;
-  }
-  Ts[tid >> 4][tid & 15] = 0.0;
-  // (the first reduction's barriers order the zeroing before any T write)
-  qr_panel(std::make_integer_sequence<int, QNB>{}, P, p0, nb, red, Ts);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = tid + 256 * q;
-    if (r >= p0 && r < L) {
-#pragma unroll
-      for (int c = 0; c < QNB; ++c)
-        if (c < nb) X[(int64_t)(p0 + c) * L + r] = P[q][c];
+    for (int e = 0; e < 4; ++e) {
+      const int row = rb + 16 * QPW * t + e;
+      P[t][e] = (row < L && lr < nb) ? Xc[row] : 0.0;
     }
+  double myscal = 1.0;
+  qr_panel(std::make_integer_sequence<int, QNB>{}, P, nt, nb, sm, myscal);
+  if (lr < nb) {
+#pragma unroll
+    for (int t = 0; t < QPT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = rb + 16 * QPW * t + e;
+        if (row < L) Xc[row] = row > p0 + lr ? P[t][e] * myscal : P[t][e];
+      }
   }
-  __syncthreads();
-  Tf[Q.tf + (int64_t)p * (QNB * QNB) + tid] = Ts[tid >> 4][tid & 15];
+  // (dots and tau are wave 0's own writes)
+  if (tid < 64) qr_panel_t(sm, nb, Tf + Q.tf + (int64_t)p * (QNB * QNB));
 }
 
-// Columns of a job in groups of 64 (one workgroup, a 16-column tile per
-// wave): item = (index into qjobs, group).
+// Columns of a job in groups of 16 (one workgroup): item = (index into qjobs,
+// group).
 struct QItem {
   int32_t q, g;
 };
 
 // Trailing update after panel p: the group's columns (after the panel) of
 // X get C -= V T^T V^T C.
-__global__ void __launch_bounds__(256) bqr_trail(double* __restrict__ Wv,
+__global__ void __launch_bounds__(QNT) bqr_trail(double* __restrict__ Wv,
                                                  const double* __restrict__ Tf,
                                                  const QJob* __restrict__ qjobs,
                                                  const QItem* __restrict__ items, int p) {
   __shared__ double Ts[QNB][QNB + 1];
-  __shared__ double Vs[64][QNB + 1];
+  __shared__ double part[QNW][256];
   const QItem it = items[blockIdx.x];
   const QJob Q = qjobs[it.q];
   const int tid = threadIdx.x;
   const int p0 = p * QNB, nb = min(QNB, Q.k - p0);
-  const int c0 = p0 + nb + 64 * it.g, c1 = min(Q.k, c0 + 64);
-  Ts[tid >> 4][tid & 15] = Tf[Q.tf + (int64_t)p * (QNB * QNB) + tid];
-  // (the first staging barrier orders Ts before its use)
+  const int c0 = p0 + nb + QNB * it.g, c1 = min(Q.k, c0 + QNB);
+  // (the reduction's barriers order Ts before its use)
+  if (tid < QNB * QNB) Ts[tid >> 4][tid & 15] = Tf[Q.tf + (int64_t)p * (QNB * QNB) + tid];
   double* X = Wv + Q.x;
-  qr_block_reflect(X, Q.L, p0, nb, Ts, true, X, Q.L, c0, c1, Vs);
+  qr_block_reflect(X, Q.L, p0, nb, Ts, true, X, Q.L, c0, c1, part);
 }
 
 // The rows of R as vectors: Rv[c * k + i] = R[c][i] (i >= c), 0 below.
@@ -305,23 +381,23 @@ __global__ void __launch_bounds__(256) bqr_qz_init(double* __restrict__ QZ,
 
 // Panel p's block reflector applied to the group's columns of Q Z (panels in
 // reverse order make Q [Z; 0]); groups at or past the job's ncols exit.
-__global__ void __launch_bounds__(256) bqr_apply(const double* __restrict__ Wv,
+__global__ void __launch_bounds__(QNT) bqr_apply(const double* __restrict__ Wv,
                                                  const double* __restrict__ Tf,
                                                  const QJob* __restrict__ qjobs,
                                                  const QItem* __restrict__ items,
                                                  const int* __restrict__ ncols, int p,
                                                  double* __restrict__ QZ) {
   __shared__ double Ts[QNB][QNB + 1];
-  __shared__ double Vs[64][QNB + 1];
+  __shared__ double part[QNW][256];
   const QItem it = items[blockIdx.x];
   const QJob Q = qjobs[it.q];
   const int nc = ncols[Q.job];
-  const int c0 = 64 * it.g, c1 = min(nc, c0 + 64);
+  const int c0 = QNB * it.g, c1 = min(nc, c0 + QNB);
   if (c0 >= c1) return;  // block-uniform
   const int tid = threadIdx.x;
   const int p0 = p * QNB, nb = min(QNB, Q.k - p0);
-  Ts[tid >> 4][tid & 15] = Tf[Q.tf + (int64_t)p * (QNB * QNB) + tid];
-  qr_block_reflect(Wv + Q.x, Q.L, p0, nb, Ts, false, QZ + Q.qz, Q.L, c0, c1, Vs);
+  if (tid < QNB * QNB) Ts[tid >> 4][tid & 15] = Tf[Q.tf + (int64_t)p * (QNB * QNB) + tid];
+  qr_block_reflect(Wv + Q.x, Q.L, p0, nb, Ts, false, QZ + Q.qz, Q.L, c0, c1, part);
 }
 
 }  // namespace tn
