@@ -363,3 +363,25 @@ def test_jacobi_inner_pairs_every_fourth_step(L, n, case):
     assert np.linalg.norm((w * lam) @ w.T - K) <= 4e-13 * ref[0] ** 2 * np.sqrt(n)
     big = int(np.count_nonzero(ref > 1e-5 * ref[0]))
     assert np.abs(w[:, :big].T @ w[:, :big] - np.eye(big)).max() <= 4e-13
+
+
+# One-launch Jacobi steps (vectors of length at most 256), from the first size
+# past one pair of blocks to the last: odd lengths, a last block of one vector,
+# zero vectors (pairs that are copied); bounds as above.
+@pytest.mark.parametrize("n", [33, 47, 129, 255, 256])
+def test_jacobi_one_launch_steps(L, n):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n))
+    a[:, n // 2:n // 2 + 16] = 0.0
+    ref = np.linalg.svd(a, compute_uv=False)
+    for m in (a, a.T):
+        u, s, vt = (x.cpu().numpy() for x in T._svd_device(dev(m.copy()), 1))
+        assert np.abs(s - ref).max() <= 2e-13 * ref[0]
+        assert np.linalg.norm((u * s) @ vt - m) <= 4e-13 * ref[0] * np.sqrt(n)
+        k = n - 16
+        assert np.abs(u[:, :k].T @ u[:, :k] - np.eye(k)).max() <= 4e-13
+        assert np.abs(vt[:k] @ vt[:k].T - np.eye(k)).max() <= 4e-13
+    K = a.T @ a
+    w, lam = (x.cpu().numpy() for x in T._eigh_psd_device(dev(K), 1)[:2])
+    assert np.linalg.norm((w * lam) @ w.T - K) <= 4e-13 * ref[0] ** 2 * np.sqrt(n)

@@ -165,6 +165,7 @@ __global__ void __launch_bounds__(256) gemm_grouped(const GJob* __restrict__ job
 // ---------------------------------------------------------------- batched Jacobi
 constexpr int BJB = 16, BJ2 = 32, BCH = 256;
 constexpr int BANT = 2, BACH = 64 * BANT;   // row tiles per wave / rows per chunk of bjac_apply
+static_assert(BCH <= kPairLen, "a row chunk fits the one-launch step's Gram");
 static_assert(BJB == JB && BJ2 == J2, "batched pairs use the shared pair layout");
 
 struct BJob {
@@ -219,43 +220,39 @@ __device__ __forceinline__ void bstate_next(const BJob& J, int j, BState cur, in
 }
 
 // acc += the 32 x 32 Gram of the pair's vectors (blocks I and K2 of the
-// job's k vectors of length L at W) over rows [r0, r1): tiles of 64 NG rows
-// staged through LDS, v_mfma_f64_16x16x4 by 4 NG waves (wave w takes the
-// 16 x 16 quarter w % 4 over the tile's rows 64 (w / 4) ..; the NG partial
-// sums are the caller's to add); the next tile's loads are issued into
-// registers before the current tile's MFMAs, so their latency overlaps the
-// MFMAs.
-template <int NG>
+// job's k vectors of length L at W) over rows [r0, r1): tiles of 64 rows
+// staged through LDS, v_mfma_f64_16x16x4 by 4 waves (wave w takes the 16 x 16
+// quarter w); the next tile's loads are issued into registers before the
+// current tile's MFMAs, so their latency overlaps the MFMAs.
 __device__ __forceinline__ void bgram_rows(const double* __restrict__ W, int64_t L, int k, int I,
                                            int K2, int64_t r0, int64_t r1,
                                            double (*Ps)[BJ2 + 1], f64x4b& acc) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ti = (wave >> 1) & 1, tj = wave & 1, kb = 64 * (wave >> 2);
-  constexpr int TR = 64 * NG;
-  constexpr int PE = TR * BJ2 / (256 * NG);
+  const int ti = wave >> 1, tj = wave & 1;
+  constexpr int PE = 64 * BJ2 / 256;
   double pv[PE];
   auto fetch = [&](int64_t rb) {
 #pragma unroll
     for (int i = 0; i < PE; ++i) {
-      const int e = tid + 256 * NG * i, row = e % TR, col = e / TR;
+      const int e = tid + 256 * i, row = e % 64, col = e / 64;
       const int64_t v = col < BJB ? (int64_t)I * BJB + col : (int64_t)K2 * BJB + (col - BJB);
       const int64_t r = rb + row;
       pv[i] = (v < k && r < r1) ? W[v * L + r] : 0.0;
     }
   };
   if (r0 < r1) fetch(r0);
-  for (int64_t rb = r0; rb < r1; rb += TR) {
+  for (int64_t rb = r0; rb < r1; rb += 64) {
 #pragma unroll
     for (int i = 0; i < PE; ++i) {
-      const int e = tid + 256 * NG * i;
-      Ps[e % TR][e / TR] = pv[i];
+      const int e = tid + 256 * i;
+      Ps[e % 64][e / 64] = pv[i];
     }
     __syncthreads();
-    if (rb + TR < r1) fetch(rb + TR);
+    if (rb + 64 < r1) fetch(rb + 64);
 #pragma unroll
     for (int k0 = 0; k0 < 64; k0 += 4) {
-      double a = Ps[kb + k0 + (lane >> 4)][16 * ti + (lane & 15)];
-      double b = Ps[kb + k0 + (lane >> 4)][16 * tj + (lane & 15)];
+      double a = Ps[k0 + (lane >> 4)][16 * ti + (lane & 15)];
+      double b = Ps[k0 + (lane >> 4)][16 * tj + (lane & 15)];
       acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
     }
     __syncthreads();
@@ -287,7 +284,7 @@ __global__ void __launch_bounds__(256) bjac_gram(double* __restrict__ Wv, const 
   if (work && tid == 0) atomicAdd(work, (unsigned long long)(r1 - r0));
   const double* base = Wv + J.wv;
   f64x4b acc = {0, 0, 0, 0};
-  bgram_rows<1>(base, J.L, J.k, I, K2, r0, r1, Ps, acc);
+  bgram_rows(base, J.L, J.k, I, K2, r0, r1, Ps, acc);
   double* out = Gpart + (int64_t)item * (BJ2 * BJ2);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -431,7 +428,7 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
                                                   const BState* __restrict__ state,
                                                   unsigned long long* __restrict__ offmax,
                                                   unsigned long long* __restrict__ work) {
-  __shared__ double Ps[128][BJ2 + 1];
+  __shared__ PairGramLds pg;
   __shared__ EigLds sm;
   const int item = blockIdx.x, tid = threadIdx.x;
   const int j = e_job[item];
@@ -440,29 +437,12 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
   if (2 * pi >= S.nb) return;
   const BJob J = jobs[j];
   const int I = brr(pi, S.s, S.nb), K2 = brr(S.nb - 1 - pi, S.s, S.nb);
-  const int wave = tid >> 6, lane = tid & 63;
-  const int ti = (wave >> 1) & 1, tj = wave & 1;
   double* W = Wv + J.wv;
   double* Z = Zb + J.z;
   double x[8][2], z[8][2];
   apply_rows_fetch<2, EIG_NW>(W, J.L, J.k, 0, J.L, I, K2, x);  // in flight during the Gram, rounds
   apply_rows_fetch<2, EIG_NW>(Z, J.k, J.k, 0, J.k, I, K2, z);
-  f64x4b acc = {0, 0, 0, 0};
-  bgram_rows<2>(W, J.L, J.k, I, K2, 0, J.L, Ps, acc);
-  // the two halves' partial sums: the second group's through G[1]
-  int gr[4], gc = eig_pos(16 * tj + (lane & 15));
-#pragma unroll
-  for (int e = 0; e < 4; ++e) gr[e] = eig_pos(16 * ti + (lane >> 4) + 4 * e);
-  if (wave >= 4) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sm.G[1][gr[e]][gc] = acc[e];
-  }
-  lds_barrier();
-  if (wave < 4) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sm.G[0][gr[e]][gc] = acc[e] + sm.G[1][gr[e]][gc];
-  }
-  lds_barrier();
+  pair_gram(sm, pg, W, J.L, J.k, I, K2);
   const bool inner = inner_step(S.s, S.nb);
   const double off = eig_off(sm, J.tol, J.neg2, inner);
   if (tid == 0) atomicMax(offmax + j, dbits(off));

@@ -17,7 +17,8 @@
 //                 applies [W_I W_J] <- [W_I W_J] Q (or [Z_I Z_J] Q) to its
 //                 row chunk by MFMA (grid: pairs x row chunks).
 // The two kernels of every step of a sweep are captured once as a HIP graph
-// and replayed.
+// and replayed.  Vectors of length at most 256 take one launch a step
+// (jac_step).
 // A sweep is nblk-1 steps; sweeps repeat until the largest normalised
 // off-diagonal of a whole sweep is <= tol.  Singular values are the vector
 // norms; they are sorted descending on the device.  At most 32 vectors of
@@ -182,6 +183,52 @@ __global__ void __launch_bounds__(EIG_NT) jac_eig_apply(double* __restrict__ Wv,
   if (off <= tol) return;
   eig_rotate(sm, tol, 0.0, inner);
   apply_rows_finish<NT, EIG_NW>(base, ld, nv, rs, re, I, J, x, sm.Q);
+}
+
+// A whole pair step in one launch, for vectors of length at most kPairLen:
+// every block of a pair (grid as jac_eig_apply's) forms the pair's Gram matrix
+// itself and rotates its own row chunk, of Win into Wout (the other blocks of
+// the pair still read Win) or of Z in place.  A pair that needs no rotation is
+// copied.  It saves the Gram launch (4.4 us and the gap to the next) and the
+// partials' trip through memory: 12.9 us a step, 254 x 636 SVD 3.09 -> 2.87 ms,
+// 64 x 64 eigensolve 618 -> 529 us.  Past 256 rows every block would repeat a
+// Gram as long as the launch it saves (512 rows: 3.4 us of MFMAs).
+__global__ void __launch_bounds__(EIG_NT) jac_step(const double* __restrict__ Win,
+                                                   double* __restrict__ Wout, int64_t L,
+                                                   double* __restrict__ Z, int64_t nv, int s,
+                                                   int nblk, int nchW, double tol,
+                                                   unsigned long long* __restrict__ offmax) {
+  constexpr int CH = 16 * EIG_NW;
+  __shared__ EigLds sm;
+  __shared__ PairGramLds pg;
+  const int pi = blockIdx.x, ch = blockIdx.y;
+  int I, J;
+  pair_blocks(pi, s, nblk, I, J);
+  const bool onW = ch < nchW;
+  const double* in = onW ? Win : Z;
+  double* out = onW ? Wout : Z;
+  const int64_t ld = onW ? L : nv, rs = (int64_t)(onW ? ch : ch - nchW) * CH;
+  const int64_t re = min(ld, rs + CH);
+  double x[8][1];
+  apply_rows_fetch<1, EIG_NW>(in, ld, nv, rs, re, I, J, x);
+  pair_gram(sm, pg, Win, L, nv, I, J);
+  const bool inner = inner_step(s, nblk);
+  const double off = eig_off(sm, tol, 0.0, inner);
+  if (ch == 0 && threadIdx.x == 0) atomicMax(offmax, dbits(off));
+  if (off <= tol) {
+    if (onW) {
+      const int lane = threadIdx.x & 63, lk = lane >> 4;
+      const int64_t r = rs + 16 * (threadIdx.x >> 6) + (lane & 15);
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) {
+        const int64_t v = pair_vec(4 * ks + lk, I, J);
+        if (v < nv && r < re) out[v * ld + r] = x[ks][0];
+      }
+    }
+    return;
+  }
+  eig_rotate(sm, tol, 0.0, inner);
+  apply_rows_finish<1, EIG_NW>(out, ld, nv, rs, re, I, J, x, sm.Q);
 }
 
 // At most 32 vectors of length at most kSmallLen (one block pair, so a sweep
@@ -658,7 +705,7 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   const int npairs = nblk / 2;
   // Z == nullptr: the rotations are not accumulated (eigensolver use)
   const int64_t kz0 = Z ? k : 0;
-  const int ent = eig_nt(npairs, L, kz0);
+  const int ent = eig_nt(npairs, L, kz0);  // (1 for the one-launch steps' sizes)
   const int nchW = (int)ceil_div(L, 128 * ent), nchZ = Z ? (int)ceil_div(k, 128 * ent) : 0;
   const int nchG = (int)ceil_div(L, GCH);
   const int64_t kz = Z ? k : 0;
@@ -672,6 +719,9 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   unsigned long long host_off = 0;
   // the sort's six launches per sweep pay off only where a sweep is long
   // (and graph-replayed): at least 16 steps, k >= 256
+  // (short vectors: the other buffer of the one-launch steps instead)
+  double* const W2 = nblk - 1 < 16 && L <= kPairLen ? sort_tmp : nullptr;
+  double *Wcur = Wv, *Wnext = W2;
   if (nblk - 1 < 16) sort_tmp = nullptr;
   auto enqueue_sweep = [&]() -> int {
     hipLaunchKernelGGL(reset_u64, dim3(1), dim3(1), 0, st, w.off);
@@ -688,6 +738,15 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
       }
     }
     for (int s = 0; s < nblk - 1; ++s) {
+      if (W2) {
+        ProfScope p(PROF_JAC_EIG, st,
+                    step_rounds(inner_step(s, nblk)) * 9216.0 * npairs + gram_fl + apply_fl,
+                    16.0 * (double)(L + kz) * J2 * npairs);
+        hipLaunchKernelGGL(jac_step, dim3(npairs, nchW + nchZ), dim3(EIG_NT), 0, st, Wcur, Wnext, L,
+                           Z, k, s, nblk, nchW, tol, w.off);
+        std::swap(Wcur, Wnext);
+        continue;
+      }
       {
         ProfScope p(PROF_JAC_GRAM, st, gram_fl, 8.0 * (double)L * J2 * npairs);
         hipLaunchKernelGGL(jac_gram, dim3(npairs, nchG), dim3(256), 0, st, Wv, L, k, s, nblk,
@@ -795,6 +854,11 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   if (exec) (void)hipGraphExecDestroy(exec);
   if (graph) (void)hipGraphDestroy(graph);
   if (rc_loop != TN_OK) return rc_loop;
+  if (Wcur != Wv) {
+    hipLaunchKernelGGL(copy_f64, dim3((unsigned)ceil_div(L * k, 256)), dim3(256), 0, st, Wcur, Wv,
+                       L * k);
+    TN_CHECK_LAUNCH();
+  }
   if (sweeps_out) *sweeps_out = sweep;
   return TN_OK;
 }
