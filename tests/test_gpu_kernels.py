@@ -385,3 +385,54 @@ def test_jacobi_one_launch_steps(L, n):
     K = a.T @ a
     w, lam = (x.cpu().numpy() for x in T._eigh_psd_device(dev(K), 1)[:2])
     assert np.linalg.norm((w * lam) @ w.T - K) <= 4e-13 * ref[0] ** 2 * np.sqrt(n)
+
+
+# QR by one workgroup (at most 64 columns and 256 rows): both variants' edges in
+# rows and columns, wide and tall, and the first sizes past them, FP64 and FP32
+# in, through transposed strides; R against LAPACK's (the same reflectors), the
+# bounds of a backward-stable factorisation.
+@pytest.mark.parametrize("m,n", [(1, 1), (1, 64), (64, 1), (2, 3), (15, 16), (16, 15), (17, 33),
+                                 (32, 32), (64, 32), (65, 32), (32, 64), (64, 64), (65, 33),
+                                 (256, 32), (255, 63), (256, 64), (257, 64), (256, 65)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_qr_in_one_workgroup(L, m, n, dtype):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(64 * m + n)
+    a = rng.standard_normal((m, n)).astype(dtype)
+    eps = 1e-13 if dtype == np.float64 else 2e-6
+    for d in (dev(a), dev(np.ascontiguousarray(a.T)).T):
+        q, r = (x.cpu().numpy().astype(np.float64) for x in T._qr_device(d, 1))
+        ref = np.linalg.qr(a.astype(np.float64))[1]
+        size = np.linalg.norm(a)
+        assert np.abs(np.tril(r, -1)).max(initial=0.0) == 0.0
+        assert np.linalg.norm(q @ r - a) <= eps * size
+        assert np.abs(q.T @ q - np.eye(min(m, n))).max() <= eps
+        # R's condition: well within 1e3 eps away from the square sizes
+        if abs(m - n) > 16:
+            assert np.abs(r - ref).max() <= 1e2 * eps * size
+    # zero columns: no reflector, the sign of the diagonal as LAPACK leaves it
+    a[:, n // 2] = 0.0
+    q, r = (x.cpu().numpy().astype(np.float64) for x in T._qr_device(dev(a), 1))
+    assert np.linalg.norm(q @ r - a) <= eps * max(np.linalg.norm(a), 1.0)
+    assert np.abs(q.T @ q - np.eye(min(m, n))).max() <= eps
+
+
+# Columns that earlier reflectors leave with rounding only (rows equal up to
+# rounding, 1e-16 smaller from column to column): their squares underflow, and
+# the reflectors stay orthogonal all the same.
+@pytest.mark.parametrize("scale", [1.0, 1e-150, 1e-300])
+@pytest.mark.parametrize("m,n", [(64, 32), (40, 64), (200, 64)])
+def test_small_qr_of_shrinking_columns(L, m, n, scale):
+    from tncontract_amd import tensor as T
+    from tncontract_amd.batched import batched_svd
+    rng = np.random.default_rng(m + n)
+    a = np.zeros((m, n))
+    a[-1] = rng.standard_normal(n) * scale
+    q, r = (x.cpu().numpy() for x in T._qr_device(dev(a), 1))
+    assert np.abs(q.T @ q - np.eye(min(m, n))).max() <= 1e-13
+    assert np.abs(q @ r - a).max() <= 1e-13 * scale
+    if scale == 1.0:
+        for u, s, vt in (T._svd_device(dev(a), 1), [x[0] for x in batched_svd([dev(a)])[:3]]):
+            u, s, vt = (x.cpu().numpy() for x in (u, s, vt))
+            assert abs(s[0] - np.linalg.norm(a)) <= 1e-13 * s[0]
+            assert np.abs((u * s) @ vt - a).max() <= 1e-13 * s[0]

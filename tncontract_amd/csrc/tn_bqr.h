@@ -28,6 +28,7 @@
 // time, and two barriered block sums per reflector, 79, 79 and 47.5.
 #pragma once
 #include "tn_common.h"
+#include "tn_hh16.h"
 #include "tn_jacobi.h"
 
 #include <utility>
@@ -236,14 +237,38 @@ __device__ __forceinline__ void qr_panel_step(double (&P)[QPT][4], int nt, int n
   lds_barrier();
   double d = column_sum(sm.part[JJ & 1][2 * lk][lr] + sm.part[JJ & 1][2 * lk + 1][lr]);
   const double prow = sm.row[JJ & 1][lr];
-  const double s = dpp_row_bcast<JJ>(d), alpha = dpp_row_bcast<JJ>(prow);
+  double s = dpp_row_bcast<JJ>(d), alpha = dpp_row_bcast<JJ>(prow), up = 1.0, down = 1.0;
+  if (hh_underflows(s, alpha)) {  // block-uniform
+    up = kHhUp;
+    down = 1.0 / kHhUpX;
+    alpha *= up;
+    double b = 0.0, c = 0.0;
+#pragma unroll
+    for (int t = 0; t < QPT; ++t) {
+      if (t >= nt) break;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[t][e] *= up;
+        b = fma(x[t][e], P[t][e] * kHhUpX, b);
+        c = fma(x[t][e], x[t][e], c);
+        if (lr == JJ && (t > 0 || wave > 0 || 4 * lk + e > JJ)) P[t][e] = x[t][e];
+      }
+    }
+    // (the pivot column's lane: the norm of the scaled column)
+    b = column_sum(lr == JJ ? c : b);
+    lds_barrier();
+    if (lk == 0) sm.part[JJ & 1][wave][lr] = b;
+    lds_barrier();
+    d = column_sum(sm.part[JJ & 1][2 * lk][lr] + sm.part[JJ & 1][2 * lk + 1][lr]);
+    s = dpp_row_bcast<JJ>(d);
+  }
   double beta = alpha, tau = 0.0, scal = 1.0;
   if (s != 0.0) {
     beta = -copysign(sqrt(fma(alpha, alpha, s)), alpha);
     tau = (beta - alpha) / beta;
     scal = 1.0 / (alpha - beta);
   }
-  const double vp = fma(scal * myscal, d, prow);  // v . (column c, or reflector c)
+  const double vp = fma(scal * myscal * down, d, prow);  // v . (column c, or reflector c)
   if (wave == 0 && lk == 0) {
     sm.dots[JJ][lr] = vp;
     sm.tau[JJ] = tau;
@@ -256,7 +281,7 @@ __device__ __forceinline__ void qr_panel_step(double (&P)[QPT][4], int nt, int n
     for (int e = 0; e < 4; ++e) P[t][e] = fma(g, x[t][e], P[t][e]);
   }
   if (lr == JJ) myscal = scal;
-  if (wave == 0 && lk == JJ / 4) P[0][JJ & 3] = lr == JJ ? beta : P[0][JJ & 3] + f;
+  if (wave == 0 && lk == JJ / 4) P[0][JJ & 3] = lr == JJ ? beta / up : P[0][JJ & 3] + f;
 }
 
 template <int... J>

@@ -94,11 +94,19 @@ __device__ __forceinline__ void pair_scaled(double gpq, double gpp, double gqq, 
 // Rotation predicate of a pair (l, h) from G_lh, G_ll, G_hh: G_lh^2 > tol^2
 // G_ll G_hh on the scaled entries, and one of the two vectors not negligible
 // (squared norm > neg2).  rot_coef_v rotates exactly the pairs for which it
-// holds, and the convergence measure eig_off counts exactly those.
+// holds, and the convergence measure eig_off counts exactly those.  A vector
+// whose squared norm underflows is not rotated with one 2^40 times longer: the
+// norm is lost and its product with the other is not, so the pair would be
+// rotated without end (the rounding that a sparse low-rank matrix leaves can
+// shrink by 1e-16 from vector to vector, down to there); nor is a pair whose
+// inner product is lost in its terms' underflow.
+constexpr double kNormMin = 0x1p-1018, kNormRatio = 0x1p-80, kDotMin = 0x1p-1060;
 __device__ __forceinline__ bool pair_rotates(double gpq, double gpp, double gqq, double tol,
                                              double neg2, double& spq, double& spp, double& sqq) {
   pair_scaled(gpq, gpp, gqq, spq, spp, sqq);
-  return spq * spq > tol * tol * fmax(spp * sqq, 0.0) && fmax(gpp, gqq) > neg2;
+  return spq * spq > tol * tol * fmax(spp * sqq, 0.0) && fmax(gpp, gqq) > neg2 &&
+         fabs(gpq) > kDotMin &&
+         (fmin(gpp, gqq) > kNormMin || fmin(spp, sqq) > kNormRatio);
 }
 
 // Convergence measure of the pair block: the largest |G_pq| / sqrt(G_pp G_qq)

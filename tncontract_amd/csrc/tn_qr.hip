@@ -10,8 +10,11 @@
 //  * the remaining columns of the 64-wide outer block are updated by a
 //    column-parallel kernel, and the trailing matrix by three MFMA GEMMs
 //    (Y = V^T A, Y = T^T Y, A -= V Y) with split-K for the first.
+// A matrix of at most 64 columns and 256 rows is factored, and its Q formed, by
+// one workgroup in one launch (qr_small).
 // Q is formed explicitly (orgqr order: blocks applied last to first to
 // [I; 0]).  Sign convention as LAPACK dlarfg: beta = -sign(alpha)*norm.
+#include "tn_hh16.h"
 #include "tn_internal.h"
 #include "tn_qr_hr.h"
 
@@ -827,6 +830,77 @@ size_t qr_workspace_bytes(int64_t m, int64_t n) { return qr_layout(m, n, nullptr
 
 using namespace tn;
 
+namespace tn {
+
+// The whole QR of an m x n matrix (m <= 16 NI, n <= NC) by one workgroup: read
+// through its modes, factored with a column per 16 lanes (tn_hh16.h), Q formed
+// from the reflectors in LDS, Q and R written row-major.  The launches, not
+// the work, were what a small QR took (64 x 32: some seventeen of 2 .. 19 us);
+// this is one, of 32 us, bound by the chain of its reflectors (20-site
+// compression with its 19 QRs of 64 x 32: 10.0 -> 8.0 ms).
+constexpr int kQrSmallCols = 64, kQrSmallRows = 256;
+
+template <typename T, int NC, int NI>
+__global__ void __launch_bounds__(16 * NC) qr_small(const T* __restrict__ A, Modes rows, Modes cols,
+                                                    int m, int n, T* __restrict__ Q,
+                                                    T* __restrict__ R) {
+  constexpr int LW = 16 * NI + 4;
+  __shared__ double W[NC][LW];
+  __shared__ double vcol[2][16 * NI], taus[NC];
+  __shared__ int64_t roff[16 * NI];
+  const int tid = threadIdx.x, q = tid >> 4, l = tid & 15, k = min(m, n), ni = (m + 15) >> 4;
+  for (int r = tid; r < m; r += 16 * NC) roff[r] = mode_offset32(rows, (uint32_t)r);
+  const int64_t co = mode_offset32(cols, (uint32_t)min(q, n - 1));
+  lds_barrier();
+  double x[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = l + 16 * i;
+    x[i] = (q < n && r < m) ? (double)A[roff[r] + co] : 0.0;
+  }
+  hh16_factor<NI, NC / 16>(x, q, l, k, ni, vcol, taus);
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+    if (i < ni) W[q][l + 16 * i] = x[i];
+#pragma unroll
+  for (int i = 0; i < NC / 16 && i < NI; ++i) {
+    const int r = l + 16 * i;
+    if (r < k && q < n) R[(int64_t)r * n + q] = (T)(r <= q ? x[i] : 0.0);
+  }
+  lds_barrier();
+  // column q of Q: reflectors past q leave e_q alone (4 columns a wave), unless
+  // one is not a number, which then reaches all of Q
+  const double tl = taus[min(tid & 63, k - 1)];
+  const int top = __any(tl != tl) ? k - 1 : min(k - 1, (tid >> 6) * 4 + 3);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) x[i] = l + 16 * i == q ? 1.0 : 0.0;
+  hh16_apply_q<NI>(x, l, top, ni, &W[0][0], LW, taus);
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+    if (i < ni) W[q][l + 16 * i] = x[i];
+  lds_barrier();
+  for (int e = tid; e < m * k; e += 16 * NC) Q[e] = (T)W[e % k][e / k];
+}
+
+template <typename T>
+static void launch_qr_small(const void* A, const Modes& rows, const Modes& cols, int m, int n,
+                            void* Q, void* R, hipStream_t st) {
+#define TN_QR_SMALL(NC, NI)                                                                    \
+  hipLaunchKernelGGL((qr_small<T, NC, NI>), dim3(1), dim3(16 * NC), 0, st, (const T*)A, rows, \
+                     cols, m, n, (T*)Q, (T*)R)
+  if (n <= 32) {
+    if (m <= 64) TN_QR_SMALL(32, 4);
+    else TN_QR_SMALL(32, 16);
+  } else {
+    if (m <= 64) TN_QR_SMALL(64, 4);
+    else TN_QR_SMALL(64, 16);
+  }
+#undef TN_QR_SMALL
+}
+
+}  // namespace tn
+
 extern "C" size_t tn_qr_workspace(int64_t m, int64_t n, int dtype) {
   (void)dtype;
   if (m <= 0 || n <= 0) return 256;
@@ -845,6 +919,14 @@ extern "C" int tn_qr(const void* A, const tn_modes* a_rows, const tn_modes* a_co
   TN_REQUIRE(A && Q && R, "tn_qr: null pointer");
   TN_REQUIRE(ws && ws_bytes >= tn_qr_workspace(m, n, dtype), "tn_qr: workspace too small");
   hipStream_t st = as_stream(stream);
+  if (n <= kQrSmallCols && m <= kQrSmallRows) {
+    if (dtype == TN_F64)
+      launch_qr_small<double>(A, rows, cols, (int)m, (int)n, Q, R, st);
+    else
+      launch_qr_small<float>(A, rows, cols, (int)m, (int)n, Q, R, st);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+  }
   QrWs w{};
   qr_layout(m, n, (char*)ws, ws_bytes, &w);
   unsigned gb = (unsigned)std::min<int64_t>(ceil_div(m * n, 256), 65536);

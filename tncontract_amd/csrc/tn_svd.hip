@@ -23,6 +23,7 @@
 // off-diagonal of a whole sweep is <= tol.  Singular values are the vector
 // norms; they are sorted descending on the device.  At most 32 vectors of
 // length at most 256 are done by one workgroup in one launch (jac_small).
+#include "tn_hh16.h"
 #include "tn_internal.h"
 #include "tn_jacobi.h"
 #include "tn_prof.h"
@@ -246,15 +247,6 @@ constexpr int kSmallLen = 256;
 // NaN ranks as -inf so that ranks stay a permutation of 0..k-1.
 __device__ __forceinline__ double rank_key(double x) { return x == x ? x : -INFINITY; }
 
-// Sum over the lane's row of 16.
-__device__ __forceinline__ double row16_sum(double v) {
-  v += dpp_f64<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f64<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f64<0x141, 0xF>(v);  // row_half_mirror
-  v += dpp_f64<0x140, 0xF>(v);  // row_mirror
-  return v;
-}
-
 template <bool QR>
 __global__ void __launch_bounds__(EIG_NT) jac_small(double* __restrict__ Wv, int L, int k,
                                                     double tol, int max_sweeps,
@@ -264,7 +256,7 @@ __global__ void __launch_bounds__(EIG_NT) jac_small(double* __restrict__ Wv, int
   constexpr int LW = kSmallLen + 4, LZ = J2 + 4, NI = kSmallLen / 16;
   __shared__ double W[J2][LW];
   __shared__ double Zs[QR ? J2 : 1][LZ], Rv[QR ? J2 : 1][LZ];
-  __shared__ double vcol[QR ? 2 : 1][QR ? kSmallLen : 1], nrm[J2], taus[J2];
+  __shared__ double vcol[QR ? 2 : 1][kSmallLen], nrm[J2], taus[J2];
   __shared__ EigLds sm;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
   const int q = tid >> 4, l = tid & 15;  // QR: this thread's column and first row (every 16th)
@@ -302,53 +294,7 @@ __global__ void __launch_bounds__(EIG_NT) jac_small(double* __restrict__ Wv, int
     lds_barrier();
 #pragma unroll
     for (int i = 0; i < NI; ++i) x[i] = i < ni ? W[q][l + 16 * i] : 0.0;
-    // Householder (dlarfg's convention), one barrier a column: column j goes
-    // to LDS, and every column sums its own dot below the pivot and the
-    // norm; v . x_q = x_q[j] + scale S_q
-    for (int j = 0; j < k; ++j) {
-      double* vc = vcol[j & 1];
-      if (q == j) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-          if (i < ni) vc[l + 16 * i] = x[i];
-      }
-      lds_barrier();
-      double v[NI], n2 = 0.0, dot = 0.0;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int r = l + 16 * i;
-        v[i] = (i < ni && r > j) ? vc[r] : 0.0;
-        n2 = fma(v[i], v[i], n2);
-        dot = fma(v[i], x[i], dot);
-      }
-      n2 = row16_sum(n2);
-      dot = row16_sum(dot);
-      const double alpha = vc[j];
-      // this column's pivot-row entry, held by lane j % 16 of its row
-      const double pv = __shfl(j < 16 ? x[0] : x[1], (lane & 48) | (j & 15), 64);
-      double tj = 0.0, scale = 0.0, beta = alpha;
-      if (n2 != 0.0) {  // NaN too: it has to reach R
-        const double h = sqrt(alpha * alpha + n2);
-        beta = alpha >= 0.0 ? -h : h;
-        tj = (beta - alpha) / beta;
-        scale = 1.0 / (alpha - beta);
-      }
-      if (q == j) {
-        if (l == 0) taus[j] = tj;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          const int r = l + 16 * i;
-          x[i] = r > j ? x[i] * scale : (r == j ? beta : x[i]);
-        }
-      } else if (q > j) {
-        const double w = tj * fma(scale, dot, pv), ws = w * scale;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          const int r = l + 16 * i;
-          x[i] = r == j ? x[i] - w : fma(-ws, v[i], x[i]);
-        }
-      }
-    }
+    hh16_factor<NI, 2>(x, q, l, k, ni, vcol, taus);
     // reflectors to W, the rows of R to Rv, Z = I
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -431,18 +377,7 @@ __global__ void __launch_bounds__(EIG_NT) jac_small(double* __restrict__ Wv, int
     double x[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) x[i] = i < 2 ? Zs[q][l + 16 * i] : 0.0;
-    for (int j = k - 1; j >= 0; --j) {
-      double v[NI], dot = 0.0;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int r = l + 16 * i;
-        v[i] = (i < ni && r > j) ? W[j][r] : (r == j ? 1.0 : 0.0);
-        dot = fma(v[i], x[i], dot);
-      }
-      const double w = taus[j] * row16_sum(dot);
-#pragma unroll
-      for (int i = 0; i < NI; ++i) x[i] = fma(-w, v[i], x[i]);
-    }
+    hh16_apply_q<NI>(x, l, k - 1, ni, &W[0][0], LW, taus);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int r = l + 16 * i;
