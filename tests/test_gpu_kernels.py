@@ -436,3 +436,32 @@ def test_small_qr_of_shrinking_columns(L, m, n, scale):
             u, s, vt = (x.cpu().numpy() for x in (u, s, vt))
             assert abs(s[0] - np.linalg.norm(a)) <= 1e-13 * s[0]
             assert np.abs((u * s) @ vt - a).max() <= 1e-13 * s[0]
+
+
+# Products of few 32 x 32 tiles (one workgroup each, K over its waves): tile
+# edges, K around a wave's eights and the last K taken, one and several modes,
+# every operand order.  Bound: K rounding errors of the absolute products.
+@pytest.mark.parametrize("m,n,k", [(33, 31, 300), (16, 1024, 17), (128, 130, 63), (64, 64, 64),
+                                   (95, 97, 65), (512, 511, 511), (256, 300, 512), (300, 256, 513),
+                                   (1000, 1024, 128), (5, 2000, 40)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_contract_few_tiles(L, m, n, k, dtype):
+    import tncontract_amd as tn
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k)).astype(dtype), rng.standard_normal((k, n)).astype(dtype)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    bound = k * np.finfo(dtype).eps * (np.abs(a).astype(np.float64) @ np.abs(b)) + 1e-300
+    for x, lx in ((a, ["m", "k"]), (a.T, ["k", "m"])):
+        for y, ly in ((b, ["k", "n"]), (b.T, ["n", "k"])):
+            z = tn.contract(tn.Tensor(dev(np.ascontiguousarray(x)), lx),
+                            tn.Tensor(dev(np.ascontiguousarray(y)), ly), "k", "k")
+            z.move_indices(["m", "n"], 0)
+            assert (np.abs(z.data.cpu().numpy() - ref) <= bound).all()
+    # both operands with two modes in every group that divides
+    if m % 4 == 0 and n % 4 == 0 and k % 4 == 0:
+        x = dev(np.ascontiguousarray(a.reshape(m // 4, 4, k // 4, 4).transpose(2, 0, 3, 1)))
+        y = dev(np.ascontiguousarray(b.reshape(k // 4, 4, n // 4, 4).transpose(1, 3, 0, 2)))
+        z = tn.contract(tn.Tensor(x, ["k0", "m0", "k1", "m1"]),
+                        tn.Tensor(y, ["k1", "n1", "k0", "n0"]), ["k0", "k1"], ["k0", "k1"])
+        z.move_indices(["m0", "m1", "n0", "n1"], 0)
+        assert (np.abs(z.data.cpu().numpy().reshape(m, n) - ref) <= bound).all()

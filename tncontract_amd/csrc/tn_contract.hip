@@ -1,6 +1,6 @@
 // Pairwise tensor contraction (np.tensordot in contract(), tensor.py:735).
 //
-// Two kernels:
+// Three kinds of kernels:
 //  * gemm_mfma<Prec>: C[m,n] = alpha*sum_k A[m,k]B[k,n] + beta*C, 128x128
 //    block tile, 4 waves (2x2) each owning a 64x64 tile of 16x16 MFMA
 //    fragments.  The row/col/k index of every operand is decoded through its
@@ -9,6 +9,8 @@
 //    Prec = FP64 (v_mfma_f64_16x16x4), FP32 (v_mfma_f32_16x16x4) or BF16X3
 //    (each FP32 operand split into hi+lo bf16, three v_mfma_f32_16x16x32_bf16
 //    per tile product: hi*hi + hi*lo + lo*hi, FP32 accumulation).
+//  * gemm_few_kernel: products of few 32 x 32 tiles, one workgroup each with K
+//    over its waves, fragments straight from memory.
 //  * contract_direct: one thread per output element, iterated in the
 //    output's memory order; used when K is small (e.g. the K = d = 2 MPO
 //    application), where the work is HBM-bound on the stores.  With 32-bit
@@ -289,6 +291,111 @@ __device__ __forceinline__ void xcd_tile(int& tx, int& ty) {
   const int in = id - r0 * nx;
   ty = r0 + in % h;
   tx = in / h;
+}
+
+// Products of few tiles: a workgroup per 32 x 32 tile of C, K split over its 8
+// waves.  Operands go from memory straight into MFMA fragments (the summation
+// index of a lane may be any k, as long as both operands agree: two neighbouring
+// ones a lane), any mode strides, the next 16 k in flight during the MFMAs of
+// the current ones; the waves' sums meet in LDS.  What bounds such a product is
+// the chain of launches, barriers and trips to memory, not its work: one launch,
+// one barrier and K / 128 trips, against LDS tiles of 128 x 128 (64 x 64), each
+// with a barrier per 16 k, and a second launch to sum a K split
+// (a call of 256 x 256 x 128, FP64: 22 -> 17 us, of which 12 are the host's).
+constexpr int GT = 32, GW = 8;
+
+template <typename T> struct Frag;
+template <> struct Frag<double> {
+  typedef double V __attribute__((ext_vector_type(4)));
+  static __device__ V mma(double a, double b, V c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ int row(int lk, int e) { return lk + 4 * e; }
+};
+template <> struct Frag<float> {
+  typedef float V __attribute__((ext_vector_type(4)));
+  static __device__ V mma(float a, float b, V c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ int row(int lk, int e) { return 4 * lk + e; }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(64 * GW) gemm_few_kernel(GemmArgs g) {
+  using V = typename Frag<T>::V;
+  __shared__ T red[GW][4][256];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  const int64_t m0 = (int64_t)blockIdx.y * GT, n0 = (int64_t)blockIdx.x * GT;
+  // rows and columns past the end read the last one; they are not stored
+  const T* ap[2];
+  const T* bp[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    ap[i] = (const T*)g.A + goff(g.am, min(m0 + 16 * i + lr, g.M - 1));
+    bp[i] = (const T*)g.B + goff(g.bn, min(n0 + 16 * i + lr, g.N - 1));
+  }
+  const int K = (int)g.K, kw = ((K + GW * 8 - 1) / (GW * 8)) * 8;  // k's of a wave, in eights
+  const int k0 = wave * kw, k1 = min(K, k0 + kw);
+  V acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = V{0, 0, 0, 0};
+  T a[2][4], b[2][4];
+  auto fetch = [&](int kb, T (&x)[2][4], T (&y)[2][4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k = kb + 8 * (s >> 1) + 2 * lk + (s & 1), kc = min(k, K - 1);
+      const int64_t oa = goff(g.ak, kc), ob = goff(g.bk, kc);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const T u = ap[i][oa], v = bp[i][ob];
+        x[i][s] = k < k1 ? u : (T)0;
+        y[i][s] = k < k1 ? v : (T)0;
+      }
+    }
+  };
+  if (k0 < k1) fetch(k0, a, b);
+  for (int kb = k0; kb < k1; kb += 16) {
+    T an[2][4], bn[2][4];
+    const bool more = kb + 16 < k1;
+    if (more) fetch(kb + 16, an, bn);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = Frag<T>::mma(a[i][s], b[j][s], acc[i][j]);
+    if (more) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          a[i][s] = an[i][s];
+          b[i][s] = bn[i][s];
+        }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[wave][t][64 * e + lane] = acc[t >> 1][t & 1][e];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int t = 2 * u + (tid >> 8), i = tid & 255;
+    T s = 0;
+#pragma unroll
+    for (int w = 0; w < GW; ++w) s += red[w][t][i];
+    const int64_t row = m0 + 16 * (t >> 1) + Frag<T>::row((i & 63) >> 4, i >> 6);
+    const int64_t col = n0 + 16 * (t & 1) + (i & 15);
+    if (row < g.M && col < g.N) {
+      T* c = (T*)g.C + goff(g.cm, row) + goff(g.cn, col);
+      T v = (T)g.alpha * s;
+      if (g.beta != 0.0) v += (T)g.beta * *c;
+      *c = v;
+    }
+  }
 }
 
 template <bool VEC, int AKF, int BNF>
@@ -812,6 +919,18 @@ int splitk_factor(int64_t M, int64_t N, int64_t K) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, K / 64), 64));
 }
 
+// Products that gemm_few_kernel takes, by the 32 x 32 tiles of C and K.  Up to
+// 2^17 tile-k's: 512 x 512 x 512 27 -> 17 .. 21 us a call, 1024 x 1024 x 128
+// 31 -> 17 .. 22, while 1024 x 512 x 512 with both operands k-contiguous goes
+// 29 -> 37 (every operand element is read M / 32 or N / 32 times) and 2048 x 1024
+// x 64 from 21 to 31.  K up to 512: then a wave's share is no longer than the
+// chains of a split K, and the error against 64 bits no larger (FP32: 0.8e-7
+// against 1.4e-7 at K = 64, 1.5e-7 for both at 512).
+static bool few_tiles(int prec, int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ceil_div(M, GT) * ceil_div(N, GT);
+  return (prec == P_F64 || prec == P_F32) && K <= 512 && tiles <= 1024 && tiles * K <= 1 << 17;
+}
+
 int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const void* B,
                     const Modes& b_k, const Modes& b_n, void* C, const Modes& c_m,
                     const Modes& c_n, int dtype, int prec, double alpha, double beta,
@@ -982,6 +1101,19 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
   g.a_kfast = a_k_unit ? 1 : 0;
   g.b_nfast = (b_k_unit && !b_n_unit) ? 0 : 1;
   TN_REQUIRE(ceil_div(M, BM) <= 65535, "contract: M too large");
+  if (few_tiles(prec, M, N, K)) {
+    ProfScope prof(prec == P_F64 ? PROF_GEMM_F64 : PROF_GEMM_F32, st,
+                   2.0 * (double)M * (double)N * (double)K,
+                   (double)(dtype == TN_F64 ? 8 : 4) *
+                       ((double)M * K + (double)K * N + (double)M * N));
+    const dim3 grid((unsigned)ceil_div(N, GT), (unsigned)ceil_div(M, GT));
+    if (prec == P_F64)
+      hipLaunchKernelGGL(gemm_few_kernel<double>, grid, dim3(64 * GW), 0, st, g);
+    else
+      hipLaunchKernelGGL(gemm_few_kernel<float>, grid, dim3(64 * GW), 0, st, g);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+  }
   const int64_t tiles = ceil_div(M, BM) * ceil_div(N, BN);
   // Split K when few output tiles would leave most CUs idle.
   int S = 1;
