@@ -475,8 +475,12 @@ __device__ inline void pair_gram(EigLds& sm, PairGramLds& pg, const double* __re
   const int nw = (int)((L + 31) >> 5);
   for (int q = tid; q < 3 * JB * JB; q += EIG_NT) {
     const int t = q >> 8, i = q & 255, m = ((i & 63) >> 4) + 4 * (i >> 6), n = i & 15;
-    double s = 0.0;
-    for (int w = 0; w < nw; ++w) s += pg.part[w][t][i];
+    // (every load issued before the first add)
+    double v[EIG_NW], s = 0.0;
+#pragma unroll
+    for (int w = 0; w < EIG_NW; ++w) v[w] = pg.part[min(w, nw - 1)][t][i];
+#pragma unroll
+    for (int w = 0; w < EIG_NW; ++w) s += w < nw ? v[w] : 0.0;
     const int pm = eig_pos(t == 2 ? JB + m : m), pn = eig_pos(t == 0 ? n : JB + n);
     sm.G[0][pm][pn] = s;
     if (t == 1) sm.G[0][pn][pm] = s;

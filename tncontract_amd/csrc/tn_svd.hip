@@ -190,19 +190,28 @@ __global__ void __launch_bounds__(EIG_NT) jac_eig_apply(double* __restrict__ Wv,
 // every block of a pair (grid as jac_eig_apply's) forms the pair's Gram matrix
 // itself and rotates its own row chunk, of Win into Wout (the other blocks of
 // the pair still read Win) or of Z in place.  A pair that needs no rotation is
-// copied.  It saves the Gram launch (4.4 us and the gap to the next) and the
+// copied.  offs: the measures of this sweep, of the one before and (cleared
+// here) of the next in turn, and the number of sweeps run; once a sweep has
+// found nothing to rotate, the steps of later ones leave everything alone, so
+// the host can enqueue sweeps ahead.  It saves the Gram launch (4.4 us and the gap to the next) and the
 // partials' trip through memory: 12.9 us a step, 254 x 636 SVD 3.09 -> 2.87 ms,
 // 64 x 64 eigensolve 618 -> 529 us.  Past 256 rows every block would repeat a
 // Gram as long as the launch it saves (512 rows: 3.4 us of MFMAs).
 __global__ void __launch_bounds__(EIG_NT) jac_step(const double* __restrict__ Win,
                                                    double* __restrict__ Wout, int64_t L,
                                                    double* __restrict__ Z, int64_t nv, int s,
-                                                   int nblk, int nchW, double tol,
-                                                   unsigned long long* __restrict__ offmax) {
+                                                   int nblk, int nchW, double tol, int sweep,
+                                                   unsigned long long* __restrict__ offs) {
   constexpr int CH = 16 * EIG_NW;
   __shared__ EigLds sm;
   __shared__ PairGramLds pg;
   const int pi = blockIdx.x, ch = blockIdx.y;
+  const bool done = sweep > 0 && __longlong_as_double((long long)offs[(sweep + 2) % 3]) <= tol;
+  if (s == 0 && pi == 0 && ch == 0 && threadIdx.x == 0) {
+    offs[(sweep + 1) % 3] = 0ull;  // (and so is every later sweep's)
+    if (!done) offs[3] = (unsigned long long)(sweep + 1);
+  }
+  if (done) return;
   int I, J;
   pair_blocks(pi, s, nblk, I, J);
   const bool onW = ch < nchW;
@@ -215,7 +224,7 @@ __global__ void __launch_bounds__(EIG_NT) jac_step(const double* __restrict__ Wi
   pair_gram(sm, pg, Win, L, nv, I, J);
   const bool inner = inner_step(s, nblk);
   const double off = eig_off(sm, tol, 0.0, inner);
-  if (ch == 0 && threadIdx.x == 0) atomicMax(offmax, dbits(off));
+  if (ch == 0 && threadIdx.x == 0) atomicMax(offs + sweep % 3, dbits(off));
   if (off <= tol) {
     if (onW) {
       const int lane = threadIdx.x & 63, lk = lane >> 4;
@@ -540,7 +549,7 @@ __global__ void gather_vectors(const T* __restrict__ src, Modes rows, Modes cols
   }
 }
 
-__global__ void reset_u64(unsigned long long* p) { *p = 0ull; }
+__global__ void reset_u64(unsigned long long* p) { p[threadIdx.x] = 0ull; }
 
 __global__ void init_identity(double* __restrict__ Z, int64_t k) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -656,8 +665,41 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   // (and graph-replayed): at least 16 steps, k >= 256
   // (short vectors: the other buffer of the one-launch steps instead)
   double* const W2 = nblk - 1 < 16 && L <= kPairLen ? sort_tmp : nullptr;
-  double *Wcur = Wv, *Wnext = W2;
   if (nblk - 1 < 16) sort_tmp = nullptr;
+  if (W2) {
+    // six sweeps, then two at a time, between looks at the measure: a look costs
+    // 25 us of an idle GPU, a sweep enqueued for nothing 2 us a step, and these
+    // sizes need 7 to 12 sweeps (254 x 636 SVD 2.85 -> 2.35 ms)
+    hipLaunchKernelGGL(reset_u64, dim3(1), dim3(4), 0, st, w.off);
+    unsigned long long h[4] = {0, 0, 0, 0};
+    for (int todo = std::min(6, max_sweeps); sweep < max_sweeps && !*converged;
+         todo = std::min(2, max_sweeps - sweep)) {
+      for (int i = 0; i < todo; ++i)
+        for (int s = 0; s < nblk - 1; ++s) {
+          ProfScope p(PROF_JAC_EIG, st,
+                      step_rounds(inner_step(s, nblk)) * 9216.0 * npairs + gram_fl + apply_fl,
+                      16.0 * (double)(L + kz) * J2 * npairs);
+          const bool flip = (((sweep + i) * (nblk - 1) + s) & 1) != 0;
+          hipLaunchKernelGGL(jac_step, dim3(npairs, nchW + nchZ), dim3(EIG_NT), 0, st,
+                             flip ? W2 : Wv, flip ? Wv : W2, L, Z, k, s, nblk, nchW, tol, sweep + i,
+                             w.off);
+        }
+      TN_CHECK_LAUNCH();
+      TN_HIP(hipMemcpyAsync(h, w.off, sizeof(h), hipMemcpyDeviceToHost, st));
+      TN_HIP(hipStreamSynchronize(st));
+      sweep = (int)h[3];
+      double off;
+      memcpy(&off, &h[(sweep + 2) % 3], sizeof(off));
+      *converged = off <= tol;
+    }
+    if ((sweep * (nblk - 1)) & 1) {
+      hipLaunchKernelGGL(copy_f64, dim3((unsigned)ceil_div(L * k, 256)), dim3(256), 0, st, W2, Wv,
+                         L * k);
+      TN_CHECK_LAUNCH();
+    }
+    if (sweeps_out) *sweeps_out = sweep;
+    return TN_OK;
+  }
   auto enqueue_sweep = [&]() -> int {
     hipLaunchKernelGGL(reset_u64, dim3(1), dim3(1), 0, st, w.off);
     if (sort_tmp) {
@@ -673,15 +715,6 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
       }
     }
     for (int s = 0; s < nblk - 1; ++s) {
-      if (W2) {
-        ProfScope p(PROF_JAC_EIG, st,
-                    step_rounds(inner_step(s, nblk)) * 9216.0 * npairs + gram_fl + apply_fl,
-                    16.0 * (double)(L + kz) * J2 * npairs);
-        hipLaunchKernelGGL(jac_step, dim3(npairs, nchW + nchZ), dim3(EIG_NT), 0, st, Wcur, Wnext, L,
-                           Z, k, s, nblk, nchW, tol, w.off);
-        std::swap(Wcur, Wnext);
-        continue;
-      }
       {
         ProfScope p(PROF_JAC_GRAM, st, gram_fl, 8.0 * (double)L * J2 * npairs);
         hipLaunchKernelGGL(jac_gram, dim3(npairs, nchG), dim3(256), 0, st, Wv, L, k, s, nblk,
@@ -789,11 +822,6 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   if (exec) (void)hipGraphExecDestroy(exec);
   if (graph) (void)hipGraphDestroy(graph);
   if (rc_loop != TN_OK) return rc_loop;
-  if (Wcur != Wv) {
-    hipLaunchKernelGGL(copy_f64, dim3((unsigned)ceil_div(L * k, 256)), dim3(256), 0, st, Wcur, Wv,
-                       L * k);
-    TN_CHECK_LAUNCH();
-  }
   if (sweeps_out) *sweeps_out = sweep;
   return TN_OK;
 }
