@@ -302,7 +302,7 @@ __device__ __forceinline__ void xcd_tile(int& tx, int& ty) {
 // one barrier and K / 128 trips, against LDS tiles of 128 x 128 (64 x 64), each
 // with a barrier per 16 k, and a second launch to sum a K split
 // (a call of 256 x 256 x 128, FP64: 22 -> 17 us, of which 12 are the host's).
-constexpr int GT = 32, GW = 8;
+constexpr int GT = 32, GW = 8, kFewK = 512;
 
 template <typename T> struct Frag;
 template <> struct Frag<double> {
@@ -320,11 +320,21 @@ template <> struct Frag<float> {
   static __device__ int row(int lk, int e) { return 4 * lk + e; }
 };
 
-template <typename T>
+// KS: one mode of contracted indices on both sides, so a lane's offsets are
+// fixed steps from its first; otherwise they come from a table in LDS.
+template <typename T, bool KS>
 __global__ void __launch_bounds__(64 * GW) gemm_few_kernel(GemmArgs g) {
   using V = typename Frag<T>::V;
   __shared__ T red[GW][4][256];
+  __shared__ int64_t koff[2][KS ? 1 : kFewK];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  if constexpr (!KS) {
+    for (int k = tid; k < (int)g.K; k += 64 * GW) {
+      koff[0][k] = goff(g.ak, k);
+      koff[1][k] = goff(g.bk, k);
+    }
+    __syncthreads();
+  }
   const int64_t m0 = (int64_t)blockIdx.y * GT, n0 = (int64_t)blockIdx.x * GT;
   // rows and columns past the end read the last one; they are not stored
   const T* ap[2];
@@ -342,11 +352,25 @@ __global__ void __launch_bounds__(64 * GW) gemm_few_kernel(GemmArgs g) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = V{0, 0, 0, 0};
   T a[2][4], b[2][4];
+  const int64_t sa = KS ? g.ak.strides[0] : 0, sb = KS ? g.bk.strides[0] : 0;
   auto fetch = [&](int kb, T (&x)[2][4], T (&y)[2][4]) {
+    if (KS && kb + 16 <= k1) {
+      const int64_t qa = (kb + 2 * lk) * sa, qb = (kb + 2 * lk) * sb;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const T *pa = ap[i] + qa, *pb = bp[i] + qb;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          x[i][s] = pa[(8 * (s >> 1) + (s & 1)) * sa];
+          y[i][s] = pb[(8 * (s >> 1) + (s & 1)) * sb];
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int k = kb + 8 * (s >> 1) + 2 * lk + (s & 1), kc = min(k, K - 1);
-      const int64_t oa = goff(g.ak, kc), ob = goff(g.bk, kc);
+      const int64_t oa = KS ? kc * sa : koff[0][kc], ob = KS ? kc * sb : koff[1][kc];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const T u = ap[i][oa], v = bp[i][ob];
@@ -928,7 +952,7 @@ int splitk_factor(int64_t M, int64_t N, int64_t K) {
 // against 1.4e-7 at K = 64, 1.5e-7 for both at 512).
 static bool few_tiles(int prec, int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ceil_div(M, GT) * ceil_div(N, GT);
-  return (prec == P_F64 || prec == P_F32) && K <= 512 && tiles <= 1024 && tiles * K <= 1 << 17;
+  return (prec == P_F64 || prec == P_F32) && K <= kFewK && tiles <= 1024 && tiles * K <= 1 << 17;
 }
 
 int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const void* B,
@@ -1107,10 +1131,15 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
                    (double)(dtype == TN_F64 ? 8 : 4) *
                        ((double)M * K + (double)K * N + (double)M * N));
     const dim3 grid((unsigned)ceil_div(N, GT), (unsigned)ceil_div(M, GT));
-    if (prec == P_F64)
-      hipLaunchKernelGGL(gemm_few_kernel<double>, grid, dim3(64 * GW), 0, st, g);
+    const bool ks = g.ak.n == 1 && g.bk.n == 1;
+    if (prec == P_F64 && ks)
+      hipLaunchKernelGGL((gemm_few_kernel<double, true>), grid, dim3(64 * GW), 0, st, g);
+    else if (prec == P_F64)
+      hipLaunchKernelGGL((gemm_few_kernel<double, false>), grid, dim3(64 * GW), 0, st, g);
+    else if (ks)
+      hipLaunchKernelGGL((gemm_few_kernel<float, true>), grid, dim3(64 * GW), 0, st, g);
     else
-      hipLaunchKernelGGL(gemm_few_kernel<float>, grid, dim3(64 * GW), 0, st, g);
+      hipLaunchKernelGGL((gemm_few_kernel<float, false>), grid, dim3(64 * GW), 0, st, g);
     TN_CHECK_LAUNCH();
     return TN_OK;
   }
