@@ -183,40 +183,48 @@ struct BJob {
 };
 
 // Where a job's Jacobi stands: step s of a sweep over its first nb blocks
-// (nb = 0: retired).  Kept twice, by the parity of the global step: a step's
-// kernels read one while the next step's is written.
+// (nb = 0: retired) after sw whole ones.  Kept twice, by the parity of the
+// global step: a step's kernels read one while another is written.
 struct BState {
-  int32_t s, nb;
+  int32_t s, nb, sw, pad;
 };
 
-// The state after this step, by one thread per job once the step's measures
-// are in offmax.  A job first sweeps over its blocks up to nact alone, until it
+// The state after a step, off being the sweep's measure if it was the sweep's
+// last; outcome: 1 if the job is done with it, 2 if it gives up.  A job first sweeps over its blocks up to nact alone, until it
 // is a sweep or two from convergence (the off-diagonal is about squared per
 // sweep, so at off <= 10 sqrt(tol)); then over all its blocks until a whole
 // sweep has nothing to rotate.  A product of rank r leaves the QR with r rows
 // and negligible ones: those then cost the last three sweeps instead of all
 // (32 products of ranks 22 .. 492 and sizes up to 1022: 46.0 -> 34.5 ms;
 // going over to all blocks a sweep later costs a sweep of the first ones).
-__device__ __forceinline__ void bstate_next(const BJob& J, int j, BState cur, int max_sweeps,
-                                            BState* __restrict__ next, int* __restrict__ done,
-                                            int* __restrict__ sweeps,
-                                            unsigned long long* __restrict__ offmax,
-                                            int* __restrict__ active) {
-  BState n{cur.s + 1, cur.nb};
+__device__ __forceinline__ BState bstate_after(const BJob& J, BState cur, double off,
+                                               int max_sweeps, int& outcome) {
+  BState n{cur.s + 1, cur.nb, cur.sw, 0};
+  outcome = 0;
   if (cur.nb > 0 && n.s == cur.nb - 1) {
-    const double off = __longlong_as_double((long long)offmax[j]);
-    offmax[j] = 0ull;
-    const int sw = ++sweeps[j];
     n.s = 0;
+    n.sw = cur.sw + 1;
     if (cur.nb < J.nblk) {
-      if (off * off <= 100.0 * J.tol || sw >= max_sweeps) n.nb = J.nblk;
-    } else if (off <= J.tol || sw >= max_sweeps + (J.nact < J.nblk ? 2 : 0)) {
-      done[j] = off <= J.tol ? 1 : 2;
-      atomicSub(active, 1);
+      if (off * off <= 100.0 * J.tol || n.sw >= max_sweeps) n.nb = J.nblk;
+    } else if (off <= J.tol || n.sw >= max_sweeps + (J.nact < J.nblk ? 2 : 0)) {
+      outcome = off <= J.tol ? 1 : 2;
       n.nb = 0;
     }
   }
-  next[j] = n;
+  return n;
+}
+
+// What the host reads of a job's state, by one thread per job and step.
+struct BOut {
+  int *done, *sweeps, *active;
+};
+__device__ __forceinline__ void bstate_note(const BOut& o, int j, BState was, BState now,
+                                            int outcome) {
+  if (now.sw != was.sw) o.sweeps[j] = now.sw;
+  if (outcome) {
+    o.done[j] = outcome;
+    atomicSub(o.active, 1);
+  }
 }
 
 // acc += the 32 x 32 Gram of the pair's vectors (blocks I and K2 of the
@@ -375,17 +383,23 @@ __global__ void __launch_bounds__(256) bjac_apply(double* __restrict__ Wv, doubl
                                                   const int* __restrict__ skip,
                                                   unsigned long long* __restrict__ work,
                                                   BState* __restrict__ next, int max_sweeps,
-                                                  int* __restrict__ done, int* __restrict__ sweeps,
                                                   unsigned long long* __restrict__ offmax,
-                                                  int* __restrict__ active) {
+                                                  BOut out) {
   __shared__ double Q[BJ2][BJ2 + 1];
   const int item = blockIdx.x;
   const int j = a_job[item];
   const BState S = state[j];
   const int pi = a_pair[item], ch = a_chunk[item];
   const BJob J = jobs[j];
-  if (pi == 0 && ch == 0 && threadIdx.x == 0)
-    bstate_next(J, j, S, max_sweeps, next, done, sweeps, offmax, active);
+  if (pi == 0 && ch == 0 && threadIdx.x == 0) {
+    // the step's measures are in: the next step's state
+    int outcome;
+    const BState n =
+        bstate_after(J, S, __longlong_as_double((long long)offmax[j]), max_sweeps, outcome);
+    if (n.sw != S.sw) offmax[j] = 0ull;
+    next[j] = n;
+    bstate_note(out, j, S, n, outcome);
+  }
   if (2 * pi >= S.nb) return;
   const int eidx = J.eig_base + pi;
   if (skip[eidx]) return;
@@ -425,17 +439,29 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
                                                   const BJob* __restrict__ jobs,
                                                   const int* __restrict__ e_job,
                                                   const int* __restrict__ e_pair,
-                                                  const BState* __restrict__ state,
-                                                  unsigned long long* __restrict__ offmax,
-                                                  unsigned long long* __restrict__ work) {
+                                                  const BState* __restrict__ prev,
+                                                  BState* __restrict__ next, int max_sweeps,
+                                                  unsigned long long* __restrict__ offs,
+                                                  unsigned long long* __restrict__ work, BOut out) {
   __shared__ PairGramLds pg;
   __shared__ EigLds sm;
   const int item = blockIdx.x, tid = threadIdx.x;
   const int j = e_job[item];
-  const BState S = state[j];
   const int pi = e_pair[item];
-  if (2 * pi >= S.nb) return;
   const BJob J = jobs[j];
+  // every block of a job works out the step's state from the one before, one
+  // keeps it; the measures of three sweeps in turn: one being read, one being
+  // formed, one being cleared
+  const BState P = prev[j];
+  int outcome;
+  const BState S = bstate_after(J, P, __longlong_as_double((long long)offs[3 * j + P.sw % 3]),
+                                max_sweeps, outcome);
+  if (pi == 0 && tid == 0) {
+    next[j] = S;
+    if (S.s == 0) offs[3 * j + (S.sw + 1) % 3] = 0ull;
+    bstate_note(out, j, P, S, outcome);
+  }
+  if (2 * pi >= S.nb) return;
   const int I = brr(pi, S.s, S.nb), K2 = brr(S.nb - 1 - pi, S.s, S.nb);
   double* W = Wv + J.wv;
   double* Z = Zb + J.z;
@@ -445,7 +471,7 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
   pair_gram(sm, pg, W, J.L, J.k, I, K2);
   const bool inner = inner_step(S.s, S.nb);
   const double off = eig_off(sm, J.tol, J.neg2, inner);
-  if (tid == 0) atomicMax(offmax + j, dbits(off));
+  if (tid == 0) atomicMax(offs + 3 * j + S.sw % 3, dbits(off));
   if (off <= J.tol) return;
   if (work && tid == 0) {
     atomicAdd(work, (unsigned long long)J.L);
@@ -457,18 +483,10 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
   apply_rows_finish<2, EIG_NW>(Z, J.k, J.k, 0, J.k, I, K2, z, sm.Q);
 }
 
-// After a fused step (bjac_apply advances the jobs itself).
-__global__ void bjac_step_end(const BJob* __restrict__ jobs, int njobs,
-                              const BState* __restrict__ state, BState* __restrict__ next,
-                              int max_sweeps, int* __restrict__ done, int* __restrict__ sweeps,
-                              unsigned long long* __restrict__ offmax, int* __restrict__ active) {
+__global__ void binit_state(const BJob* __restrict__ jobs, int njobs, int s,
+                            BState* __restrict__ state) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < njobs) bstate_next(jobs[j], j, state[j], max_sweeps, next, done, sweeps, offmax, active);
-}
-
-__global__ void binit_state(const BJob* __restrict__ jobs, int njobs, BState* __restrict__ state) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < njobs) state[j] = BState{0, jobs[j].nact};
+  if (j < njobs) state[j] = BState{s, jobs[j].nact, 0, 0};
 }
 
 __global__ void binit_identity(double* __restrict__ Zb, const BJob* __restrict__ jobs) {
@@ -772,7 +790,7 @@ static size_t batched_ws_bytes(const std::vector<int64_t>& ms, const std::vector
   a.take<AJob>((size_t)njobs);
   a.take<int>((size_t)njobs * 2);  // tile base + ids
   a.take<int>((size_t)njobs * 4);  // done, sweeps, kept, active
-  a.take<unsigned long long>((size_t)njobs);
+  a.take<unsigned long long>((size_t)njobs * 3);
   a.take<unsigned long long>(3);  // work counters
   a.take<double>(sv * 2);
   a.take<int>(sv);
@@ -943,7 +961,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   int* dsweeps = a.take<int>((size_t)njobs);
   int* dkept = a.take<int>((size_t)njobs);
   int* dactive = a.take<int>((size_t)njobs);
-  unsigned long long* doff = a.take<unsigned long long>((size_t)njobs);
+  unsigned long long* doff = a.take<unsigned long long>((size_t)njobs * 3);
   unsigned long long* dwork = a.take<unsigned long long>(3);
   double* dsig = a.take<double>((size_t)sv);
   double* dS = a.take<double>((size_t)sv);
@@ -977,7 +995,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   }
   TN_HIP(hipMemsetAsync(ddone, 0, sizeof(int) * njobs, st));
   TN_HIP(hipMemsetAsync(dsweeps, 0, sizeof(int) * njobs, st));
-  TN_HIP(hipMemsetAsync(doff, 0, sizeof(unsigned long long) * njobs, st));
+  TN_HIP(hipMemsetAsync(doff, 0, sizeof(unsigned long long) * njobs * 3, st));
   // rows through the Gram and rotation kernels and eigensolves that rotated,
   // counted only while launch timing is on (they give the Jacobi rooflines)
   unsigned long long* cnt = prof_on() ? dwork : nullptr;
@@ -1069,12 +1087,14 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     hipLaunchKernelGGL(bjob_neg2, dim3((unsigned)njobs), dim3(256), 0, st, dsig, dsbase, dbj,
                        rel_threshold);
   }
-  const unsigned njb = (unsigned)ceil_div(njobs, 256);
-  hipLaunchKernelGGL(binit_state, dim3(njb), dim3(256), 0, st, dbj, njobs, dstate);
   TN_CHECK_LAUNCH();
   // every job within one row chunk: the one-launch step
   bool fused = true;
   for (int j = 0; j < njobs; ++j) fused = fused && bj[j].L <= BCH && bj[j].k <= BCH;
+  // (a fused step's state follows the one before it; the others' is ready)
+  hipLaunchKernelGGL(binit_state, dim3((unsigned)ceil_div(njobs, 256)), dim3(256), 0, st, dbj,
+                     njobs, fused ? -1 : 0, fused ? dstate + njobs : dstate);
+  const BOut outcomes{ddone, dsweeps, dactive};
   // A step set of `period` steps is enqueued as one unit (captured once as a
   // HIP graph and replayed; launched kernel by kernel while launch timing is
   // on).  The host reads the active-job count of a set while the next set
@@ -1084,15 +1104,12 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   constexpr int period = 16;
   auto enqueue_set = [&]() {
     for (int o = 0; o < period; ++o) {
-      const BState* cur = dstate + (o & 1) * njobs;
-      BState* next = dstate + (~o & 1) * njobs;
+      BState *cur = dstate + (o & 1) * njobs, *other = dstate + (~o & 1) * njobs;
       // work is counted on the device (cnt) and added once at the end
       if (fused) {
         ProfScope p(PROF_JAC_EIG, st, 0.0, 0.0);
         hipLaunchKernelGGL(bjac_fused, dim3(nei), dim3(EIG_NT), 0, st, dWv, dZ, dbj, det, det + nei,
-                           cur, doff, cnt);
-        hipLaunchKernelGGL(bjac_step_end, dim3(njb), dim3(256), 0, st, dbj, njobs, cur, next,
-                           max_sweeps, ddone, dsweeps, doff, dactive);
+                           other, cur, max_sweeps, doff, cnt, outcomes);
       } else {
         {
           ProfScope p(PROF_JAC_GRAM, st, 0.0, 0.0);
@@ -1107,8 +1124,8 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
         {
           ProfScope p(PROF_JAC_APPLY, st, 0.0, 0.0);
           hipLaunchKernelGGL(bjac_apply, dim3(nai), dim3(256), 0, st, dWv, dZ, dbj, dat, dat + nai,
-                             dat + 2 * nai, cur, dQ, dskip, cnt, next, max_sweeps, ddone, dsweeps,
-                             doff, dactive);
+                             dat + 2 * nai, cur, dQ, dskip, cnt, other, max_sweeps, doff,
+                             outcomes);
         }
       }
     }
@@ -1138,7 +1155,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     set_error(TN_ERR_HIP, "%s: host buffer or event creation failed", who);
     rc_loop = TN_ERR_HIP;
   }
-  const int nsets = (int)ceil_div((int64_t)maxsteps * (max_sweeps + 2), period);
+  const int nsets = (int)ceil_div((int64_t)maxsteps * (max_sweeps + 2) + 1, period);
   for (int p = 0; rc_loop == TN_OK && p < nsets; ++p) {
     if (exec) {
       if (hipGraphLaunch(exec, st) != hipSuccess) {
