@@ -669,7 +669,7 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   if (W2) {
     // six sweeps, then two at a time, between looks at the measure: a look costs
     // 25 us of an idle GPU, a sweep enqueued for nothing 2 us a step, and these
-    // sizes need 7 to 12 sweeps (254 x 636 SVD 2.85 -> 2.35 ms)
+    // sizes need 7 to 12 sweeps (254 x 636 SVD 2.85 -> 2.63 ms)
     hipLaunchKernelGGL(reset_u64, dim3(1), dim3(4), 0, st, w.off);
     unsigned long long h[4] = {0, 0, 0, 0};
     for (int todo = std::min(6, max_sweeps); sweep < max_sweeps && !*converged;
