@@ -227,58 +227,19 @@ __device__ __forceinline__ void bstate_note(const BOut& o, int j, BState was, BS
   }
 }
 
-// acc += the 32 x 32 Gram of the pair's vectors (blocks I and K2 of the
-// job's k vectors of length L at W) over rows [r0, r1): tiles of 64 rows
-// staged through LDS, v_mfma_f64_16x16x4 by 4 waves (wave w takes the 16 x 16
-// quarter w); the next tile's loads are issued into registers before the
-// current tile's MFMAs, so their latency overlaps the MFMAs.
-__device__ __forceinline__ void bgram_rows(const double* __restrict__ W, int64_t L, int k, int I,
-                                           int K2, int64_t r0, int64_t r1,
-                                           double (*Ps)[BJ2 + 1], f64x4b& acc) {
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ti = wave >> 1, tj = wave & 1;
-  constexpr int PE = 64 * BJ2 / 256;
-  double pv[PE];
-  auto fetch = [&](int64_t rb) {
-#pragma unroll
-    for (int i = 0; i < PE; ++i) {
-      const int e = tid + 256 * i, row = e % 64, col = e / 64;
-      const int64_t v = col < BJB ? (int64_t)I * BJB + col : (int64_t)K2 * BJB + (col - BJB);
-      const int64_t r = rb + row;
-      pv[i] = (v < k && r < r1) ? W[v * L + r] : 0.0;
-    }
-  };
-  if (r0 < r1) fetch(r0);
-  for (int64_t rb = r0; rb < r1; rb += 64) {
-#pragma unroll
-    for (int i = 0; i < PE; ++i) {
-      const int e = tid + 256 * i;
-      Ps[e % 64][e / 64] = pv[i];
-    }
-    __syncthreads();
-    if (rb + 64 < r1) fetch(rb + 64);
-#pragma unroll
-    for (int k0 = 0; k0 < 64; k0 += 4) {
-      double a = Ps[k0 + (lane >> 4)][16 * ti + (lane & 15)];
-      double b = Ps[k0 + (lane >> 4)][16 * tj + (lane & 15)];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    }
-    __syncthreads();
-  }
-}
-
 __device__ __forceinline__ int brr(int pos, int step, int nblk) {
   return pos == 0 ? 0 : 1 + (pos - 1 + step) % (nblk - 1);
 }
 
-__global__ void __launch_bounds__(256) bjac_gram(double* __restrict__ Wv, const BJob* __restrict__ jobs,
-                                                 const int* __restrict__ it_job,
-                                                 const int* __restrict__ it_pair,
-                                                 const int* __restrict__ it_chunk,
-                                                 const BState* __restrict__ state,
-                                                 double* __restrict__ Gpart,
-                                                 unsigned long long* __restrict__ work) {
-  __shared__ double Ps[64][BJ2 + 1];
+__global__ void __launch_bounds__(EIG_NT) bjac_gram(double* __restrict__ Wv,
+                                                    const BJob* __restrict__ jobs,
+                                                    const int* __restrict__ it_job,
+                                                    const int* __restrict__ it_pair,
+                                                    const int* __restrict__ it_chunk,
+                                                    const BState* __restrict__ state,
+                                                    double* __restrict__ Gpart,
+                                                    unsigned long long* __restrict__ work) {
+  __shared__ PairGramLds pg;
   const int item = blockIdx.x;
   const int j = it_job[item];
   const BState S = state[j];
@@ -286,19 +247,11 @@ __global__ void __launch_bounds__(256) bjac_gram(double* __restrict__ Wv, const 
   if (2 * pi >= S.nb) return;
   const BJob J = jobs[j];
   const int I = brr(pi, S.s, S.nb), K2 = brr(S.nb - 1 - pi, S.s, S.nb);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ti = wave >> 1, tj = wave & 1;
-  const int64_t r0 = (int64_t)ch * BCH, r1 = min((int64_t)J.L, r0 + BCH);
-  if (work && tid == 0) atomicAdd(work, (unsigned long long)(r1 - r0));
-  const double* base = Wv + J.wv;
-  f64x4b acc = {0, 0, 0, 0};
-  bgram_rows(base, J.L, J.k, I, K2, r0, r1, Ps, acc);
+  const int r0 = ch * BCH, rows = min(J.L - r0, BCH);
+  if (work && threadIdx.x == 0) atomicAdd(work, (unsigned long long)rows);
   double* out = Gpart + (int64_t)item * (BJ2 * BJ2);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    int r = 16 * ti + (lane >> 4) + 4 * e, c = 16 * tj + (lane & 15);
-    out[r * BJ2 + c] = acc[e];
-  }
+  pair_gram_rows(pg, Wv + J.wv + r0, J.L, rows, J.k, I, K2,
+                 [&](int r, int c, double v) { out[r * BJ2 + c] = v; });
 }
 
 // a pair eigensolve in the work counter: the number in the low half, the
@@ -1113,7 +1066,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
       } else {
         {
           ProfScope p(PROF_JAC_GRAM, st, 0.0, 0.0);
-          hipLaunchKernelGGL(bjac_gram, dim3(ngi), dim3(256), 0, st, dWv, dbj, dgt, dgt + ngi,
+          hipLaunchKernelGGL(bjac_gram, dim3(ngi), dim3(EIG_NT), 0, st, dWv, dbj, dgt, dgt + ngi,
                              dgt + 2 * ngi, cur, dG, cnt);
         }
         {

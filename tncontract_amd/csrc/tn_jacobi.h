@@ -421,32 +421,37 @@ __device__ inline void eig_rotate(EigLds& sm, double tol, double neg2 = 0.0, boo
   lds_barrier();
 }
 
-// G (sm.G[0]) of the pair's 32 vectors of length L <= kPairLen (vector v at
-// W + v * L, nv vectors) by the whole workgroup of 8 waves, straight from
-// memory: wave w takes rows 32 w .. 32 w + 31, two neighbouring rows a lane and
-// load, as operands of v_mfma_f64_16x16x4 (the summation index may be any row,
-// as long as both operands agree), for the three 16 x 16 quarters that are not
-// each other's mirror; the waves' sums meet in LDS.  No staging and no barrier
-// before the last: what bounds it is one trip to memory and 24 MFMAs a wave.
+// Gram matrix of a pair's 32 vectors over at most kPairLen rows (vector v at
+// W + v * ld, nv vectors, `rows` rows) by the whole workgroup of 8 waves,
+// straight from memory: wave w takes rows 32 w .. 32 w + 31, two neighbouring
+// rows a lane and load, as operands of v_mfma_f64_16x16x4 (the summation index
+// may be any row, as long as both operands agree), for the three 16 x 16
+// quarters that are not each other's mirror; the waves' sums meet in LDS and
+// put(r, c, s) takes the entries (both mirrored ones).  No staging and no
+// barrier before the last: what bounds it is one trip to memory and 24 MFMAs a
+// wave.
 constexpr int kPairLen = 32 * EIG_NW;
-typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));  // odd L: 8-byte aligned
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));  // odd ld: 8-byte aligned
 
 struct PairGramLds {
   double part[EIG_NW][3][JB * JB];
 };
 
-__device__ inline void pair_gram(EigLds& sm, PairGramLds& pg, const double* __restrict__ W,
-                                 int64_t L, int64_t nv, int I, int J) {
+template <typename Put>
+__device__ __forceinline__ void pair_gram_rows(PairGramLds& pg, const double* __restrict__ W,
+                                               int64_t ld, int rows, int64_t nv, int I, int J,
+                                               Put put) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
-  const int64_t r0 = 32 * wave, vi = (int64_t)I * JB + lr, vj = (int64_t)J * JB + lr;
+  const int r0 = 32 * wave;
+  const int64_t vi = (int64_t)I * JB + lr, vj = (int64_t)J * JB + lr;
   f64x4 acc[3] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
-  if (r0 < L) {
+  if (r0 < rows) {
     double xi[8], xj[8];
-    if (r0 + 32 <= L && ((int64_t)max(I, J) + 1) * JB <= nv) {
+    if (r0 + 32 <= rows && ((int64_t)max(I, J) + 1) * JB <= nv) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int64_t r = r0 + 8 * j + 2 * lk;
-        const f64x2u a = *(const f64x2u*)(W + vi * L + r), b = *(const f64x2u*)(W + vj * L + r);
+        const int r = r0 + 8 * j + 2 * lk;
+        const f64x2u a = *(const f64x2u*)(W + vi * ld + r), b = *(const f64x2u*)(W + vj * ld + r);
         xi[2 * j] = a[0];
         xi[2 * j + 1] = a[1];
         xj[2 * j] = b[0];
@@ -455,9 +460,9 @@ __device__ inline void pair_gram(EigLds& sm, PairGramLds& pg, const double* __re
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int64_t r = r0 + 8 * (j >> 1) + 2 * lk + (j & 1);
-        xi[j] = (vi < nv && r < L) ? W[vi * L + r] : 0.0;
-        xj[j] = (vj < nv && r < L) ? W[vj * L + r] : 0.0;
+        const int r = r0 + 8 * (j >> 1) + 2 * lk + (j & 1);
+        xi[j] = (vi < nv && r < rows) ? W[vi * ld + r] : 0.0;
+        xj[j] = (vj < nv && r < rows) ? W[vj * ld + r] : 0.0;
       }
     }
 #pragma unroll
@@ -472,7 +477,7 @@ __device__ inline void pair_gram(EigLds& sm, PairGramLds& pg, const double* __re
       for (int e = 0; e < 4; ++e) pg.part[wave][t][64 * e + lane] = acc[t][e];
   }
   lds_barrier();
-  const int nw = (int)((L + 31) >> 5);
+  const int nw = (rows + 31) >> 5;
   for (int q = tid; q < 3 * JB * JB; q += EIG_NT) {
     const int t = q >> 8, i = q & 255, m = ((i & 63) >> 4) + 4 * (i >> 6), n = i & 15;
     // (every load issued before the first add)
@@ -481,10 +486,17 @@ __device__ inline void pair_gram(EigLds& sm, PairGramLds& pg, const double* __re
     for (int w = 0; w < EIG_NW; ++w) v[w] = pg.part[min(w, nw - 1)][t][i];
 #pragma unroll
     for (int w = 0; w < EIG_NW; ++w) s += w < nw ? v[w] : 0.0;
-    const int pm = eig_pos(t == 2 ? JB + m : m), pn = eig_pos(t == 0 ? n : JB + n);
-    sm.G[0][pm][pn] = s;
-    if (t == 1) sm.G[0][pn][pm] = s;
+    const int r = t == 2 ? JB + m : m, c = t == 0 ? n : JB + n;
+    put(r, c, s);
+    if (t == 1) put(c, r, s);
   }
+}
+
+// ... over all L <= kPairLen rows into sm.G[0].
+__device__ inline void pair_gram(EigLds& sm, PairGramLds& pg, const double* __restrict__ W,
+                                 int64_t L, int64_t nv, int I, int J) {
+  pair_gram_rows(pg, W, L, (int)L, nv, I, J,
+                 [&](int r, int c, double s) { sm.G[0][eig_pos(r)][eig_pos(c)] = s; });
   lds_barrier();
 }
 

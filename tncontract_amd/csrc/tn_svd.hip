@@ -7,8 +7,8 @@
 // (length L = max(m,n)); Z (k x k) accumulates the rotations.  Vectors are
 // grouped in blocks of 16; each outer step pairs the blocks round-robin and,
 // for every pair (I,J) at once:
-//   1. jac_gram:  partial Gram G = P^T P of P = [W_I W_J] over a row chunk,
-//                 v_mfma_f64_16x16x4 from an LDS tile (grid: pairs x chunks);
+//   1. jac_gram:  partial Gram G = P^T P of P = [W_I W_J] over a row chunk by
+//                 v_mfma_f64_16x16x4 (grid: pairs x chunks);
 //   2. jac_eig_apply: every block of a pair sums the partials, records the
 //                 largest normalised off-diagonal |G_pq|/sqrt(G_pp G_qq),
 //                 runs one cyclic sweep of two-sided Jacobi on the 32x32 G
@@ -46,59 +46,11 @@ static int eig_nt(int npairs, int64_t L, int64_t kz) {
     nt *= 2;
   return nt;
 }
-constexpr int GCH = 128;     // rows per Gram partial of jac_gram (twice the blocks)
+// Rows per Gram partial of jac_gram: what a workgroup reads in one trip (four
+// partials a pair at n = 1024; eight of 128 rows through LDS took the same 5.0 us
+// but the step 0.5 us more: 1024 x 2560 SVD 17.0 -> 16.7 ms).
+constexpr int GCH = kPairLen;
 
-// Partial Gram P^T P of the pair's 32 vectors over rows [r0, r1) into out
-// (32 x 32, row stride ostride; global or LDS), v_mfma_f64_16x16x4 from a
-// double-buffered LDS tile.  256 threads.
-__device__ void gram_partial(double (*Ps)[64][J2 + 1], const double* __restrict__ Wv, int64_t L,
-                             int64_t nv, int I, int J, int64_t r0, int64_t r1,
-                             double* __restrict__ out, int ostride = J2) {
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int ti = wave >> 1, tj = wave & 1;
-  f64x4 acc = {0, 0, 0, 0};
-  double reg[8];
-  auto load = [&](int64_t rb) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      int e = tid + 256 * j;
-      int row = e & 63, col = e >> 6;
-      int64_t v = pair_vec(col, I, J);
-      int64_t r = rb + row;
-      reg[j] = (v < nv && r < r1) ? Wv[v * L + r] : 0.0;
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      int e = tid + 256 * j;
-      Ps[buf][e & 63][e >> 6] = reg[j];
-    }
-  };
-  const int nsub = (int)((r1 - r0 + 63) / 64);
-  if (nsub > 0) {
-    load(r0);
-    store(0);
-  }
-  lds_barrier();
-  for (int sb = 0; sb < nsub; ++sb) {
-    const int buf = sb & 1;
-    if (sb + 1 < nsub) load(r0 + (int64_t)(sb + 1) * 64);
-#pragma unroll
-    for (int k0 = 0; k0 < 64; k0 += 4) {
-      double a = Ps[buf][k0 + (lane >> 4)][16 * ti + (lane & 15)];
-      double b = Ps[buf][k0 + (lane >> 4)][16 * tj + (lane & 15)];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    }
-    if (sb + 1 < nsub) store(buf ^ 1);
-    lds_barrier();
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    int r = 16 * ti + (lane >> 4) + 4 * e, c = 16 * tj + (lane & 15);
-    out[r * ostride + c] = acc[e];
-  }
-}
 
 // G (sm.G[0]) = sum of the pair's nchunk partials (fixed order, so every
 // block that sums them gets the same bits).  The partials are read eight
@@ -138,16 +90,17 @@ __device__ void eig_load(EigLds& sm, const double* __restrict__ Gp, int nchunk) 
   lds_barrier();
 }
 
-__global__ void __launch_bounds__(256) jac_gram(const double* __restrict__ Wv, int64_t L,
-                                                int64_t nv, int s, int nblk, int nchunk,
-                                                double* __restrict__ Gpart) {
-  __shared__ double Ps[2][64][J2 + 1];
+__global__ void __launch_bounds__(EIG_NT) jac_gram(const double* __restrict__ Wv, int64_t L,
+                                                   int64_t nv, int s, int nblk, int nchunk,
+                                                   double* __restrict__ Gpart) {
+  __shared__ PairGramLds pg;
   const int pi = blockIdx.x, ch = blockIdx.y;
   int I, J;
   pair_blocks(pi, s, nblk, I, J);
   const int64_t r0 = (int64_t)ch * GCH;
-  const int64_t r1 = min(L, r0 + GCH);
-  gram_partial(Ps, Wv, L, nv, I, J, r0, r1, Gpart + ((int64_t)pi * nchunk + ch) * (J2 * J2));
+  double* out = Gpart + ((int64_t)pi * nchunk + ch) * (J2 * J2);
+  pair_gram_rows(pg, Wv + r0, L, (int)min(L - r0, (int64_t)GCH), nv, I, J,
+                 [&](int r, int c, double v) { out[r * J2 + c] = v; });
 }
 
 // Pair eigensolve + apply, grid pairs x (row chunks of Wv, then of Z):
@@ -717,7 +670,7 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
     for (int s = 0; s < nblk - 1; ++s) {
       {
         ProfScope p(PROF_JAC_GRAM, st, gram_fl, 8.0 * (double)L * J2 * npairs);
-        hipLaunchKernelGGL(jac_gram, dim3(npairs, nchG), dim3(256), 0, st, Wv, L, k, s, nblk,
+        hipLaunchKernelGGL(jac_gram, dim3(npairs, nchG), dim3(EIG_NT), 0, st, Wv, L, k, s, nblk,
                            nchG, w.Gpart);
       }
       {
