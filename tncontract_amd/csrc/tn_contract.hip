@@ -1151,7 +1151,9 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
     S = splitk_factor(M, N, K);
     while (S > 1 && (size_t)S * M * N * esz > splitk_bytes) --S;
   }
-  g.kchunk = S > 1 ? ceil_div(ceil_div(K, S), 32) * 32 : K;
+  // (whole k-tiles: of 16, or 32 for bf16)
+  const int64_t kt = prec == P_BF16X3 ? 32 : 16;
+  g.kchunk = S > 1 ? ceil_div(ceil_div(K, S), kt) * kt : K;
   if (S > 1) S = (int)ceil_div(K, g.kchunk);
   g.part = S > 1 ? splitk_ws : nullptr;
   // FP64 products with few 128 x 128 tiles and no K split (short K): 64 x 64
