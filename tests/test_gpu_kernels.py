@@ -465,3 +465,20 @@ def test_contract_few_tiles(L, m, n, k, dtype):
                         tn.Tensor(y, ["k1", "n1", "k0", "n0"]), ["k0", "k1"], ["k0", "k1"])
         z.move_indices(["m0", "m1", "n0", "n1"], 0)
         assert (np.abs(z.data.cpu().numpy().reshape(m, n) - ref) <= bound).all()
+
+
+# Permuted copies: the general gather and the tiled transpose (whole and ragged
+# tiles), element for element.
+@pytest.mark.parametrize("shape,perm", [((3, 5), (1, 0)), ((2, 3, 5, 7), (2, 0, 3, 1)),
+                                        ((5, 51, 2), (2, 1, 0)), ((509, 2, 5, 52), (1, 3, 0, 2)),
+                                        ((7, 1, 9, 2, 3, 5), (5, 1, 0, 4, 2, 3)),
+                                        ((64, 128), (1, 0)), ((65, 3, 130), (2, 1, 0)),
+                                        ((1000, 2, 700), (1, 2, 0)), ((2, 600, 5, 400), (2, 1, 3, 0))])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_permuted_copies(L, shape, perm, dtype):
+    from tncontract_amd import _lib
+    x = torch.arange(int(np.prod(shape)), dtype=dtype, device="cuda").reshape(shape)
+    y = x.permute(perm)
+    assert torch.equal(_lib.contiguous(y), y.contiguous())
+    z = x[tuple(slice(0, None, 2) for _ in shape)].permute(perm)
+    assert torch.equal(_lib.contiguous(z), z.contiguous())

@@ -56,11 +56,24 @@ __global__ void __launch_bounds__(256) permute_tiled(const T* __restrict__ src, 
   int64_t so = mode_offset(outer, ob);
   int64_t doff = mode_offset(outer_dst, ob);
   int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
-  // read: consecutive lanes along s (unit stride in src)
-  for (int r = ty; r < 64; r += 4) {
-    int64_t s = bs + tx, o = bo + r;
-    if (s < ds && o < do_) tile[r][tx] = src[so + s * dsrc_s + o * src_o];
+  // read: consecutive lanes along s (unit stride in src); all 16 loads of a
+  // thread before the first store to LDS
+  // (one load at a time paid a trip to memory each: the structured sweep's FP32
+  // copies 10.0 -> 5.5 us)
+  T v[16];
+  if (bs + 64 <= ds && bo + 64 <= do_) {
+    const T* p = src + so + (bs + tx) * dsrc_s + (bo + ty) * src_o;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = p[4 * i * src_o];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int64_t s = bs + tx, o = bo + ty + 4 * i;
+      v[i] = s < ds && o < do_ ? src[so + s * dsrc_s + o * src_o] : (T)0;
+    }
   }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) tile[ty + 4 * i][tx] = v[i];
   __syncthreads();
   // write: consecutive lanes along o (unit stride in dst)
   for (int r = ty; r < 64; r += 4) {
