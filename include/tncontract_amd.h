@@ -179,6 +179,9 @@ int tn_cholqr(const void* A, const tn_modes* a_rows, const tn_modes* a_cols, int
  * most 256, the vectors are first ordered by norm and QR-factored (Cholesky
  * QR, Householder when that does not reach orthogonality 1e-13; Householder
  * for k <= 32 of length at most 256) and the Jacobi runs on the rows of R.
+ * FP64 matrices of any finite magnitude: the vectors are scaled by a power of
+ * two where their squares would leave the range (tn_batched_svd and, for K's
+ * diagonal, tn_eigh_psd alike).
  * tol: orthogonality tolerance (<= 0 -> (vector length) * eps, as LAPACK
  * dgesvj); max_sweeps <= 0 -> 40.  *sweeps_out (host, may be NULL) receives
  * the number of sweeps used.  Returns TN_ERR_NOCONV if not converged.

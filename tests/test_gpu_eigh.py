@@ -135,3 +135,21 @@ def test_eigh_psd_scaled_by_powers_of_two(T, n, exp):
     K = A.T @ A
     u, lam = T._eigh_psd_device(dev(np.ldexp(K, exp)), 1)
     check_eig(K, u.cpu().numpy(), np.ldexp(lam.cpu().numpy(), -exp), n)
+
+
+# Magnitudes at which the factor's inner products would leave the range; the
+# power of two is exact, the eigenvalues' own rounding is below 2^-1022 only.
+@pytest.mark.parametrize("n", [17, 33, 130, 300])
+@pytest.mark.parametrize("exp", [-1000, -960, -720, -690, 690, 720, 960])
+def test_eigh_psd_at_any_magnitude(T, n, exp):
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n + 5, n))
+    K = A.T @ A
+    u, lam = T._eigh_psd_device(dev(np.ldexp(K, exp)), 1)
+    check_eig(K, u.cpu().numpy(), np.ldexp(lam.cpu().numpy(), -exp), n)
+    # rank-deficient: the vectors of the null space are orthonormal as well
+    half = A[:n // 2].T @ A[:n // 2]
+    u, lam = T._eigh_psd_device(dev(np.ldexp(half, exp)), 1)
+    u = u.cpu().numpy()
+    check_eig(half, u, np.ldexp(lam.cpu().numpy(), -exp), n // 2)
+    assert np.abs(u.T @ u - np.eye(n)).max() <= 1e-11

@@ -482,3 +482,67 @@ def test_permuted_copies(L, shape, perm, dtype):
     assert torch.equal(_lib.contiguous(y), y.contiguous())
     z = x[tuple(slice(0, None, 2) for _ in shape)].permute(perm)
     assert torch.equal(_lib.contiguous(z), z.contiguous())
+
+
+# FP64 matrices whose squared entries leave the range (2^(+-511) and beyond),
+# beside the last that need no scaling: one workgroup's sizes, vectors without
+# the preconditioning QR, one-launch and two-launch Jacobi steps, the batched
+# SVD.  The power of two is exact, so the bounds are those at 2^0 (plus the
+# rounding of singular values below 2^-1022).
+MAGNITUDES = [-1030, -530, -517, -505, -190, 190, 505, 530, 1000]
+
+
+def check_svd_at(a, u, s, vt, exp):
+    ref = np.linalg.svd(a, compute_uv=False)
+    s = np.ldexp(s, -exp)
+    assert np.abs(s - ref).max() <= (2e-13 + 2.0 ** (-1074 - exp)) * ref[0]
+    assert np.linalg.norm((u * s) @ vt - a) <= 4e-13 * ref[0] * np.sqrt(len(ref)) \
+        + 2.0 ** (-1074 - exp) * len(ref)
+    big = int(np.count_nonzero(ref > 1e-10 * ref[0]))
+    assert np.abs(u[:, :big].T @ u[:, :big] - np.eye(big)).max() <= 4e-13
+    assert np.abs(vt[:big] @ vt[:big].T - np.eye(big)).max() <= 4e-13
+
+
+@pytest.mark.parametrize("exp", MAGNITUDES)
+@pytest.mark.parametrize("m,n", [(24, 16), (32, 256), (300, 20), (40, 70), (130, 129), (300, 290)])
+def test_svd_at_any_magnitude(L, m, n, exp):
+    from tncontract_amd import tensor as T
+    from tncontract_amd.batched import batched_svd
+    rng = np.random.default_rng(m + n)
+    low = rng.standard_normal((m, 7)) @ rng.standard_normal((7, n))
+    sparse = low * (rng.random(n) < 0.5)
+    one = rng.standard_normal((20, 30))
+    for g in (rng.standard_normal((m, n)), low, sparse):
+        x = np.ldexp(g, exp)
+        a = np.ldexp(x, -exp)  # (what is left of g in subnormals)
+        u, s, vt = (t.cpu().numpy() for t in T._svd_device(dev(x), 1))
+        check_svd_at(a, u, s, vt, exp)
+        if g is not sparse:  # each job of a batch has its own scale
+            U, S, Vt, _ = batched_svd([dev(x), dev(one)])
+            check_svd_at(a, U[0].cpu().numpy(), S[0].cpu().numpy(), Vt[0].cpu().numpy(), exp)
+            check_svd_at(one, U[1].cpu().numpy(), S[1].cpu().numpy(), Vt[1].cpu().numpy(), 0)
+
+
+@pytest.mark.parametrize("m,n", [(24, 16), (300, 20), (100, 100)])
+@pytest.mark.parametrize("big", [1e200, 1e-200])
+def test_svd_with_one_large_entry(L, m, n, big):
+    from tncontract_amd import tensor as T
+    a = np.random.default_rng(m).standard_normal((m, n)) * min(big, 1.0)
+    a[m // 2, n // 3] = big * 1e3
+    u, s, vt = (t.cpu().numpy() for t in T._svd_device(dev(a), 1))
+    check_svd_at(a / big, u, s / big, vt, 0)
+
+
+@pytest.mark.parametrize("scale", [1e-150, 1e-300, 1e150])
+def test_svd_of_shrinking_columns_at_any_magnitude(L, scale):
+    from tncontract_amd import tensor as T
+    from tncontract_amd.batched import batched_svd
+    for m, n in [(64, 32), (40, 64), (200, 64), (31, 20)]:
+        a = np.zeros((m, n))
+        a[-1] = np.random.default_rng(m + n).standard_normal(n)
+        for u, s, vt in (T._svd_device(dev(a * scale), 1),
+                         [x[0] for x in batched_svd([dev(a * scale)])[:3]]):
+            u, s, vt = (x.cpu().numpy() for x in (u, s, vt))
+            s = s / scale
+            assert abs(s[0] - np.linalg.norm(a)) <= 1e-13 * s[0]
+            assert np.abs((u * s) @ vt - a).max() <= 1e-13 * s[0]

@@ -557,17 +557,42 @@ struct AJob {
   int64_t x;  // offset of the job's vector matrix (L x k) in the vector buffer
 };
 
+// codes[j] raised to the largest entry code of job j's matrix.
+__global__ void __launch_bounds__(256) bcodes_f64(const AJob* __restrict__ ajobs,
+                                                  const OJob* __restrict__ outs,
+                                                  int* __restrict__ codes) {
+  const int j = blockIdx.y;
+  const int64_t tot = (int64_t)outs[j].m * outs[j].n;
+  const double* A = ajobs[j].A;
+  __shared__ int tops[4];
+  int top = 0;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < tot; e += (int64_t)gridDim.x * 256)
+    top = max(top, entry_code(A[e]));
+  top = (int)wave_max((float)top);
+  if ((threadIdx.x & 63) == 0) tops[threadIdx.x >> 6] = top;
+  __syncthreads();
+  // one atomic a block, and none where the value is that high already (the
+  // jobs' codes share cache lines: with one a wave, 63 jobs of 128 x 128 took 41 us)
+  if (threadIdx.x == 0) {
+    top = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
+    if (top > __hip_atomic_load(codes + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(codes + j, top);
+  }
+}
+
+// ... scaled by the power of two of its largest entry code.
 __global__ void bgather_f64(double* __restrict__ Wv, const AJob* __restrict__ ajobs,
-                            const OJob* __restrict__ outs) {
+                            const OJob* __restrict__ outs, const int* __restrict__ codes) {
   const int j = blockIdx.y;
   const OJob O = outs[j];
   const double* A = ajobs[j].A;
   const int64_t L = O.tall ? O.m : O.n, k = O.tall ? O.n : O.m;
   const int64_t tot = L * k;
+  const int scale = -code_scale(codes[j]);
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < tot;
        e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t v = e / L, i = e - v * L;
-    Wv[ajobs[j].x + e] = O.tall ? A[i * O.n + v] : A[v * O.n + i];
+    Wv[ajobs[j].x + e] = __builtin_amdgcn_ldexp(O.tall ? A[i * O.n + v] : A[v * O.n + i], scale);
   }
 }
 
@@ -576,10 +601,12 @@ __global__ void bgather_f64(double* __restrict__ Wv, const AJob* __restrict__ aj
 // Z.  QR-preconditioned jobs (X = Q R, Jacobi on the rows of R): U_X = Q Z
 // (O.qz, columns c < kept in sorted order; zero beyond), V_X = the rotated
 // rows of R / S.  Tall: U = U_X, V^T = V_X^T; wide: U = V_X, V^T = U_X^T.
+// S is that of the scaled vectors, O.S the matrix's (code 0: not scaled).
 __global__ void bout(const double* __restrict__ Wv, const double* __restrict__ Zb,
                      const BJob* __restrict__ jobs, const OJob* __restrict__ outs,
                      const int64_t* __restrict__ sbase, const int* __restrict__ perm,
-                     const double* __restrict__ Ss, const int* __restrict__ kept) {
+                     const double* __restrict__ Ss, const int* __restrict__ kept,
+                     const int* __restrict__ codes) {
   const int j = blockIdx.y;
   const BJob J = jobs[j];
   const OJob O = outs[j];
@@ -588,6 +615,7 @@ __global__ void bout(const double* __restrict__ Wv, const double* __restrict__ Z
   const int64_t tot = (int64_t)O.m * k + k * O.n;
   const int* pm = perm + sbase[j];
   const double* S = Ss + sbase[j];
+  const int up = code_scale(codes[j]);
   if (O.qz) {
     const int64_t L = O.tall ? O.m : O.n, kp = kept[j];
     for (; idx < tot; idx += (int64_t)gridDim.x * blockDim.x) {
@@ -608,7 +636,8 @@ __global__ void bout(const double* __restrict__ Wv, const double* __restrict__ Z
       }
     }
     if (blockIdx.x == 0)
-      for (int64_t c = threadIdx.x; c < k; c += blockDim.x) O.S[c] = S[c];
+      for (int64_t c = threadIdx.x; c < k; c += blockDim.x)
+        O.S[c] = __builtin_amdgcn_ldexp(S[c], up);
     return;
   }
   for (; idx < tot; idx += (int64_t)gridDim.x * blockDim.x) {
@@ -630,7 +659,7 @@ __global__ void bout(const double* __restrict__ Wv, const double* __restrict__ Z
     }
   }
   if (blockIdx.x == 0)
-    for (int64_t c = threadIdx.x; c < k; c += blockDim.x) O.S[c] = S[c];
+    for (int64_t c = threadIdx.x; c < k; c += blockDim.x) O.S[c] = __builtin_amdgcn_ldexp(S[c], up);
 }
 
 // ---------------------------------------------------------------- autotune
@@ -742,7 +771,7 @@ static size_t batched_ws_bytes(const std::vector<int64_t>& ms, const std::vector
   a.take<GJob>((size_t)njobs);
   a.take<AJob>((size_t)njobs);
   a.take<int>((size_t)njobs * 2);  // tile base + ids
-  a.take<int>((size_t)njobs * 4);  // done, sweeps, kept, active
+  a.take<int>((size_t)njobs * 5);  // done, sweeps, codes, kept, active
   a.take<unsigned long long>((size_t)njobs * 3);
   a.take<unsigned long long>(3);  // work counters
   a.take<double>(sv * 2);
@@ -910,8 +939,9 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   AJob* daj = a.take<AJob>((size_t)njobs);
   int* dtile = a.take<int>((size_t)njobs);
   int* dids = a.take<int>((size_t)njobs);
-  int* ddone = a.take<int>((size_t)njobs);
-  int* dsweeps = a.take<int>((size_t)njobs);
+  int* ddone = a.take<int>((size_t)njobs * 3);
+  int* dsweeps = ddone + njobs;
+  int* dcodes = ddone + 2 * (size_t)njobs;
   int* dkept = a.take<int>((size_t)njobs);
   int* dactive = a.take<int>((size_t)njobs);
   unsigned long long* doff = a.take<unsigned long long>((size_t)njobs * 3);
@@ -946,8 +976,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     TN_HIP(hipMemcpyAsync(dapply, apply_items.data(), sizeof(QItem) * apply_items.size(),
                           hipMemcpyHostToDevice, st));
   }
-  TN_HIP(hipMemsetAsync(ddone, 0, sizeof(int) * njobs, st));
-  TN_HIP(hipMemsetAsync(dsweeps, 0, sizeof(int) * njobs, st));
+  TN_HIP(hipMemsetAsync(ddone, 0, sizeof(int) * 3 * njobs, st));  // done, sweeps, codes
   TN_HIP(hipMemsetAsync(doff, 0, sizeof(unsigned long long) * njobs * 3, st));
   // rows through the Gram and rotation kernels and eigensolves that rotated,
   // counted only while launch timing is on (they give the Jacobi rooflines)
@@ -961,8 +990,11 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   if (sj) {
     int64_t maxe = 1;
     for (int j = 0; j < njobs; ++j) maxe = std::max<int64_t>(maxe, ms[j] * ns[j]);
+    // (the products of FP32 factors never need a scale)
+    hipLaunchKernelGGL(bcodes_f64, dim3((unsigned)std::min<int64_t>(ceil_div(maxe, 1024), 64), njobs),
+                       dim3(256), 0, st, daj, doj, dcodes);
     hipLaunchKernelGGL(bgather_f64, dim3((unsigned)std::min<int64_t>(ceil_div(maxe, 256), 4096), njobs),
-                       dim3(256), 0, st, dWv, daj, doj);
+                       dim3(256), 0, st, dWv, daj, doj, dcodes);
     TN_CHECK_LAUNCH();
   } else {
     std::vector<int> byb[4];
@@ -1161,7 +1193,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     }
   }
   hipLaunchKernelGGL(bout, dim3(256, njobs), dim3(256), 0, st, dWv, dZ, dbj, doj, dsbase, dperm, dS,
-                     dkept);
+                     dkept, dcodes);
   TN_CHECK_LAUNCH();
   std::vector<int> done(njobs);
   if (kept_out)

@@ -54,6 +54,24 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Scale of a matrix whose vectors meet the Jacobi.  Squared norms and inner
+// products of entries around 2^(+-500) leave FP64's range: the norms are then
+// lost, and pair_rotates' lower limits would leave pairs alone whose vectors
+// are as long as any other.  The vectors are therefore multiplied by the power
+// of two that brings their largest entry to [0.5, 1) when its exponent is
+// beyond a limit (kScaleExp for matrices whose entries are squared), and the
+// singular values by its inverse: exact, and everything within the limit keeps
+// its bits.  Codes: entry_code(x) = exponent + 2048, 0 for what has none (0,
+// inf, NaN); code_scale(largest code) = the exponent to take out.
+constexpr int kScaleExp = 200;
+__device__ __forceinline__ int entry_code(double x) {
+  return x != 0.0 && fabs(x) < INFINITY ? __builtin_amdgcn_frexp_exp(x) + 2048 : 0;
+}
+__device__ __forceinline__ int code_scale(int code, int limit = kScaleExp) {
+  const int e = code - 2048;
+  return code == 0 || abs(e) <= limit ? 0 : e;
+}
+
 constexpr int EIG_NT = 512;  // threads of a pair eigensolve (8 waves)
 constexpr int EIG_NW = EIG_NT / 64;
 constexpr int GPAD = 2;      // G row padding: rows stay 16-byte aligned
@@ -99,7 +117,9 @@ __device__ __forceinline__ void pair_scaled(double gpq, double gpp, double gqq, 
 // norm is lost and its product with the other is not, so the pair would be
 // rotated without end (the rounding that a sparse low-rank matrix leaves can
 // shrink by 1e-16 from vector to vector, down to there); nor is a pair whose
-// inner product is lost in its terms' underflow.
+// inner product is lost in its terms' underflow.  The limits are absolute: the
+// callers scale the vectors (code_scale), so they lie far below the rounding of
+// the longest one.
 constexpr double kNormMin = 0x1p-1018, kNormRatio = 0x1p-80, kDotMin = 0x1p-1060;
 __device__ __forceinline__ bool pair_rotates(double gpq, double gpp, double gqq, double tol,
                                              double neg2, double& spq, double& spp, double& sqq) {

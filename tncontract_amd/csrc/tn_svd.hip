@@ -203,7 +203,8 @@ __global__ void __launch_bounds__(EIG_NT) jac_step(const double* __restrict__ Wi
 // QR = false: one-sided Jacobi of the vectors in Wv (in place).  QR = true,
 // the preconditioned SVD: the vectors by descending norm (order in vp),
 // X' = Q R by Householder's method, Jacobi on the rows of R (rotated rows to
-// R, vector-contiguous) and Q Z to QZ.  info = {sweeps, converged}.
+// R, vector-contiguous) and Q Z to QZ; the vectors scaled as they are read
+// (code_scale).  info = {sweeps, converged, largest entry code}.
 constexpr int kSmallLen = 256;
 
 // NaN ranks as -inf so that ranks stay a permutation of 0..k-1.
@@ -231,11 +232,24 @@ __global__ void __launch_bounds__(EIG_NT) jac_small(double* __restrict__ Wv, int
     lds_barrier();
   } else {
     double x[NI];
-    double s2 = 0.0;
+    int code = 0;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int r = l + 16 * i;
       x[i] = (q < k && r < L) ? Wv[(int64_t)q * L + r] : 0.0;
+      code = max(code, entry_code(x[i]));
+    }
+    code = (int)wave_max_dpp((float)code);
+    if (lane == 0) sm.red[wave] = (float)code;
+    lds_barrier();
+#pragma unroll
+    for (int w = 0; w < EIG_NW; ++w) code = max(code, (int)sm.red[w]);
+    if (tid == 0) info[2] = code;
+    const int scale = -code_scale(code);
+    double s2 = 0.0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      x[i] = __builtin_amdgcn_ldexp(x[i], scale);
       s2 = fma(x[i], x[i], s2);
     }
     s2 = row16_sum(s2);
@@ -444,16 +458,19 @@ static void launch_rank_sort(const double* sig, int64_t k, int* perm, double* S,
 // a "scaled" source holds sigma_j * (unit vector) and is divided by S[j].
 // upm / vpm (nullable): component i of a U source vector is row upm[i] of U,
 // component c of a V source vector is column vpm[c] of Vt (the pivot order
-// of the preconditioned path).
+// of the preconditioned path).  S is that of the scaled vectors; Sout gets the
+// matrix's (code: the vectors' largest entry code, null if they were not scaled).
 template <typename T>
 __global__ void svd_out_kernel(const double* __restrict__ Uvec, int64_t ldu, int u_scaled,
                                const double* __restrict__ Vvec, int64_t ldv, int v_scaled,
                                int64_t k, const int* __restrict__ perm,
                                const double* __restrict__ S, const int* __restrict__ upm,
                                const int* __restrict__ vpm, T* __restrict__ U,
-                               T* __restrict__ Vt, int64_t m, int64_t n) {
+                               T* __restrict__ Vt, int64_t m, int64_t n,
+                               const int* __restrict__ code, double* __restrict__ Sout) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= m * k + k * n) return;
+  if (idx < k) Sout[idx] = code ? __builtin_amdgcn_ldexp(S[idx], code_scale(*code)) : S[idx];
   if (idx < m * k) {
     int64_t i = idx / k, j = idx - i * k;
     double v = Uvec[(int64_t)perm[j] * ldu + i];
@@ -489,17 +506,37 @@ __global__ void r_rows_kernel(const double* __restrict__ W, int64_t L, int64_t k
   V[idx] = c >= j ? W[j + c * L] : 0.0;
 }
 
+// code (may be null): raised to the largest entry code.
 template <typename T>
 __global__ void gather_vectors(const T* __restrict__ src, Modes rows, Modes cols, int64_t m,
-                               int64_t n, int tall, double* __restrict__ Wv) {
+                               int64_t n, int tall, double* __restrict__ Wv, int* code) {
   // tall: Wv[j*m + i] = A(i,j)   wide: Wv[i*n + j] = A(i,j)
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  int top = 0;
   for (; idx < m * n; idx += stride) {
     int64_t i, j;
     if (tall) { j = idx / m; i = idx - j * m; } else { i = idx / n; j = idx - i * n; }
-    Wv[idx] = (double)src[mode_offset(rows, i) + mode_offset(cols, j)];
+    const double x = (double)src[mode_offset(rows, i) + mode_offset(cols, j)];
+    Wv[idx] = x;
+    top = max(top, entry_code(x));
   }
+  if (code == nullptr) return;
+  top = (int)wave_max((float)top);
+  // (few waves find the value they read still below theirs)
+  if ((threadIdx.x & 63) == 0 && top > __hip_atomic_load(code, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(code, top);
+}
+
+// The vectors times the power of two of their largest entry code (nothing to
+// do for most).
+__global__ void __launch_bounds__(256) scale_vectors(double* __restrict__ Wv, int64_t n,
+                                                     const int* __restrict__ code) {
+  const int e = code_scale(*code);
+  if (e == 0) return;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+    Wv[i] = __builtin_amdgcn_ldexp(Wv[i], -e);
 }
 
 __global__ void reset_u64(unsigned long long* p) { p[threadIdx.x] = 0ull; }
@@ -514,6 +551,7 @@ struct SvdWs {
   double *Wv, *Z, *Gpart, *sig, *S, *R, *QZ, *Rtmp;
   int *perm, *vp;
   unsigned long long* off;
+  int* code;  // largest entry code of the vectors
   QrWs qr;
   char* cq;  // Cholesky QR workspace
   size_t cq_bytes;
@@ -557,7 +595,8 @@ static size_t svd_layout(int64_t m, int64_t n, char* base, size_t cap, SvdWs* ou
   w.sig = a.take<double>((size_t)k);
   w.S = a.take<double>((size_t)k);
   w.perm = a.take<int>((size_t)k);
-  w.off = a.take<unsigned long long>(4);
+  w.off = a.take<unsigned long long>(5);
+  w.code = (int*)(w.off + 4);
   if (w.precond) {
     w.R = a.take<double>((size_t)(k * k));
     w.Rtmp = a.take<double>((size_t)(k * k));
@@ -812,14 +851,21 @@ static int svd_impl(const void* A, const tn_modes* a_rows, const tn_modes* a_col
   SvdWs w{};
   svd_layout(m, n, (char*)ws, ws_bytes, &w);
   const int tall = m >= n ? 1 : 0;
-  // X (L x k, column-major) holds the vectors: columns of A (tall) or rows (wide)
+  // X (L x k, column-major) holds the vectors: columns of A (tall) or rows (wide),
+  // scaled (FP32 entries never need it; jac_small does it itself)
+  const bool scaled = dtype == TN_F64 && !(w.precond && small_jacobi(L, k));
+  const int* code = scaled ? w.code : nullptr;
   unsigned gb = (unsigned)std::min<int64_t>(ceil_div(m * n, 256), 65536);
+  if (scaled) hipLaunchKernelGGL(reset_u64, dim3(1), dim3(1), 0, st, w.off + 4);
   if (dtype == TN_F64)
     hipLaunchKernelGGL(gather_vectors<double>, dim3(gb), dim3(256), 0, st, (const double*)A, rows,
-                       cols, m, n, tall, w.Wv);
+                       cols, m, n, tall, w.Wv, scaled ? w.code : nullptr);
   else
     hipLaunchKernelGGL(gather_vectors<float>, dim3(gb), dim3(256), 0, st, (const float*)A, rows,
-                       cols, m, n, tall, w.Wv);
+                       cols, m, n, tall, w.Wv, (int*)nullptr);
+  if (scaled)
+    hipLaunchKernelGGL(scale_vectors, dim3(std::min(gb, 1024u)), dim3(256), 0, st, w.Wv, m * n,
+                       w.code);
   TN_CHECK_LAUNCH();
   bool converged = false;
   const double* Uvec;
@@ -836,6 +882,7 @@ static int svd_impl(const void* A, const tn_modes* a_rows, const tn_modes* a_col
                        max_sweeps, w.R, w.QZ, w.vp, (int*)w.off);
     TN_CHECK_LAUNCH();
     TN_TRY(small_outcome((int*)w.off, sweeps_out, &converged, st));
+    code = (const int*)w.off + 2;
     orth_src = w.R;
     orth_len = k;
     if (tall) { Uvec = w.QZ; ldu = L; u_scaled = 0; Vvec = w.R; ldv = k; v_scaled = 1; vpm = w.vp; }
@@ -895,17 +942,17 @@ static int svd_impl(const void* A, const tn_modes* a_rows, const tn_modes* a_col
     else { Uvec = w.Z; ldu = k; u_scaled = 0; Vvec = w.Wv; ldv = L; v_scaled = 1; }
   }
   hipLaunchKernelGGL(vec_norms, dim3((unsigned)k), dim3(256), 0, st, orth_src, orth_len, w.sig);
-  launch_rank_sort(w.sig, k, w.perm, S, st);
+  launch_rank_sort(w.sig, k, w.perm, w.S, st);
   TN_CHECK_LAUNCH();
   unsigned ob = (unsigned)ceil_div(m * k + k * n, 256);
   if (dtype == TN_F64)
     hipLaunchKernelGGL(svd_out_kernel<double>, dim3(ob), dim3(256), 0, st, Uvec, ldu, u_scaled,
-                       Vvec, ldv, v_scaled, k, w.perm, S, upm, vpm, (double*)U, (double*)Vt, m,
-                       n);
+                       Vvec, ldv, v_scaled, k, w.perm, w.S, upm, vpm, (double*)U, (double*)Vt, m,
+                       n, code, S);
   else
     hipLaunchKernelGGL(svd_out_kernel<float>, dim3(ob), dim3(256), 0, st, Uvec, ldu, u_scaled,
-                       Vvec, ldv, v_scaled, k, w.perm, S, upm, vpm, (float*)U, (float*)Vt, m,
-                       n);
+                       Vvec, ldv, v_scaled, k, w.perm, w.S, upm, vpm, (float*)U, (float*)Vt, m,
+                       n, code, S);
   TN_CHECK_LAUNCH();
   if (!converged) {
     set_error(TN_ERR_NOCONV, "tn_svd: Jacobi did not converge in %d sweeps", max_sweeps);
@@ -1001,17 +1048,35 @@ namespace tn {
 
 constexpr int CB = 64;  // Cholesky block
 
-// diag[j] = A[j][j]; delta = 8 sqrt(n) eps_in sum_j |A[j][j]|
+// The matrix is scaled like the SVD's vectors, past an exponent at which its
+// factor's squared norms (its own entries, times eps for the shifted ones) would
+// near FP64's limits.
+constexpr int kPsdScaleExp = 700;
+
+// diag[j] = A[j][j]; *code = the largest of its entry codes (a positive
+// semi-definite matrix has no larger entry); of the scaled matrix delta = 8
+// sqrt(n) eps_in sum_j |A[j][j]|
 __global__ void __launch_bounds__(256) psd_diag(const double* __restrict__ A, int64_t n,
                                                 double eps_in, double* __restrict__ diag,
-                                                double* __restrict__ delta) {
+                                                double* __restrict__ delta,
+                                                int* __restrict__ code) {
   __shared__ double red[4];
-  double acc = 0.0;
+  __shared__ int top[4];
+  int mine = 0;
   for (int64_t j = threadIdx.x; j < n; j += 256) {
     const double v = A[j * n + j];
     diag[j] = v;
-    acc += fabs(v);
+    mine = max(mine, entry_code(v));
   }
+  mine = (int)wave_max((float)mine);
+  if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = mine;
+  __syncthreads();
+  mine = max(max(top[0], top[1]), max(top[2], top[3]));
+  if (threadIdx.x == 0) *code = mine;
+  const int e = code_scale(mine, kPsdScaleExp);
+  double acc = 0.0;
+  for (int64_t j = threadIdx.x; j < n; j += 256)
+    acc += fabs(__builtin_amdgcn_ldexp(diag[j], -e));  // (this thread's own store)
   acc = wave_sum(acc);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
@@ -1019,31 +1084,34 @@ __global__ void __launch_bounds__(256) psd_diag(const double* __restrict__ A, in
     *delta = 8.0 * sqrt((double)n) * eps_in * (red[0] + red[1] + red[2] + red[3]);
 }
 
-// B[c][r] = sym(A)[p[c]][p[r]] + delta [r == c]   (column-major, ld n);
+// B[c][r] = sym(A)[p[c]][p[r]] + delta [r == c]   (column-major, ld n), A scaled;
 // the symmetric part, since a K formed by rounded products is symmetric only
 // to rounding
 __global__ void psd_permute(const double* __restrict__ A, int64_t n, const int* __restrict__ p,
-                            const double* __restrict__ delta, double* __restrict__ B) {
+                            const double* __restrict__ delta, const int* __restrict__ code,
+                            double* __restrict__ B) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= n * n) return;
   const int64_t c = idx / n, r = idx - c * n;
   const int64_t pc = p[c], pr = p[r];
-  double v = 0.5 * (A[pc * n + pr] + A[pr * n + pc]);
+  const int e = code_scale(*code, kPsdScaleExp);
+  double v = 0.5 * (__builtin_amdgcn_ldexp(A[pc * n + pr], -e) +
+                    __builtin_amdgcn_ldexp(A[pr * n + pc], -e));
   if (r == c) v += *delta;
   B[idx] = v;
 }
 
-// U[p[i]][j] = Wv[perm[j]][i] / S[j];  lam[j] = S[j]^2 - delta
+// U[p[i]][j] = Wv[perm[j]][i] / S[j];  lam[j] = S[j]^2 - delta, unscaled
 __global__ void eig_out_kernel(const double* __restrict__ Wv, int64_t n, const int* __restrict__ p,
                                const int* __restrict__ perm, const double* __restrict__ S,
-                               const double* __restrict__ delta, double* __restrict__ U,
-                               double* __restrict__ lam) {
+                               const double* __restrict__ delta, const int* __restrict__ code,
+                               double* __restrict__ U, double* __restrict__ lam) {
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= n * n) return;
   const int64_t i = idx / n, j = idx - i * n;
   const double s = S[j];
   U[(int64_t)p[i] * n + j] = s > 0.0 ? Wv[(int64_t)perm[j] * n + i] / s : 0.0;
-  if (i == 0) lam[j] = s * s - *delta;
+  if (i == 0) lam[j] = __builtin_amdgcn_ldexp(s * s - *delta, code_scale(*code, kPsdScaleExp));
 }
 
 struct EigWs {
@@ -1069,7 +1137,8 @@ static size_t eig_layout(int64_t n, char* base, size_t cap, EigWs* out) {
   e.jw.sig = a.take<double>((size_t)n);
   e.jw.S = a.take<double>((size_t)n);
   e.jw.perm = a.take<int>((size_t)n);
-  e.jw.off = a.take<unsigned long long>(4);
+  e.jw.off = a.take<unsigned long long>(5);
+  e.jw.code = (int*)(e.jw.off + 4);
   if (out) *out = e;
   return a.used;
 }
@@ -1103,17 +1172,19 @@ extern "C" int tn_eigh_psd(const void* K, const tn_modes* k_rows, const tn_modes
   unsigned gb = (unsigned)std::min<int64_t>(ceil_div(n * n, 256), 65536);
   if (dtype == TN_F64)
     hipLaunchKernelGGL(gather_vectors<double>, dim3(gb), dim3(256), 0, st, (const double*)K, rows,
-                       cols, n, n, 1, Wv);
+                       cols, n, n, 1, Wv, (int*)nullptr);
   else
     hipLaunchKernelGGL(gather_vectors<float>, dim3(gb), dim3(256), 0, st, (const float*)K, rows,
-                       cols, n, n, 1, Wv);
+                       cols, n, n, 1, Wv, (int*)nullptr);
   // shift allowance from the input's precision (K formed in FP32 is
   // indefinite at ~eps_32 |K|)
   const double eps_in = dtype == TN_F64 ? 2.220446049250313e-16 : 1.1920928955078125e-07;
-  hipLaunchKernelGGL(psd_diag, dim3(1), dim3(256), 0, st, Wv, n, eps_in, e.diag, e.delta);
+  hipLaunchKernelGGL(psd_diag, dim3(1), dim3(256), 0, st, Wv, n, eps_in, e.diag, e.delta,
+                     e.jw.code);
   launch_rank_sort(e.diag, n, e.p, e.Sd, st);
   const unsigned nb = (unsigned)ceil_div(n * n, 256);
-  hipLaunchKernelGGL(psd_permute, dim3(nb), dim3(256), 0, st, Wv, n, e.p, e.delta, e.B);
+  hipLaunchKernelGGL(psd_permute, dim3(nb), dim3(256), 0, st, Wv, n, e.p, e.delta, e.jw.code,
+                     e.B);
   TN_CHECK_LAUNCH();
   TN_HIP(hipMemsetAsync(Wv, 0, sizeof(double) * (size_t)(n * n), st));
   // 2. blocked Cholesky: B (working copy) -> L in Wv
@@ -1142,7 +1213,7 @@ extern "C" int tn_eigh_psd(const void* K, const tn_modes* k_rows, const tn_modes
   hipLaunchKernelGGL(vec_norms, dim3((unsigned)n), dim3(256), 0, st, Wv, n, e.jw.sig);
   launch_rank_sort(e.jw.sig, n, e.jw.perm, e.jw.S, st);
   hipLaunchKernelGGL(eig_out_kernel, dim3(nb), dim3(256), 0, st, Wv, n, e.p, e.jw.perm, e.jw.S,
-                     e.delta, U, lam);
+                     e.delta, e.jw.code, U, lam);
   TN_CHECK_LAUNCH();
   if (!converged) {
     set_error(TN_ERR_NOCONV, "tn_eigh_psd: Jacobi did not converge in %d sweeps", max_sweeps);
