@@ -546,3 +546,23 @@ def test_svd_of_shrinking_columns_at_any_magnitude(L, scale):
             s = s / scale
             assert abs(s[0] - np.linalg.norm(a)) <= 1e-13 * s[0]
             assert np.abs((u * s) @ vt - a).max() <= 1e-13 * s[0]
+
+
+# Blocks that pass the tests of the orthonormal-factor path although two of
+# their columns are nearly dependent on others (smallest singular value about
+# 1 / c): the factorisation is backward stable column by column all the same.
+@pytest.mark.parametrize("m,n", [(256, 64), (1280, 64), (1280, 200)])
+@pytest.mark.parametrize("c", [1, 30, 100, 300, 1000, 3000])
+def test_qr_of_nearly_dependent_columns(L, m, n, c):
+    from tncontract_amd import tensor as T
+    for seed in range(3):
+        rng = np.random.default_rng(1000 * seed + c)
+        a = rng.standard_normal((m, n))
+        for j in range(10, n, 64):
+            w = rng.standard_normal(m)
+            a[:, j] = a[:, j - 10:j] @ (rng.standard_normal(10) / 10) + w / c
+            a[:, j + 1] = w + 0.3 * rng.standard_normal(m)
+        q, r = (x.cpu().numpy() for x in T._qr_device(dev(a), 1))
+        assert np.abs(q.T @ q - np.eye(n)).max() <= 1e-13
+        res = np.linalg.norm(q @ r - a, axis=0) / np.linalg.norm(a, axis=0)
+        assert res.max() <= 1e-14

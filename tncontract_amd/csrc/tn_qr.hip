@@ -705,14 +705,15 @@ static int hr_block(double* P, int64_t mr, int64_t ld, double* V, double* T, con
   hipLaunchKernelGGL(hr_scale, dim3(16), dim3(256), 0, st, h.part, nc, h.G, h.d, h.delta, h.bad);
   TN_CHECK_LAUNCH();
   TN_TRY(chol_block(h.G, HB, 0, HB, h.delta, h.F, h.X, st, h.bad));
-  hipLaunchKernelGGL(hr_apply, dim3((unsigned)ceil_div(mr, HROWS)), dim3(256), 0, st, P, mr, ld,
-                     h.X, h.d, V, mr, (double*)nullptr, (int64_t)0, h.bad);
+  hipLaunchKernelGGL(hr_apply<true>, dim3((unsigned)ceil_div(mr, HROWS)), dim3(256), 0, st, P, mr,
+                     ld, h.X, h.F, h.d, V, mr, (double*)nullptr, (int64_t)0, h.bad);
   hipLaunchKernelGGL(hr_gram, dim3(nc), dim3(256), 0, st, V, mr, mr, nc, h.part, h.bad, 0);
   hipLaunchKernelGGL(hr_gram_sum, dim3(16), dim3(256), 0, st, h.part, nc, h.G, h.bad, 0);
   hipLaunchKernelGGL(hr_reflect, dim3(1), dim3(512), 0, st, h.G, h.F, h.d, V, mr, P, ld, h.M, T,
                      h.bad);
-  hipLaunchKernelGGL(hr_apply, dim3((unsigned)ceil_div(mr - HB, HROWS)), dim3(256), 0, st, V + HB,
-                     mr - HB, mr, h.M, (const double*)nullptr, V + HB, mr, P + HB, ld, h.bad);
+  hipLaunchKernelGGL(hr_apply<false>, dim3((unsigned)ceil_div(mr - HB, HROWS)), dim3(256), 0, st,
+                     V + HB, mr - HB, mr, h.M, (const double*)nullptr, (const double*)nullptr, V + HB,
+                     mr, P + HB, ld, h.bad);
   TN_CHECK_LAUNCH();
   return TN_OK;
 }

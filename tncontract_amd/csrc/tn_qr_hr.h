@@ -9,7 +9,10 @@
 // matrix cores idle meanwhile.  Here the columns' long dimension only meets
 // 64 x 64 matrices:
 //   1. G = (P D)^T (P D) over row chunks (D: powers of two that bring the
-//      columns' norms to [1, 2)), G = L L^T, Q1 = P D L^{-T};
+//      columns' norms to [1, 2)), G = L L^T, Q1 = P D L^{-T} by the inverse X of
+//      L and one step of refinement, Q1 += (P D - Q1 L^T) X^T: the inverse alone
+//      leaves P D - Q1 L^T at cond(P D) eps (up to 2e-13 of a column's norm for
+//      blocks that pass below), the refined one at rounding;
 //   2. E = Q1^T Q1 - I (about cond(P D)^2 eps), N = its strict upper triangle
 //      plus half its diagonal: Q = Q1 (I - N) is orthonormal and
 //      P = Q R, R = (I + N) L^T D^{-1}, to O(|E|^2);
@@ -150,21 +153,28 @@ __global__ void __launch_bounds__(256) hr_scale(const double* __restrict__ part,
   if (e == 0) *delta = 2e-8;
 }
 
-// Out (rows x 64) = In (rows x 64) B, both column-major; B[i][c] = d_i
-// B0[i * 64 + c] (d may be null).  Out2 (null or a second copy, ld2).  Each
+// Out (rows x 64) = In (rows x 64) B, both column-major; B[i][c] =
+// B0[i * 64 + c].  Out2 (null or a second copy, ld2).  Each
 // wave 16 rows, as the transposed product (B^T In^T): In is read and Out
 // written straight from and to memory, 128 bytes of a column at a time (more
 // and shorter workgroups measured better: 64 rows 9 us against 128 rows 13.8
 // us at 5120 rows).  In
 // and Out may be the same array (a row is read before it is written, by the
 // wave that writes it).
+// SOLVE: Out = (In D) L^{-T} with B0 = X^T, X = L^{-1}, and one step of
+// refinement against L (F: its lower triangle, column-major; D = diag(d)).  A
+// product comes out in the layout of its operand, so the three of them chain in
+// registers.
+template <bool SOLVE>
 __global__ void __launch_bounds__(256) hr_apply(const double* In, int64_t rows, int64_t ldi,
                                                 const double* __restrict__ B0,
+                                                const double* __restrict__ F,
                                                 const double* __restrict__ d, double* Out,
                                                 int64_t ldo, double* __restrict__ Out2,
                                                 int64_t ld2, const int* __restrict__ bad) {
   if (*bad) return;
   __shared__ double Bs[HB][HB + 1];
+  __shared__ double Ls[SOLVE ? HB : 1][HB + 1];  // L^T
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const int64_t r = (int64_t)blockIdx.x * HROWS + 16 * wave + lr;
   double x[16];
@@ -172,27 +182,56 @@ __global__ void __launch_bounds__(256) hr_apply(const double* In, int64_t rows, 
   for (int k = 0; k < 16; ++k) x[k] = r < rows ? In[(int64_t)(4 * k + lk) * ldi + r] : 0.0;
   {
     // (every load of B before the first LDS store)
-    double v[HB * HB / 256];
+    constexpr int PER = HB * HB / 256;
+    double v[PER], f[SOLVE ? PER : 1];
 #pragma unroll
-    for (int k = 0; k < HB * HB / 256; ++k) {
+    for (int k = 0; k < PER; ++k) {
       const int e = threadIdx.x + 256 * k;
-      v[k] = d ? d[e >> 6] * B0[e] : B0[e];
+      v[k] = B0[e];
+      if constexpr (SOLVE) f[k] = (e & 63) >= (e >> 6) ? F[e] : 0.0;
+    }
+    if constexpr (SOLVE) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) x[k] *= d[4 * k + lk];
     }
 #pragma unroll
-    for (int k = 0; k < HB * HB / 256; ++k) {
+    for (int k = 0; k < PER; ++k) {
       const int e = threadIdx.x + 256 * k;
       Bs[e >> 6][e & 63] = v[k];
+      if constexpr (SOLVE) Ls[e >> 6][e & 63] = f[k];
     }
   }
   __syncthreads();
+  // acc += y M, lane (lr, lk) holding columns 4 k + lk (k = 0 .. 15) of row lr
+  // of y and of acc (acc[i][e]: k = 4 i + e)
   hf64x4 acc[4];
+  auto mul = [&](const double (*M)[HB + 1], const double (&y)[16]) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(M[4 * k + lk][16 * i + lr], y[k], acc[i], 0,
+                                                      0, 0);
+  };
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc[i] = hf64x4{0, 0, 0, 0};
+  mul(Bs, x);
+  if constexpr (SOLVE) {
+    double q[16], y[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k)
+    for (int k = 0; k < 16; ++k) {
+      q[k] = acc[k >> 2][k & 3];
+      y[k] = -q[k];
+      acc[k >> 2][k & 3] = x[k];
+    }
+    mul(Ls, y);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(Bs[4 * k + lk][16 * i + lr], x[k], acc[i], 0, 0, 0);
+    for (int k = 0; k < 16; ++k) {
+      y[k] = acc[k >> 2][k & 3];
+      acc[k >> 2][k & 3] = q[k];
+    }
+    mul(Bs, y);
+  }
   if (r >= rows) return;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
