@@ -143,3 +143,26 @@ def test_batched_qr_tile_edges(tn):
         k = int(np.count_nonzero(ref > 1e-10 * ref[0]))
         assert np.abs(u[:, :k].T @ u[:, :k] - np.eye(k)).max(initial=0.0) <= 4e-13
         assert np.abs(vt[:k] @ vt[:k].T - np.eye(k)).max(initial=0.0) <= 4e-13
+
+
+# The sweep limit holds for jobs that first sweep over their vectors that are
+# not negligible alone, on both sides of the limit from which they do so.
+@pytest.mark.parametrize("sizes", [[(100, 31, 64), (250, 64, 256)], [(300, 32, 290), (100, 31, 64)]])
+@pytest.mark.parametrize("limit", [1, 2, 3, 29, 30, 60])
+def test_batched_truncate_keeps_to_the_sweep_limit(tn, monkeypatch, sizes, limit):
+    from tncontract_amd import batched
+    rng = np.random.default_rng(7)
+    jobs = [(rng.standard_normal((m, k)).astype(np.float32),
+             rng.standard_normal((k, n)).astype(np.float32)) for m, k, n in sizes]
+    codes = []
+    monkeypatch.setattr(batched.L, "check", codes.append)
+    U, S, Vt, kept, sweeps = batched.batched_truncate([torch.from_numpy(a).cuda() for a, _ in jobs],
+                                                      [torch.from_numpy(b).cuda() for _, b in jobs],
+                                                      rel_threshold=1e-8, max_sweeps=limit)
+    assert sweeps.max() <= limit
+    if limit < 4:
+        assert codes[-1] == batched.L.TN_ERR_NOCONV
+        return
+    assert codes[-1] == batched.L.TN_OK
+    for j, (Lm, Rm) in enumerate(jobs):
+        check_job(Lm, Rm, U[j], S[j], Vt[j], int(kept[j]), 1e-8, 0)

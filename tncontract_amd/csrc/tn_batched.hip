@@ -197,6 +197,10 @@ struct BState {
 // and negligible ones: those then cost the last three sweeps instead of all
 // (32 products of ranks 22 .. 492 and sizes up to 1022: 46.0 -> 34.5 ms;
 // going over to all blocks a sweep later costs a sweep of the first ones).
+// Both parts count against max_sweeps: at least its second half is left for all
+// the blocks, and below kSplitSweeps, where that might be too few, a job sweeps
+// over all of them from the start (jobs take up to about fifteen).
+constexpr int kSplitSweeps = 30;
 __device__ __forceinline__ BState bstate_after(const BJob& J, BState cur, double off,
                                                int max_sweeps, int& outcome) {
   BState n{cur.s + 1, cur.nb, cur.sw, 0};
@@ -205,8 +209,8 @@ __device__ __forceinline__ BState bstate_after(const BJob& J, BState cur, double
     n.s = 0;
     n.sw = cur.sw + 1;
     if (cur.nb < J.nblk) {
-      if (off * off <= 100.0 * J.tol || n.sw >= max_sweeps) n.nb = J.nblk;
-    } else if (off <= J.tol || n.sw >= max_sweeps + (J.nact < J.nblk ? 2 : 0)) {
+      if (off * off <= 100.0 * J.tol || n.sw >= max_sweeps / 2) n.nb = J.nblk;
+    } else if (off <= J.tol || n.sw >= max_sweeps) {
       outcome = off <= J.tol ? 1 : 2;
       n.nb = 0;
     }
@@ -436,10 +440,11 @@ __global__ void __launch_bounds__(EIG_NT) bjac_fused(double* __restrict__ Wv, do
   apply_rows_finish<2, EIG_NW>(Z, J.k, J.k, 0, J.k, I, K2, z, sm.Q);
 }
 
-__global__ void binit_state(const BJob* __restrict__ jobs, int njobs, int s,
+__global__ void binit_state(const BJob* __restrict__ jobs, int njobs, int s, int max_sweeps,
                             BState* __restrict__ state) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < njobs) state[j] = BState{s, jobs[j].nact, 0, 0};
+  if (j < njobs)
+    state[j] = BState{s, max_sweeps < kSplitSweeps ? jobs[j].nblk : jobs[j].nact, 0, 0};
 }
 
 __global__ void binit_identity(double* __restrict__ Zb, const BJob* __restrict__ jobs) {
@@ -1078,7 +1083,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   for (int j = 0; j < njobs; ++j) fused = fused && bj[j].L <= BCH && bj[j].k <= BCH;
   // (a fused step's state follows the one before it; the others' is ready)
   hipLaunchKernelGGL(binit_state, dim3((unsigned)ceil_div(njobs, 256)), dim3(256), 0, st, dbj,
-                     njobs, fused ? -1 : 0, fused ? dstate + njobs : dstate);
+                     njobs, fused ? -1 : 0, max_sweeps, fused ? dstate + njobs : dstate);
   const BOut outcomes{ddone, dsweeps, dactive};
   // A step set of `period` steps is enqueued as one unit (captured once as a
   // HIP graph and replayed; launched kernel by kernel while launch timing is
@@ -1140,7 +1145,7 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
     set_error(TN_ERR_HIP, "%s: host buffer or event creation failed", who);
     rc_loop = TN_ERR_HIP;
   }
-  const int nsets = (int)ceil_div((int64_t)maxsteps * (max_sweeps + 2) + 1, period);
+  const int nsets = (int)ceil_div((int64_t)maxsteps * max_sweeps + 1, period);
   for (int p = 0; rc_loop == TN_OK && p < nsets; ++p) {
     if (exec) {
       if (hipGraphLaunch(exec, st) != hipSuccess) {
