@@ -508,7 +508,7 @@ __global__ void r_rows_kernel(const double* __restrict__ W, int64_t L, int64_t k
 
 // code (may be null): raised to the largest entry code.
 template <typename T>
-__global__ void gather_vectors(const T* __restrict__ src, Modes rows, Modes cols, int64_t m,
+__global__ void __launch_bounds__(256) gather_vectors(const T* __restrict__ src, Modes rows, Modes cols, int64_t m,
                                int64_t n, int tall, double* __restrict__ Wv, int* code) {
   // tall: Wv[j*m + i] = A(i,j)   wide: Wv[i*n + j] = A(i,j)
   int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -522,11 +522,17 @@ __global__ void gather_vectors(const T* __restrict__ src, Modes rows, Modes cols
     top = max(top, entry_code(x));
   }
   if (code == nullptr) return;
+  __shared__ int tops[4];
   top = (int)wave_max((float)top);
-  // (few waves find the value they read still below theirs)
-  if ((threadIdx.x & 63) == 0 && top > __hip_atomic_load(code, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT))
-    atomicMax(code, top);
+  if ((threadIdx.x & 63) == 0) tops[threadIdx.x >> 6] = top;
+  __syncthreads();
+  // one access to the common word a block, few of which still find it below
+  // theirs (with one a wave and a block per 256 elements, 1024 x 2560: 14 -> 121 us)
+  if (threadIdx.x == 0) {
+    top = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
+    if (top > __hip_atomic_load(code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(code, top);
+  }
 }
 
 // The vectors times the power of two of their largest entry code (nothing to
@@ -855,7 +861,7 @@ static int svd_impl(const void* A, const tn_modes* a_rows, const tn_modes* a_col
   // scaled (FP32 entries never need it; jac_small does it itself)
   const bool scaled = dtype == TN_F64 && !(w.precond && small_jacobi(L, k));
   const int* code = scaled ? w.code : nullptr;
-  unsigned gb = (unsigned)std::min<int64_t>(ceil_div(m * n, 256), 65536);
+  unsigned gb = (unsigned)std::min<int64_t>(ceil_div(m * n, 256), scaled ? 1024 : 65536);
   if (scaled) hipLaunchKernelGGL(reset_u64, dim3(1), dim3(1), 0, st, w.off + 4);
   if (dtype == TN_F64)
     hipLaunchKernelGGL(gather_vectors<double>, dim3(gb), dim3(256), 0, st, (const double*)A, rows,
@@ -864,7 +870,7 @@ static int svd_impl(const void* A, const tn_modes* a_rows, const tn_modes* a_col
     hipLaunchKernelGGL(gather_vectors<float>, dim3(gb), dim3(256), 0, st, (const float*)A, rows,
                        cols, m, n, tall, w.Wv, (int*)nullptr);
   if (scaled)
-    hipLaunchKernelGGL(scale_vectors, dim3(std::min(gb, 1024u)), dim3(256), 0, st, w.Wv, m * n,
+    hipLaunchKernelGGL(scale_vectors, dim3(gb), dim3(256), 0, st, w.Wv, m * n,
                        w.code);
   TN_CHECK_LAUNCH();
   bool converged = false;
