@@ -566,3 +566,19 @@ def test_qr_of_nearly_dependent_columns(L, m, n, c):
         assert np.abs(q.T @ q - np.eye(n)).max() <= 1e-13
         res = np.linalg.norm(q @ r - a, axis=0) / np.linalg.norm(a, axis=0)
         assert res.max() <= 1e-14
+
+
+# The rotations keep lengths: a singular vector has met about ten rotations per
+# other vector, whose cosines and sines are rounded without bias, so the vectors
+# that accumulate them stay within a random walk of 10 n steps of 2^-53 of length
+# one (their mean well within).
+@pytest.mark.parametrize("m,n", [(32, 32), (64, 32), (64, 64), (254, 636), (300, 290), (300, 20)])
+def test_rotations_keep_lengths(L, m, n):
+    from tncontract_amd import tensor as T
+    from tncontract_amd.batched import batched_svd
+    a = np.random.default_rng(m + n).standard_normal((m, n))
+    k = min(m, n)
+    for u, s, vt in (T._svd_device(dev(a), 1), [x[0] for x in batched_svd([dev(a)])[:3]]):
+        for v in (u.cpu().numpy(), vt.cpu().numpy().T):
+            w = v.astype(np.longdouble)
+            assert abs(float(((w * w).sum(axis=0) - 1).mean())) <= np.sqrt(10 * k) * 2.0 ** -53

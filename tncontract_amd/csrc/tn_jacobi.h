@@ -173,16 +173,18 @@ __device__ inline double eig_off(EigLds& sm, double tol, double neg2 = 0.0, bool
   return (double)off;
 }
 
-// 1/sqrt(x) for FP64 from the hardware estimate (v_rsq_f64) refined by two
-// Newton steps to full double precision: a far shorter dependent chain than
-// an IEEE square root and division.
-__device__ __forceinline__ double rsq_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double hx = 0.5 * x;
-  double e = fma(-hx * y, y, 0.5);
-  y = fma(y, e, y);
-  e = fma(-hx * y, y, 0.5);
-  return fma(y, e, y);
+// 1 / sqrt(1 + t^2) from the hardware estimate y (v_rsq_f64, up to 3e-8 off) by
+// one third-order step, y (1 + e / 2 + 3 e^2 / 8), on a short dependent chain.
+// Its defect e = 1 - (1 + t^2) y^2 is taken as (1 - y^2) - (t y)^2, never from
+// the rounded 1 + t^2: that lies on a grid of 2^-52, the result on one of 2^-53,
+// and of small angles (|t| in 1e-9 .. 1e-3) it made the cosine 6e-17 too long on
+// average (3e-17 with two Newton steps).  Each rotation then lengthened its two
+// vectors, and a column of Z ended 7e-14 too long after an SVD of 254 vectors.
+__device__ __forceinline__ double cos_of_tan(double t) {
+  const double y = __builtin_amdgcn_rsq(fma(t, t, 1.0));
+  const double p = t * y;
+  const double e = fma(-p, p, fma(-y, y, 1.0));
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
 // Rotation coefficients for index x against partner px: G' = J^T G J with
@@ -198,7 +200,7 @@ __device__ __forceinline__ double rsq_nr(double x) {
 // reciprocal times the scaled |P| in FP64, so an angle far below FP32's
 // range (a nearly-null vector against a large one) is still |P| / (2 |D|)
 // and rotates.  Orthogonality comes from c = 1/sqrt(1 + t^2) in FP64
-// (v_rsq_f64 + two Newton steps) and s = t c, so c^2 + s^2 = 1 to FP64
+// (cos_of_tan) and s = t c, so c^2 + s^2 = 1 to FP64
 // rounding.  A pair is rotated when pair_rotates holds; the coefficients are
 // computed without a branch
 // (a pair that is not rotated selects c = 1, s = 0, discarding whatever the
@@ -216,7 +218,7 @@ __device__ __forceinline__ void rot_coef_v(double gpq, double gpp, double gqq, b
   const float hyp = __builtin_amdgcn_sqrtf(fmaf(d, d, p * p));
   const double tabs = pp * (double)__builtin_amdgcn_rcpf(d + hyp);
   const double t = ((D < 0.0) == (P < 0.0)) ? tabs : -tabs;
-  const double c = rsq_nr(fma(t, t, 1.0));
+  const double c = cos_of_tan(t);
   const double sn = t * c;
   a = rot ? c : 1.0;
   b = rot ? (x_is_l ? -sn : sn) : 0.0;
@@ -257,9 +259,7 @@ __device__ __forceinline__ double dpp_from_prev_ring(double v) {
 // rot_coef_v(..., x_is_l = true) for Gram entries whose products stay in
 // range (EIG_RANGE), on a shorter chain: no scaling, the hypotenuse and the
 // tangent from v_rsq_f64 and v_rcp_f64 (about 2^-23 relative, as good as the
-// FP32 angle), and c from v_rsq_f64 by one third-order step,
-// y (1 + e / 2 + 3 e^2 / 8) with e = 1 - x y^2 (relative error about e^3 / 3,
-// below 2^-65).
+// FP32 angle).
 __device__ __forceinline__ void rot_coef_n(double gpq, double gpp, double gqq, double tol2,
                                            double neg2, double& a, double& b) {
   const bool rot = gpq * gpq > tol2 * gpp * gqq && fmax(gpp, gqq) > neg2;
@@ -270,10 +270,7 @@ __device__ __forceinline__ void rot_coef_n(double gpq, double gpp, double gqq, d
   // -t: the sign of P, flipped where D is not negative
   const long long flip = ~__double_as_longlong(D) & (long long)0x8000000000000000ull;
   const double u = __longlong_as_double(__double_as_longlong(tp) ^ flip);
-  const double x = fma(u, u, 1.0);
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
-  const double c = fma(y * e, fma(e, 0.375, 0.5), y);
+  const double c = cos_of_tan(u);
   a = rot ? c : 1.0;
   b = rot ? u * c : 0.0;
 }
