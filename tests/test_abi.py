@@ -85,3 +85,18 @@ def test_contract_axes_rejects_bad_groups_on_the_host():
         axes = (ctypes.c_int64 * len(bad))(*bad)
         rc = lib.tn_contract_axes(None, None, None, axes, L.TN_F64, 0, 1.0, 0.0, None, 0, None)
         assert rc == L.TN_ERR_INVALID and lib.tn_last_error()
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="library not built")
+def test_contract_workspace_only_for_products_that_split():
+    import torch  # noqa: F401
+    from tncontract_amd import _lib as L
+    need = L.lib().tn_contract_workspace
+    # FP64 products of few 32 x 32 tiles take one launch without partial sums
+    for m, n, k in [(512, 512, 512), (256, 256, 128), (1024, 1024, 128), (64, 64, 512)]:
+        assert need(m, n, k, L.TN_F64) == 0
+    # the first sizes past them, long products of few outputs, and FP32 (whose
+    # split-bf16 products split) keep theirs
+    for m, n, k, dtype in [(512, 512, 513, L.TN_F64), (1024, 544, 512, L.TN_F64),
+                           (8, 8, 70000, L.TN_F64), (512, 512, 512, L.TN_F32)]:
+        assert need(m, n, k, dtype) > 0

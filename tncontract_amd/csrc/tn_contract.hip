@@ -1273,6 +1273,8 @@ extern "C" int tn_contract(const void* A, const tn_modes* a_m, const tn_modes* a
 
 extern "C" size_t tn_contract_workspace(int64_t M, int64_t N, int64_t K, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
+  // (FP32 data may be multiplied in split bf16, which does split these)
+  if (dtype == TN_F64 && few_tiles(P_F64, M, N, K)) return 0;
   const int S = splitk_factor(M, N, K);
   return S > 1 ? (size_t)S * (size_t)M * (size_t)N * (dtype == TN_F64 ? 8 : 4) : 0;
 }
