@@ -1090,8 +1090,12 @@ static int batched_driver(const tn_trunc_job* tj, const tn_svd_job* sj, int njob
   // on).  The host reads the active-job count of a set while the next set
   // runs, so the GPU never waits for the host; a set enqueued after the last
   // job retired exits at once in every block.  Even (the parity of a step
-  // picks its state), and long enough that a set outlasts its launch.
-  constexpr int period = 16;
+  // picks its state), and long enough that a set outlasts its launch: 16 steps,
+  // or 8 of three launches each where the longest sweep is no longer than that
+  // (long vectors, few of them), as such jobs may be done within a few steps and
+  // up to two sets then run for nothing (60 jobs of 300 x 20, graded: 976 us with
+  // 16, 848 with 8; one-launch steps of 100 x 100 jobs 5 % slower with 8).
+  const int period = !fused && maxsteps <= 8 ? 8 : 16;
   auto enqueue_set = [&]() {
     for (int o = 0; o < period; ++o) {
       BState *cur = dstate + (o & 1) * njobs, *other = dstate + (~o & 1) * njobs;
