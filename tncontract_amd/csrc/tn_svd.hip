@@ -146,7 +146,8 @@ __global__ void __launch_bounds__(EIG_NT) jac_eig_apply(double* __restrict__ Wv,
 // copied.  offs: the measures of this sweep, of the one before and (cleared
 // here) of the next in turn, and the number of sweeps run; once a sweep has
 // found nothing to rotate, the steps of later ones leave everything alone, so
-// the host can enqueue sweeps ahead.  It saves the Gram launch (4.4 us and the gap to the next) and the
+// the host can enqueue sweeps ahead; mail (may be null): the sweeps ended before
+// this one, twice, plus one if the last of them rotated nothing.  It saves the Gram launch (4.4 us and the gap to the next) and the
 // partials' trip through memory: 12.9 us a step, 254 x 636 SVD 3.09 -> 2.87 ms,
 // 64 x 64 eigensolve 618 -> 529 us.  Past 256 rows every block would repeat a
 // Gram as long as the launch it saves (512 rows: 3.4 us of MFMAs).
@@ -154,7 +155,8 @@ __global__ void __launch_bounds__(EIG_NT) jac_step(const double* __restrict__ Wi
                                                    double* __restrict__ Wout, int64_t L,
                                                    double* __restrict__ Z, int64_t nv, int s,
                                                    int nblk, int nchW, double tol, int sweep,
-                                                   unsigned long long* __restrict__ offs) {
+                                                   unsigned long long* __restrict__ offs,
+                                                   unsigned long long* __restrict__ mail) {
   constexpr int CH = 16 * EIG_NW;
   __shared__ EigLds sm;
   __shared__ PairGramLds pg;
@@ -163,6 +165,9 @@ __global__ void __launch_bounds__(EIG_NT) jac_step(const double* __restrict__ Wi
   if (s == 0 && pi == 0 && ch == 0 && threadIdx.x == 0) {
     offs[(sweep + 1) % 3] = 0ull;  // (and so is every later sweep's)
     if (!done) offs[3] = (unsigned long long)(sweep + 1);
+    if (mail)
+      __hip_atomic_store(mail, 2ull * sweep + (done ? 1 : 0), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
   }
   if (done) return;
   int I, J;
@@ -564,6 +569,75 @@ struct SvdWs {
   int precond;
 };
 
+// One word of pinned host memory that a kernel writes and the host polls, from a
+// pool of the process (any thread, device and stream; a call holds its own word
+// until the kernels of its stream that write it have ended: idle, or waited for).
+// None (word == nullptr) if not wanted or not to be had.
+struct Mailbox {
+  unsigned long long* word = nullptr;
+  bool idle = false;
+  Mailbox(bool wanted, hipStream_t stream) : st(stream) {
+    if (!wanted) return;
+    {
+      std::lock_guard<std::mutex> lk(mu());
+      if (!pool().empty()) {
+        word = pool().back();
+        pool().pop_back();
+      }
+    }
+    if (word == nullptr) {
+      // (another thread's stream capture is none of this allocation's business)
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+      if (hipHostMalloc((void**)&word, sizeof(*word),
+                        hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess)
+        word = nullptr;
+      if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+      if (word == nullptr) (void)hipGetLastError();
+    }
+    if (word) __atomic_store_n(word, 0ull, __ATOMIC_RELAXED);
+  }
+  Mailbox(const Mailbox&) = delete;
+  Mailbox& operator=(const Mailbox&) = delete;
+  ~Mailbox() {
+    if (word == nullptr) return;
+    if (!idle) (void)hipStreamSynchronize(st);
+    {
+      std::lock_guard<std::mutex> lk(mu());
+      if (pool().size() < kKept) {
+        pool().push_back(word);
+        return;
+      }
+    }
+    (void)hipHostFree(word);
+  }
+  // The word once it is at least `least`; 0 if the stream ends or fails before.
+  unsigned long long wait(unsigned long long least) const {
+    for (;;) {
+      for (int i = 0; i < 2000; ++i) {
+        const unsigned long long v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        if (v >= least) return v;
+        __builtin_ia32_pause();
+      }
+      const hipError_t e = hipStreamQuery(st);
+      if (e == hipErrorNotReady) continue;
+      if (e != hipSuccess) return 0;
+      const unsigned long long v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+      return v >= least ? v : 0;
+    }
+  }
+
+ private:
+  hipStream_t st;
+  static constexpr size_t kKept = 16;  // words kept for later calls
+  // (never destroyed: the HIP runtime may be gone by then)
+  static std::mutex& mu() { static std::mutex* m = new std::mutex; return *m; }
+  static std::vector<unsigned long long*>& pool() {
+    static auto* v = new std::vector<unsigned long long*>;
+    return *v;
+  }
+};
+
 // One workgroup and one launch (jac_small).
 static bool small_jacobi(int64_t L, int64_t k) { return k <= J2 && L <= kSmallLen; }
 
@@ -665,23 +739,43 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
   double* const W2 = nblk - 1 < 16 && L <= kPairLen ? sort_tmp : nullptr;
   if (nblk - 1 < 16) sort_tmp = nullptr;
   if (W2) {
-    // six sweeps, then two at a time, between looks at the measure: a look costs
-    // 25 us of an idle GPU, a sweep enqueued for nothing 2 us a step, and these
-    // sizes need 7 to 12 sweeps (254 x 636 SVD 2.85 -> 2.63 ms)
     hipLaunchKernelGGL(reset_u64, dim3(1), dim3(4), 0, st, w.off);
     unsigned long long h[4] = {0, 0, 0, 0};
-    for (int todo = std::min(6, max_sweeps); sweep < max_sweeps && !*converged;
-         todo = std::min(2, max_sweeps - sweep)) {
-      for (int i = 0; i < todo; ++i)
-        for (int s = 0; s < nblk - 1; ++s) {
-          ProfScope p(PROF_JAC_EIG, st,
-                      step_rounds(inner_step(s, nblk)) * 9216.0 * npairs + gram_fl + apply_fl,
-                      16.0 * (double)(L + kz) * J2 * npairs);
-          const bool flip = (((sweep + i) * (nblk - 1) + s) & 1) != 0;
-          hipLaunchKernelGGL(jac_step, dim3(npairs, nchW + nchZ), dim3(EIG_NT), 0, st,
-                             flip ? W2 : Wv, flip ? Wv : W2, L, Z, k, s, nblk, nchW, tol, sweep + i,
-                             w.off);
+    Mailbox mail(allow_graph, st);  // (no allocation for tn_svd_noalloc)
+    auto enqueue = [&](int sw) {
+      for (int s = 0; s < nblk - 1; ++s) {
+        ProfScope p(PROF_JAC_EIG, st,
+                    step_rounds(inner_step(s, nblk)) * 9216.0 * npairs + gram_fl + apply_fl,
+                    16.0 * (double)(L + kz) * J2 * npairs);
+        const bool flip = ((sw * (nblk - 1) + s) & 1) != 0;
+        hipLaunchKernelGGL(jac_step, dim3(npairs, nchW + nchZ), dim3(EIG_NT), 0, st,
+                           flip ? W2 : Wv, flip ? Wv : W2, L, Z, k, s, nblk, nchW, tol, sw, w.off,
+                           mail.word);
+      }
+    };
+    // With a mailbox the host keeps one sweep enqueued beyond the one it waits
+    // for, whose first step posts the outcome: the GPU waits for nothing, and one
+    // sweep of steps that return at once (2 us each) is enqueued for nothing.
+    int queued = 0;
+    if (mail.word) {
+      enqueue(queued++);
+      while (queued < max_sweeps && !*converged) {
+        enqueue(queued++);
+        TN_CHECK_LAUNCH();
+        const unsigned long long v = mail.wait(2ull * (queued - 1));
+        if (v == 0) {
+          set_error(TN_ERR_HIP, "tn_svd: a Jacobi sweep failed");
+          return TN_ERR_HIP;
         }
+        sweep = queued - 1;
+        *converged = (v & 1) != 0;
+      }
+    }
+    // Without one, and for the last sweep: a copy after one, six and then every
+    // two sweeps (each costs 25 us of an idle GPU).
+    for (int next = queued ? max_sweeps : std::min(1, max_sweeps);
+         sweep < max_sweeps && !*converged; next = std::min(next < 6 ? 6 : next + 2, max_sweeps)) {
+      while (queued < next) enqueue(queued++);
       TN_CHECK_LAUNCH();
       TN_HIP(hipMemcpyAsync(h, w.off, sizeof(h), hipMemcpyDeviceToHost, st));
       TN_HIP(hipStreamSynchronize(st));
@@ -690,6 +784,7 @@ static int jacobi_run(double* Wv, int64_t L, double* Z, int64_t k, const SvdWs& 
       memcpy(&off, &h[(sweep + 2) % 3], sizeof(off));
       *converged = off <= tol;
     }
+    mail.idle = true;
     if ((sweep * (nblk - 1)) & 1) {
       hipLaunchKernelGGL(copy_f64, dim3((unsigned)ceil_div(L * k, 256)), dim3(256), 0, st, W2, Wv,
                          L * k);
