@@ -582,3 +582,59 @@ def test_rotations_keep_lengths(L, m, n):
         for v in (u.cpu().numpy(), vt.cpu().numpy().T):
             w = v.astype(np.longdouble)
             assert abs(float(((w * w).sum(axis=0) - 1).mean())) <= np.sqrt(10 * k) * 2.0 ** -53
+
+
+# One-launch Jacobi steps: sweeps are enqueued ahead of their outcomes, which
+# reach the host through a word of pinned memory (tn_svd) or by copies
+# (tn_svd_noalloc).  Both count and stop alike, at every limit.
+@pytest.mark.parametrize("limit", [1, 2, 5, 6, 7, 8, 40])
+@pytest.mark.parametrize("case", ["identity", "full"])
+def test_sweep_counts_of_one_launch_steps(L, limit, case):
+    from tncontract_amd import tensor as T
+    n = 100
+    a = np.eye(n) if case == "identity" else np.random.default_rng(1).standard_normal((n, n))
+    d = dev(a)
+    rows, cols, _, _ = T._matrix_modes(d, 1)
+    lib = L.lib()
+    ws = L.workspace(lib.tn_svd_workspace(n, n, 0))
+    got = []
+    for noalloc in (False, True):
+        u, s, vt = L.empty((n, n)), L.empty((n,)), L.empty((n, n))
+        sweeps = ctypes.c_int(-1)
+        args = [L.ptr(d), ctypes.byref(rows), ctypes.byref(cols), n, n, L.ptr(u), L.ptr(s),
+                L.ptr(vt), 0, 0.0, limit, ctypes.byref(sweeps)]
+        rc = lib.tn_svd_noalloc(*args, L.stream_ptr()) if noalloc else \
+            lib.tn_svd(*args, L.ptr(ws), ws.numel(), L.stream_ptr())
+        got.append((rc, sweeps.value, u.cpu().numpy(), s.cpu().numpy(), vt.cpu().numpy()))
+    (rc, used, u, s, vt), other = got
+    assert other[:2] == (rc, used) and all(np.array_equal(x, y) for x, y in zip(got[0][2:], other[2:]))
+    assert used <= limit
+    if case == "identity":
+        assert rc == L.TN_OK and used == 1
+    elif limit <= 2:
+        assert rc == L.TN_ERR_NOCONV and used == limit
+    if rc == L.TN_OK:
+        assert np.linalg.norm((u * s) @ vt - a) <= 4e-13 * s[0] * np.sqrt(n)
+
+
+def test_svds_of_threads_with_their_own_streams(L):
+    import threading
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(2)
+    mats = [rng.standard_normal((m, n)) for m, n in [(100, 100), (64, 200), (250, 130), (40, 40)] * 3]
+    errs = [None] * len(mats)
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            d = dev(mats[i])
+            for _ in range(4):
+                u, s, vt = (x.cpu().numpy() for x in T._svd_device(d, 1))
+                e = np.linalg.norm((u * s) @ vt - mats[i]) / s[0]
+                errs[i] = max(errs[i] or 0.0, e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(mats))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(e is not None and e <= 4e-13 * np.sqrt(200) for e in errs), errs
