@@ -638,3 +638,29 @@ def test_svds_of_threads_with_their_own_streams(L):
     for t in threads:
         t.join()
     assert all(e is not None and e <= 4e-13 * np.sqrt(200) for e in errs), errs
+
+
+# Split-bf16 products with one row or column, and with operands that repeat one
+# (stride 0) or are sliced (no unit stride: the tables); bound as for the tiles.
+@pytest.mark.parametrize("M,K,N", [(1, 300, 2000), (2000, 300, 1), (1, 4000, 70), (128, 64, 128),
+                                   (200, 130, 300)])
+@pytest.mark.parametrize("kind", ["dense", "rows_of_a", "columns_of_b", "k_of_a", "k_of_b", "sliced"])
+def test_contract_bf16x3_broadcast_operands(L, M, K, N, kind):
+    from tncontract_amd import tensor as T
+    rng = np.random.default_rng(M + 3 * K + 7 * N)
+    a, b = (dev(rng.standard_normal(s).astype(np.float32)) for s in ((M, K), (K, N)))
+    if kind == "rows_of_a":
+        a = a[:1].expand(M, K)
+    elif kind == "columns_of_b":
+        b = b[:, :1].expand(K, N)
+    elif kind == "k_of_a":
+        a = a[:, :1].expand(M, K)
+    elif kind == "k_of_b":
+        b = b[:1].expand(K, N)
+    elif kind == "sliced":
+        a, b = dev(rng.standard_normal((M, 2 * K)).astype(np.float32))[:, ::2], \
+            dev(rng.standard_normal((K, 3 * N)).astype(np.float32))[:, ::3]
+    c = T._contract_data(a, [1], b, [0], precision="bf16x3").cpu().numpy().astype(np.float64)
+    a, b = a.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64)
+    bound = (3 * 2.0 ** -18 + (3 * K + 8) * 2.0 ** -24) * (np.abs(a) @ np.abs(b))
+    assert np.all(np.abs(c - a @ b) <= bound)

@@ -1175,8 +1175,11 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
       (double)(K + 64) * st1(g.bk) + (double)(N + BN) * st1(g.bn) < lim &&
       (double)(M + BM) * st1(g.cm) + (double)(N + BN) * st1(g.cn) < lim;
   // operands with a unit stride along k or along their free index: 16-byte
-  // loads (negative strides, a size-1 operand axis or a stride-0 one take the
-  // table path)
+  // loads, whatever (non-negative) stride the other index has: 0 too, for a
+  // broadcast axis or an empty group, which only re-reads the same data.  Partial
+  // tiles test every element, so a size-1 axis reads nothing past it.  Negative
+  // strides, and operands without a unit stride (sliced views, which took the
+  // tables before there were 16-byte loads, in the same time), take the tables.
   const bool vak = st1(g.ak) == 1, vbk = st1(g.bk) == 1;
   const bool vec = simple && st1(g.am) >= 0 && st1(g.ak) >= 0 && st1(g.bk) >= 0 &&
                    st1(g.bn) >= 0 && st1(g.cm) >= 0 && st1(g.cn) >= 0 &&
