@@ -641,7 +641,8 @@ def test_svds_of_threads_with_their_own_streams(L):
 
 
 # Split-bf16 products with one row or column, and with operands that repeat one
-# (stride 0) or are sliced (no unit stride: the tables); bound as for the tiles.
+# (stride 0) or are sliced (no unit stride: the tables).  A bf16 has an 8-bit
+# significand, so a half's rounding is 2^-8 of it: x y is kept but for 3 * 2^-16.
 @pytest.mark.parametrize("M,K,N", [(1, 300, 2000), (2000, 300, 1), (1, 4000, 70), (128, 64, 128),
                                    (200, 130, 300)])
 @pytest.mark.parametrize("kind", ["dense", "rows_of_a", "columns_of_b", "k_of_a", "k_of_b", "sliced"])
@@ -662,5 +663,5 @@ def test_contract_bf16x3_broadcast_operands(L, M, K, N, kind):
             dev(rng.standard_normal((K, 3 * N)).astype(np.float32))[:, ::3]
     c = T._contract_data(a, [1], b, [0], precision="bf16x3").cpu().numpy().astype(np.float64)
     a, b = a.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64)
-    bound = (3 * 2.0 ** -18 + (3 * K + 8) * 2.0 ** -24) * (np.abs(a) @ np.abs(b))
+    bound = (3 * 2.0 ** -16 + (3 * K + 8) * 2.0 ** -24) * (np.abs(a) @ np.abs(b))
     assert np.all(np.abs(c - a @ b) <= bound)
