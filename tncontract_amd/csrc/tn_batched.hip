@@ -12,12 +12,15 @@
 //    wide).  Two tile shapes (64x64, 128x128); a small autotuner times both
 //    per size bucket on first use and caches the choice.
 //  * batched one-sided block Jacobi: every job advances its own round-robin
-//    schedule (step g mod (nblk_j - 1)) in the same gram / eig / apply
-//    launches; a per-job sweep-end kernel retires converged jobs on the
-//    device.  A set of steps (at least one sweep of the largest job) is
-//    captured once as a HIP graph and replayed, the device advancing its own
-//    step counter; the host reads each set's active-job count while the next
-//    set runs and stops replaying when none is left.
+//    schedule (step s of a sweep over its first nb blocks, kept on the device:
+//    BState) in the same launches: gram / eig / apply, the last of which works
+//    out the next step's state, or, where every job's vectors fit one row chunk,
+//    one launch that does all of it (bjac_fused).  A converged job's state
+//    retires it.  A set of 16 (or 8) steps is captured once as a HIP graph and
+//    replayed; the host reads each set's active-job count while the next set
+//    runs and stops replaying when none is left.
+//    A job whose later vectors are all negligible first sweeps over the blocks
+//    before them alone (bstate_after).
 //    Vectors whose squared norm is below (thr / 2k)^2 ||C_j||_F^2 are not
 //    rotated against each other (bjob_neg2): the rounding-level vectors of a
 //    rank-deficient product lie below the keep threshold whatever their

@@ -1039,7 +1039,11 @@ int contract_launch(const void* A, const Modes& a_m, const Modes& a_k, const voi
       h.beta = beta;
       // four lanes from 9 terms on, 16 from 64, a wave from 256, the block
       // from 4096: four to sixteen terms a lane where the outputs alone do
-      // not fill the chip
+      // not fill the chip.  Calls back to back, 15 x 15 outputs: any number of
+      // lanes 6.6 .. 7.1 us up to 255 terms (one lane 7.2 at 16, 21 at 64, 78 at
+      // 255), 1000 terms 19.8 / 8.4 / 8.6 / 8.4 us by 4 / 16 / 64 / 256 lanes,
+      // 4096 terms 72.9 / 20.4 / 8.5 / 8.5; the block's 256 pay for one output of
+      // 20000 terms and more
       const int G = K < 64 ? 4 : (K < 256 ? 16 : (K < 4096 ? 64 : 256));
       const int64_t ob = ceil_div(g.nout, 256 / G);
       // ... and ranges of at least 4096 terms over more blocks

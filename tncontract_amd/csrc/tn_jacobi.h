@@ -111,8 +111,9 @@ __device__ __forceinline__ void pair_scaled(double gpq, double gpp, double gqq, 
 
 // Rotation predicate of a pair (l, h) from G_lh, G_ll, G_hh: G_lh^2 > tol^2
 // G_ll G_hh on the scaled entries, and one of the two vectors not negligible
-// (squared norm > neg2).  rot_coef_v rotates exactly the pairs for which it
-// holds, and the convergence measure eig_off counts exactly those.  A vector
+// (squared norm > neg2).  The convergence measure eig_off counts the pairs for
+// which it holds at tol; the rounds rotate those for which it holds at tol / 4
+// (rot_coef_v; rot_coef_n tests the first two conditions alone).  A vector
 // whose squared norm underflows is not rotated with one 2^40 times longer: the
 // norm is lost and its product with the other is not, so the pair would be
 // rotated without end (the rounding that a sparse low-rank matrix leaves can
@@ -131,9 +132,11 @@ __device__ __forceinline__ bool pair_rotates(double gpq, double gpp, double gqq,
 
 // Convergence measure of the pair block: the largest |G_pq| / sqrt(G_pp G_qq)
 // (an FP32 estimate from the scaled entries, at least just above tol) over
-// the pairs of this step (inner: all; otherwise those across the blocks) that
-// pair_rotates would rotate, 0 if there are none; so "off <= tol" holds
-// exactly when a sweep would rotate nothing.  Pairs of two
+// the pairs of this step (inner: all; otherwise those across the blocks) for
+// which pair_rotates holds, 0 if there are none.  A block pair with off <= tol is
+// left alone, so a sweep whose every step had that, inner pairs at every fourth
+// step included, has changed nothing: every pair of vectors is then within tol.
+// Pairs of two
 // negligible vectors (squared norms <= neg2) are left out: the caller has
 // shown that the space they span lies below its truncation threshold
 // whether or not they are orthogonalised (neg2 = 0: every pair).

@@ -839,6 +839,10 @@ namespace tn {
 // the work, were what a small QR took (64 x 32: some seventeen of 2 .. 19 us);
 // this is one, of 32 us, bound by the chain of its reflectors (20-site
 // compression with its 19 QRs of 64 x 32: 10.0 -> 8.0 ms).
+// Its limits are the registers' and LDS's; against the panels: 8 x 8 15 / 58 us,
+// 64 x 32 39 / 158, 256 x 32 75 / 179, 64 x 64 107 / 294, 128 x 64 181 / 295,
+// 256 x 40 123 / 212, and at the corner, 256 x 64, 189 / 181 by a block of
+// tn_qr_hr.h.
 constexpr int kQrSmallCols = 64, kQrSmallRows = 256;
 
 template <typename T, int NC, int NI>

@@ -51,7 +51,6 @@ static int eig_nt(int npairs, int64_t L, int64_t kz) {
 // but the step 0.5 us more: 1024 x 2560 SVD 17.0 -> 16.7 ms).
 constexpr int GCH = kPairLen;
 
-
 // G (sm.G[0]) = sum of the pair's nchunk partials (fixed order, so every
 // block that sums them gets the same bits).  The partials are read eight
 // chunks at a time with every load issued before the first add: a load-add
@@ -368,8 +367,9 @@ __global__ void __launch_bounds__(EIG_NT) jac_small(double* __restrict__ Wv, int
 }
 
 // Convergence of the whole vector set from its Gram matrix G = Wv^T Wv
-// (k x k, either triangle): eig_off's measure over every pair (p < q), so
-// "off <= tol" holds exactly when a sweep would rotate no pair of G.
+// (k x k, either triangle): eig_off's measure over every pair (p < q), so with
+// off <= tol every pair of vectors is within tol, as after a sweep that leaves
+// every block pair alone.
 __global__ void __launch_bounds__(256) gram_off(const double* __restrict__ G, int64_t k,
                                                 double tol, unsigned long long* __restrict__ offmax) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -406,7 +406,6 @@ __global__ void __launch_bounds__(256) vec_norms(const double* __restrict__ Wv, 
 
 // perm[rank] = j with rank = #{i : s_i > s_j or (s_i == s_j and i < j)};
 // NaN ranks as -inf so that the ranks stay a permutation of 0..k-1.
-
 // 64 elements j per block of 256 threads (k = 1024 spreads over 16 CUs;
 // 1024-thread blocks of 256 elements kept it on 4 and took 15.5 us): the
 // four lanes l, l + 16, l + 32, l + 48 of a wave count over every fourth key
