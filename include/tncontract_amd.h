@@ -179,6 +179,8 @@ int tn_cholqr(const void* A, const tn_modes* a_rows, const tn_modes* a_cols, int
  * most 256, the vectors are first ordered by norm and QR-factored (Cholesky
  * QR, Householder when that does not reach orthogonality 1e-13; Householder
  * for k <= 32 of length at most 256) and the Jacobi runs on the rows of R.
+ * tn_svd and tn_eigh_psd read outcomes through a word of pinned host memory; up to
+ * 16 such words stay allocated in the process.
  * FP64 matrices of any finite magnitude: the vectors are scaled by a power of
  * two where their squares would leave the range (tn_batched_svd and, for K's
  * diagonal, tn_eigh_psd alike).
