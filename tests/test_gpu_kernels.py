@@ -665,3 +665,21 @@ def test_contract_bf16x3_broadcast_operands(L, M, K, N, kind):
     a, b = a.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64)
     bound = (3 * 2.0 ** -16 + (3 * K + 8) * 2.0 ** -24) * (np.abs(a) @ np.abs(b))
     assert np.all(np.abs(c - a @ b) <= bound)
+
+
+# Products of few tiles allocate their result alone; a product that splits K
+# gets the same partial sums in every precision.
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_contract_allocates_no_unused_buffer(L, dtype):
+    from tncontract_amd import tensor as T
+    for n, k, splits in [(512, 512, False), (256, 128, False), (256, 2000, True)]:
+        a, b = (torch.ones(s, dtype=dtype, device="cuda") for s in ((n, k), (k, n)))
+        torch.cuda.synchronize()
+        base = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        c = T._contract_data(a, [1], b, [0])
+        used = torch.cuda.max_memory_allocated() - base
+        sums = L.lib().tn_contract_workspace(n, n, k, L.dtype_code(a)) if splits else 0
+        assert used <= c.numel() * c.element_size() + sums + 1024
+        assert splits == (used > 2 * c.numel() * c.element_size())
+        assert (c == k).all()

@@ -209,7 +209,11 @@ def contract_axes(d1, free1, ax1, d2, ax2, free2, out, ostrides, prec, M, N, K):
     code = dtype_code(d1)
     ws, nb = None, 0
     if K >= 128:
-        nb = L.tn_contract_workspace(M, N, K, code)
+        # (FP32 products split like FP64 ones, into sums half as wide, unless they
+        # are multiplied in split bf16)
+        nb = L.tn_contract_workspace(M, N, K, code if prec == PREC["bf16x3"] else TN_F64)
+        if code == TN_F32 and prec != PREC["bf16x3"]:
+            nb //= 2
         if nb:
             buf = torch.empty(nb, dtype=torch.uint8, device=d1.device)
             ws = buf.data_ptr()
