@@ -620,7 +620,10 @@ struct Mailbox {
         __builtin_ia32_pause();
       }
       const hipError_t e = hipStreamQuery(st);
-      if (e == hipErrorNotReady) continue;
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();  // (not an error for the launch checks that follow)
+        continue;
+      }
       if (e != hipSuccess) return 0;
       const unsigned long long v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
       return v >= least ? v : 0;
